@@ -34,6 +34,7 @@
 #include "pg_common.h"
 #include "pg_eop.h"
 #include "pg_eop_mask.h"
+#include "pg_factor.h"
 
 namespace pg {
 
@@ -138,6 +139,15 @@ __device__ __forceinline__ R tab_next(const R* __restrict__ t, R (&tb)[2][KB], i
     __builtin_amdgcn_sched_barrier(0);
   }
   return tb[(off / KB) & 1][off % KB];
+}
+
+// the value of the neighbouring lane (lane ^ 1)
+__device__ inline int swap_pair(int v) {
+  return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);  // quad_perm [1, 0, 3, 2]
+}
+__device__ inline float swap_pair(float v) { return __int_as_float(swap_pair(__float_as_int(v))); }
+__device__ inline double swap_pair(double v) {
+  return __hiloint2double(swap_pair(__double2hiint(v)), swap_pair(__double2loint(v)));
 }
 
 template <int NV>
@@ -500,126 +510,95 @@ __global__ void __launch_bounds__(kBS) k_eop_sum(int64_t nent, const int32_t* __
 // ---------------------------------------------------------------------------
 // multi-right-hand-side local products for the batched solver: column r of the
 // (ndof, R) row-major block x gets y_e,r = (K_e - i omega_r mu0 M_e) x_e,r.
-// One workgroup of R threads (thread = column; R = 64 .. 256) per part of a
-// slot group w of the single-RHS layout (64 elements of one orientation
-// combination, split into 256 / R parts), which takes its elements one after
-// another.  Per element the threads first form
-// the n(n+1)/2 entry pairs (K_ij, M_ij) from the raw coefficients and the
-// combination's table (pdesc[k] = {table offset, zero mask} of pair k) into
-// LDS, double buffered so that one barrier per element suffices; then every
-// thread gathers its column of x_e (R contiguous values per DOF) and applies
-// the symmetric element matrix, each pair read once from LDS as a broadcast
-// and applied to rows i and j.  The entries are formed once per element for
-// all R columns.  Local results ye[((w N + i) 64 + l) R + r]: the single-RHS
-// slot numbering times R, so the per-entity summation reuses the slot lists.
-// With `dpart` each thread also sums x_e,r^T y_e,r over its elements (FP64):
-// dpart[(k R + r) gridDim + block], k = 0 real, 1 imaginary part, the element
-// share of x_r^T A_r x_r (PEC DOFs are zero in x_e and add nothing here).
+// One workgroup of 2 R threads (thread 2 r + part = the real or imaginary part
+// of column r; R = 64 .. 256) per part of a slot group w of the single-RHS
+// layout (64 elements, split into `split` parts), which takes its elements one
+// after another.  The element is the same for the whole workgroup, so its
+// entities, orientation and coefficients are scalars, and each of its DOFs is
+// one contiguous load of 2 R values; K x_e and M x_e of the thread's real
+// vector are formed without the element matrix (pg_factor.h), in FP64 for
+// complex64 columns too (the same issue rate), and the two parts of a column
+// exchange M x_e across neighbouring lanes.  Local results
+// ye[((w N + i) 64 + l) R + r]: the single-RHS slot numbering times R, so the
+// per-entity summation reuses the slot lists.
+// With `dpart` each thread also sums its share of x_e,r^T y_e,r over its
+// elements (FP64): dpart[(k R + r) gridDim + block], k = 0 real, 1 imaginary
+// part, the element share of x_r^T A_r x_r (PEC DOFs are zero in x_e and add
+// nothing here).
+// Bound: FP64 issue on small meshes, the traffic of x and ye on large ones.
+// Forming the 210 entry pairs of an element in LDS and applying them, one
+// thread per column, 16 elements per workgroup, took 177, 281 and 1479 us at
+// 2 058, 24 576 and 162 000 elements (64 complex128 columns); this takes 19, 184
+// and 1261 us.  The first pays for filling the chip (140 workgroups then, 2 200
+// now), the last is within 1.5 of the copy rate.  At most 168 registers (three
+// waves per SIMD): M x_e is finished before K x_e begins.
 // ---------------------------------------------------------------------------
-template <int P, typename RT>
-__global__ void __launch_bounds__(256) k_meop_local(
-    int64_t nw, int R, int split, const int32_t* __restrict__ done,
-    const int32_t* __restrict__ wcombo,
-    const int32_t* __restrict__ edofs, const double* __restrict__ coefm,
-    const double* __restrict__ tab, const int2* __restrict__ pdesc,
-    const double* __restrict__ omu, const typename Cx<RT>::T* __restrict__ x,
-    typename Cx<RT>::T* __restrict__ ye, double* __restrict__ dpart) {
-  using C = typename Cx<RT>::T;
-  constexpr int N = P * (P + 2) * (P + 3) / 2;
-  constexpr int NP = N * (N + 1) / 2;
+template <int P, typename R>
+__global__ void __launch_bounds__(512, 3) k_meop_local(
+    int64_t nw, int nrhs, int split, const int32_t* __restrict__ done,
+    const int32_t* __restrict__ edofs, const int32_t* __restrict__ ocode,
+    const double* __restrict__ coefm, const double* __restrict__ omu, const R* __restrict__ x,
+    R* __restrict__ ye, double* __restrict__ dpart) {
+  constexpr int N = fac::n_dofs<P>();
   constexpr int NLE = n_local_entities<P>();
   if (done && *done) return;
-  constexpr int NTS = table_stride<P>();
-  __shared__ C ent[2][NP];
-  __shared__ double tl[NTS];  // the combination's table, staged once per workgroup
-  // workgroup b: part b % split of slot group b / split (`split` workgroups per
-  // group, so that narrow batches still launch several waves per SIMD)
   const int64_t nb = gridDim.x;
   int64_t b = blockIdx.x;
   if (nb % 8 == 0) b = (b % 8) * (nb / 8) + b / 8;  // XCD-contiguous ranges of slot groups
   const int64_t w = b / split;
-  const int part = (int)(b - w * split);
   if (w >= nw) return;
-  const int r = threadIdx.x;
-  const RT om = (RT)omu[r];
-  const int combo = wcombo[w];
-  const double* __restrict__ t = tab + (int64_t)combo * NTS;
-  for (int k = threadIdx.x; k < NTS; k += blockDim.x) tl[k] = t[k];
-  __syncthreads();
-  const int l0 = part * (kWave / split), l1 = l0 + kWave / split;
-  double dre = 0.0, dim = 0.0;  // x^T y over this thread's elements
-  for (int l = l0; l < l1; ++l) {
-    int fv[NLE];
+  const int per = kWave / split, l0 = (int)(b - w * split) * per;
+  const int t = threadIdx.x, r = t >> 1;
+  // y_re = K x_re + omega mu0 M x_im, y_im = K x_im - omega mu0 M x_re
+  const double om = (t & 1) ? -omu[r] : omu[r];
+  const int64_t ld = 2 * (int64_t)nrhs;
+  double dre = 0.0, dim = 0.0;  // this part's share of x^T y over the elements
+  for (int l = l0; l < l0 + per; ++l) {
+    int f[NLE];
     bool any = false;
 #pragma unroll
     for (int la = 0; la < NLE; ++la) {
-      fv[la] = edofs[(w * NLE + la) * kWave + l];
-      any |= fv[la] >= 0;
+      f[la] = edofs[(w * NLE + la) * kWave + l];
+      any |= f[la] >= 0;
     }
     if (!any) continue;  // empty slot (or every entity PEC): no products; uniform branch
-    C* e = ent[l & 1];
-    double cfl[12];  // the element's raw coefficients (uniform: scalar loads)
+    double g[6], h[6];
 #pragma unroll
-    for (int c = 0; c < 12; ++c) cfl[c] = coefm[(w * 12 + c) * kWave + l];
-    for (int k = threadIdx.x; k < NP; k += blockDim.x) {
-      const int2 pd = pdesc[k];
-      int o = pd.x;
-      double m = 0.0, kk = 0.0;
-      for (int c = 0; c < 6; ++c)
-        if (!((pd.y >> c) & 1)) m = fma(cfl[c], tl[o++], m);
-      for (int c = 6; c < 12; ++c)
-        if (!((pd.y >> c) & 1)) kk = fma(cfl[c], tl[o++], kk);
-      e[k] = C{(RT)kk, (RT)m};
+    for (int c = 0; c < 6; ++c) {
+      g[c] = coefm[(w * 12 + c) * kWave + l];
+      h[c] = coefm[(w * 12 + 6 + c) * kWave + l];
     }
-    C xv[N];
+    double xv[N], y[N], m[N];
 #pragma unroll
     for (int la = 0; la < NLE; ++la)
 #pragma unroll
       for (int k = 0; k < loc_nd<P>(la); ++k)
-        xv[loc_off<P>(la) + k] = fv[la] >= 0 ? x[(int64_t)(fv[la] + k) * R + r] : C{0, 0};
-    __syncthreads();
-    C y[N];
+        xv[loc_off<P>(la) + k] = f[la] >= 0 ? (double)x[(f[la] + k) * ld + t] : 0.0;
+    int code = ocode[w * kWave + l];
+    fac::Orient<P, double>(code).in(xv);
+    fac::mass_product<P, double>(xv, g, m);
 #pragma unroll
-    for (int i = 0; i < N; ++i) y[i] = C{0, 0};
+    for (int i = 0; i < N; ++i) m[i] = om * swap_pair(m[i]);
+    __builtin_amdgcn_sched_barrier(0);  // one part's intermediates at a time
+    fac::curl_product<P, double>(xv, h, y);
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-#pragma unroll
-      for (int j = i; j < N; ++j) {
-        const int k = i * N - (i * (i - 1)) / 2 + (j - i);
-        const unsigned zm = zero_mask<P>(k);
-        const bool hasM = (zm & 0x3Fu) != 0x3Fu, hasK = (zm & 0xFC0u) != 0xFC0u;
-        if (!hasM && !hasK) continue;
-        const C a = e[k];  // (K_ij, M_ij)
-        if (hasK) {
-          y[i].x = fma(a.x, xv[j].x, y[i].x);
-          y[i].y = fma(a.x, xv[j].y, y[i].y);
-          if (j != i) {
-            y[j].x = fma(a.x, xv[i].x, y[j].x);
-            y[j].y = fma(a.x, xv[i].y, y[j].y);
-          }
-        }
-        if (hasM) {  // -i omega mu0 M_ij
-          const RT wm = om * a.y;
-          y[i].x = fma(wm, xv[j].y, y[i].x);
-          y[i].y = fma(-wm, xv[j].x, y[i].y);
-          if (j != i) {
-            y[j].x = fma(wm, xv[i].y, y[j].x);
-            y[j].y = fma(-wm, xv[i].x, y[j].y);
-          }
-        }
-      }
-    }
+    for (int i = 0; i < N; ++i) y[i] += m[i];
+    // x^T y is the same in the code-0 functions
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      ye[(((int64_t)w * N + i) * kWave + l) * R + r] = y[i];
-      const double xr = xv[i].x, xi = xv[i].y, yr = y[i].x, yi = y[i].y;
-      dre += xr * yr - xi * yi;
-      dim += xr * yi + xi * yr;
+      dre += xv[i] * y[i];
+      dim += xv[i] * swap_pair(y[i]);
     }
+    asm("" : "+s"(code));  // the coefficients again, not kept through the products
+    fac::Orient<P, double>(code).out(y);
+#pragma unroll
+    for (int i = 0; i < N; ++i) ye[((w * N + i) * kWave + l) * ld + t] = (R)y[i];
   }
   if (dpart) {
-    dpart[(int64_t)r * gridDim.x + blockIdx.x] = dre;
-    dpart[((int64_t)R + r) * gridDim.x + blockIdx.x] = dim;
+    // real: re re - im im; imaginary: re im + im re
+    dre -= swap_pair(dre);
+    dim += swap_pair(dim);
+    dpart[((t & 1) * (int64_t)nrhs + r) * gridDim.x + blockIdx.x] = (t & 1) ? dim : dre;
   }
 }
 
@@ -661,11 +640,11 @@ struct ElemOp {
   float* tab32 = nullptr;
   double2* ye64 = nullptr;
   float2* ye32 = nullptr;
+  // packed element orientation per slot (orient_of)
+  int32_t* ocode = nullptr;
   // multi-right-hand-side products (eop_multi_prepare): raw coefficients in
-  // slot order (mass part without -omega mu0) and per entry pair {offset in
-  // the combination's table, zero mask}
+  // slot order (mass part without -omega mu0)
   double* coefm = nullptr;
-  int2* pdesc = nullptr;
   // p = 3 complex128 products on the matrix cores (k_eop_mfma3): Tf fragments
   // per combination and the kept (c, j) columns
   double* afrag = nullptr;
@@ -806,19 +785,8 @@ int eop_multi_prepare(ElemOp* op, const void* ws, hipStream_t st) {
   if (op->p > 2)
     PG_FAIL(PG_ERR_UNSUPPORTED, "multi-right-hand-side element products: p <= 2 only");
   if (op->coefm) return PG_OK;
-  const int N = op->N, NP = N * (N + 1) / 2;
-  std::vector<int2> pd(NP);
-  int o = 0;
-  for (int k = 0; k < NP; ++k) {
-    const unsigned zm = op->p == 1 ? eop::zero_mask<1>(k) : eop::zero_mask<2>(k);
-    pd[k] = make_int2(o, (int)zm);
-    o += 12 - eop::popcount12(zm);
-  }
   int rc;
-  if ((rc = op->alloc(&op->pdesc, NP)) != PG_OK || (rc = op->alloc(&op->coefm, op->nw * kWave * 12)) != PG_OK)
-    return rc;
-  PG_HIP(hipMemcpyAsync(op->pdesc, pd.data(), NP * sizeof(int2), hipMemcpyHostToDevice, st));
-  PG_HIP(hipStreamSynchronize(st));
+  if ((rc = op->alloc(&op->coefm, op->nw * kWave * 12)) != PG_OK) return rc;
   const int64_t nslot = op->nw * kWave;
   const dim3 g((unsigned)((nslot + 255) / 256)), b(256);
   hipLaunchKernelGGL(eop::k_eop_coef<double>, g, b, 0, st, nslot, op->perm,
@@ -852,24 +820,29 @@ const float2* eop_local_segments(const ElemOp* op, const int32_t* done, int dstr
   return op->ye32;
 }
 
-// workgroups of R threads; a slot group split over 256 / R workgroups (at
-// most 4), about 4 waves per slot group at every width
-static int multi_split(int R) { return std::max(1, std::min(4, 256 / R)); }
-int64_t eop_multi_parts(const ElemOp* op, int R) { return op->nw * multi_split(R); }
+// workgroups per slot group: 16 elements each on large meshes, fewer (down to
+// one) while the launch has under eight waves per SIMD of the chip
+static int multi_split(const ElemOp* op, int R) {
+  int split = 4;
+  while (split < kWave && op->nw * split * (R / 32) < 8192) split *= 2;
+  return split;
+}
+int64_t eop_multi_parts(const ElemOp* op, int R) { return op->nw * multi_split(op, R); }
 
 template <typename RT>
 static void multi_local(const ElemOp* op, int R, const int32_t* done, const double* omu,
                         const typename eop::Cx<RT>::T* x, typename eop::Cx<RT>::T* ye,
                         double* part, hipStream_t st) {
-  const int split = multi_split(R);
-  const dim3 g((unsigned)(op->nw * split)), b(R);
-  const double* tab = op->tab64;
+  const int split = multi_split(op, R);
+  const dim3 g((unsigned)(op->nw * split)), b(2 * R);
+  const RT* xr = reinterpret_cast<const RT*>(x);
+  RT* yr = reinterpret_cast<RT*>(ye);
   if (op->p == 1)
     hipLaunchKernelGGL((eop::k_meop_local<1, RT>), g, b, 0, st, op->nw, R, split, done,
-                       op->wcombo, op->edofs, op->coefm, tab, op->pdesc, omu, x, ye, part);
+                       op->edofs, op->ocode, op->coefm, omu, xr, yr, part);
   else
     hipLaunchKernelGGL((eop::k_meop_local<2, RT>), g, b, 0, st, op->nw, R, split, done,
-                       op->wcombo, op->edofs, op->coefm, tab, op->pdesc, omu, x, ye, part);
+                       op->edofs, op->ocode, op->coefm, omu, xr, yr, part);
 }
 void eop_multi_local(const ElemOp* op, int R, const int32_t* done, const double* omu,
                      const double2* x, double2* ye, double* part, hipStream_t st) {
@@ -1000,6 +973,9 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   }
   const int64_t nw = (int64_t)wcombo.size(), nslot = nw * kWave;
   if (nslot * N >= (1LL << 31)) PG_FAIL(PG_ERR_UNSUPPORTED, "too many elements");
+  std::vector<int32_t> hoc(nslot, 0);  // orientation per slot
+  for (int64_t s = 0; s < nslot; ++s)
+    if (perm[s] >= 0) hoc[s] = hor[perm[s]];
   // per slot and local entity: the entity's first DOF (-1: PEC or empty)
   std::vector<int32_t> hed((size_t)nslot * nle, -1);
   for (int64_t s = 0; s < nslot; ++s) {
@@ -1143,6 +1119,7 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   PG_A(op->wcombo, nw);
   PG_A(op->edofs, hed.size());
   PG_A(op->perm, nslot);
+  PG_A(op->ocode, nslot);
   PG_A(op->gm, nblocks);
   PG_A(op->gslot, gslot.size());
   PG_A(op->coef64, nslot * 12);
@@ -1176,6 +1153,7 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   } up[] = {{op->wcombo, wcombo.data(), wcombo.size() * sizeof(int32_t)},
             {op->edofs, hed.data(), hed.size() * sizeof(int32_t)},
             {op->perm, perm.data(), perm.size() * sizeof(int32_t)},
+            {op->ocode, hoc.data(), hoc.size() * sizeof(int32_t)},
             {op->gm, gm.data(), gm.size() * sizeof(int4)},
             {op->gslot, gslot.data(), gslot.size() * sizeof(int32_t)},
             {op->tab64, tab.data(), tab.size() * sizeof(double)},
