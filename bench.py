@@ -44,13 +44,17 @@ def spmv_bytes(nnz, n, bv):
 
 
 def eop_flops(n_elems, p):
-    """Algorithmic flops of one element-by-element product.  Per element and
-    upper-triangle pair (i, j >= i): the mass part of the entry from its m
+    """Flops of one element-by-element product.  p = 1, 2: the additions and
+    multiplications of the factored product (csrc/pg_factor.h) for one real
+    vector (orientation, curl, mass, their sum), twice per element.  p = 3: per
+    element and upper-triangle pair (i, j >= i): the mass part of the entry from its m
     nonzero table components (one MUL + m-1 FMA = 2m-1 flops), the curl-curl
     part likewise, then each nonzero part applied to x_j (2 FMA = 4 flops) and,
     off the diagonal, to x_i (4 more).  The components that vanish for every
     orientation (csrc/pg_eop_mask.h) are not computed and not counted."""
     import re
+    if p <= 2:
+        return n_elems * 2 * (162 if p == 1 else 822)
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "petgem_amd", "csrc",
                         "pg_eop_mask.h")
     body = re.search(r"kZero%d\[\d+\] = \{([^}]*)\}" % p, open(path).read()).group(1)
@@ -72,11 +76,10 @@ def spmv_key(code, dmax, vt, p=2):
     """Kernel name (as the profile summaries print it) of the solve's SpMV from the
     solver's configuration code kind*1000 + G*10 + U."""
     kind, g, u = code // 1000, (code % 1000) // 10, code % 10
-    if kind == 3:  # element products (p = 2: paired gathers on the solver's aligned vectors)
-        if p == 3 and vt != "float2":
-            return "k_eop_mfma3"  # p = 3 complex128: the matrix-core kernel
-        return "k_eop_local<{},{},{}>".format(p, "float" if vt == "float2" else "double",
-                                              "true" if p == 2 else "false")
+    if kind == 3:  # element products
+        if p == 3:  # complex128: the matrix-core kernel
+            return "k_eop_local3" if vt == "float2" else "k_eop_mfma3"
+        return "k_eop_fac<{},{}>".format(p, "float" if vt == "float2" else "double")
     if kind == 2:
         return f"k_spmv_er2<{g},{u},1,{vt},{vt}>"
     if kind == 1:

@@ -2,17 +2,17 @@
 //     A = sum_e P_e^T (K_e - i omega mu0 M_e) P_e,   PEC rows and columns -> identity,
 // for gfx950, as an alternative to the CSR SpMV inside the Krylov solver.
 //
-// The element matrices are never stored.  With the reference-tensor form used
-// by the assembly (K_e, M_e linear in 6 + 6 geometric coefficients, tables T
-// per orientation variant), one element's product costs about 4100 FMAs
-// (symmetric, upper triangle) on 288 bytes of input and output per element
-// in complex64, against about 2800 bytes per element for streaming the CSR
-// rows the element contributes to.  The product is split in two kernels:
+// The element matrices are never stored.  The product is split in two kernels:
 //
-//  k_eop_local  one lane per element, 64 elements of one orientation
-//               combination per wavefront, so every table entry is a
-//               wave-uniform (scalar) load; writes the element's n local
-//               results y_e = A_e x_e (slot layout [wave][i][lane]).
+//  k_eop_fac    p = 1, 2: two lanes per element (real and imaginary part), any
+//               orientation, K_e x and M_e x from 12 geometric coefficients by
+//               expanding field and curl in Bernstein monomials (pg_factor.h):
+//               820 operations per real vector and no table at p = 2; writes
+//               the element's n local results y_e = A_e x_e (slot layout
+//               [group][i][element of 64]).
+//  k_eop_local3, k_eop_mfma3   p = 3 (complex64, complex128): 64 elements of one
+//               orientation combination per wave, entries from the
+//               combination's reference table.
 //  k_eop_sum    one thread per mesh entity (edge, face), in the entity
 //               schedule: sums the entity's local results over its elements
 //               in a fixed order (atomic-free, bitwise reproducible), and
@@ -42,19 +42,11 @@ namespace eop {
 
 constexpr int kBS = 256;
 constexpr int kMaxGrid = 2048;
-// workgroup size of the element products: one wavefront in complex64
-// (measured 10 % faster than four: finer dispatch of the last, partial round
-// of waves), four in complex128 (4 % faster than one at two waves per SIMD)
+// waves per SIMD the factored products are compiled for: three in complex128
+// (at most 168 registers), six in complex64
 template <typename R>
-constexpr int local_bs() {
-  return sizeof(R) == 4 ? 64 : 256;
-}
-// waves per SIMD the element products are compiled for: five in complex64 at
-// p <= 2 (at most 102 VGPRs; the register allocator otherwise settles on 104
-// and four); at p = 3 the 45 values of p and of the products need about 190
-template <int P, typename R>
-constexpr int min_waves() {
-  return sizeof(R) == 4 && P <= 2 ? 5 : 1;
+constexpr int fac_waves() {
+  return sizeof(R) == 8 ? 3 : 6;
 }
 constexpr double kMu0 = 4.0 * 3.14159265358979323846 * 1e-7;  // petgem/solver.py:175
 
@@ -63,12 +55,10 @@ struct Cx;
 template <>
 struct Cx<double> {
   using T = double2;
-  using T2 = double4;  // two consecutive complex values
 };
 template <>
 struct Cx<float> {
   using T = float2;
-  using T2 = float4;
 };
 
 // local entities carrying DOFs (edges; faces from p = 2; the volume at p = 3),
@@ -113,34 +103,6 @@ __device__ inline double2 to_d(float2 v) { return make_double2(v.x, v.y); }
 __device__ inline void store(double2* p, double2 v) { *p = v; }
 __device__ inline void store(float2* p, double2 v) { *p = make_float2((float)v.x, (float)v.y); }
 
-// Table value `off` of a wavefront's element products, streamed through
-// scalar registers in batches of KB values, double buffered: at the start of
-// batch b the wave waits for the scalar loads in flight (batch b, issued one
-// batch earlier), issues the loads of batch b + 1 and then computes with batch
-// b, so that every scalar load has one batch of arithmetic to arrive.  Left to
-// itself the compiler issues each load just before its first use and waits for
-// it at once; measured at C2 (p = 2) the batches take the complex128 product
-// from 0.205 to 0.153 ms and the complex64 product from 0.086 to 0.069 ms.
-// Scalar loads can return out of order, so the wait is for all of them
-// (lgkmcnt(0)).  `off` is a compile-time constant after unrolling; the tables
-// are zero-padded to a multiple of KB, so whole batches load unconditionally
-// (conditional loads here cost the compiler minutes).
-constexpr unsigned kWaitScalarLoads = 0xC07F;  // s_waitcnt lgkmcnt(0), other counters untouched
-template <int KB, int NTS, typename R>
-__device__ __forceinline__ R tab_next(const R* __restrict__ t, R (&tb)[2][KB], int off) {
-  if (off % KB == 0) {
-    const int b = off / KB;
-    __builtin_amdgcn_s_waitcnt(kWaitScalarLoads);
-    __builtin_amdgcn_sched_barrier(0);
-    if ((b + 1) * KB < NTS) {
-#pragma unroll
-      for (int k = 0; k < KB; ++k) tb[(b + 1) & 1][k] = t[(b + 1) * KB + k];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  return tb[(off / KB) & 1][off % KB];
-}
-
 // the value of the neighbouring lane (lane ^ 1)
 __device__ inline int swap_pair(int v) {
   return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);  // quad_perm [1, 0, 3, 2]
@@ -170,37 +132,107 @@ __device__ inline void write_partials(double (&v)[NV], double* part) {
 }
 
 // ---------------------------------------------------------------------------
-// local products.  coef[w][c][lane]: c < 6 the mass coefficients times
-// -omega mu0, c >= 6 the curl-curl coefficients; tab[combo][...] the table
-// components of the pairs k = (i, j >= i) (row-major upper triangle; per pair
-// c < 6 mass, c >= 6 curl-curl), structural zeros left out.  edofs[w][la][lane]
-// = first global DOF of local entity la (its P DOFs at p = 1 and 2 are
-// consecutive: 1 at p = 1, 2 at p = 2), -1 for a PEC entity or an empty lane
-// (its x is taken as 0).  PAIR: at p = 2 both DOFs of an entity are loaded as
-// one 16-byte (complex64) or 32-byte (complex128) value; the first DOF of
-// every entity is even, so this needs x aligned to that size.
+// local products, p = 1 and 2, in factored form (pg_factor.h).  Slots: group w
+// of 64 elements, element l of the group; edofs[w][la][l] = first global DOF of
+// local entity la, -1 for a PEC entity or an empty slot (its x is taken as 0);
+// ocode[w][l] the packed orientation; coef[w][c][l]: c < 6 the mass
+// coefficients times -omega mu0, c >= 6 the curl-curl coefficients.  Two
+// neighbouring lanes take one element: lane 2 i the real part of x, lane
+// 2 i + 1 the imaginary part, each forming K x and M x of its real vector and
+// giving the other M x (y_re = K x_re - M' x_im, y_im = K x_im + M' x_re), so
+// a wave holds 32 elements and the registers of one real vector each.
+// Bound: memory, about 220 MB of indices, coefficients, x and local results in
+// 48 us at 384 000 elements in complex128 (4.6 TB/s; a copy reaches 5.1).  With
+// one lane per element of one orientation combination per wave, entries formed
+// from scalar table loads (two waves per SIMD, waiting for the scalar cache),
+// it took 107 us; on a mesh of 55 566 elements with arbitrary orientations, one
+// element per wave, 420 us against 12 us now.
 // ---------------------------------------------------------------------------
-template <int P, typename R, bool PAIR>
-__global__ void __launch_bounds__(local_bs<R>(), (min_waves<P, R>())) k_eop_local(int64_t nw, const int32_t* __restrict__ done,
-                                                   const int32_t* __restrict__ wseg, int dstride,
-                                                   const int32_t* __restrict__ wcombo,
-                                                   const int32_t* __restrict__ edofs,
-                                                   const R* __restrict__ coef,
-                                                   const R* __restrict__ tab,
-                                                   const typename Cx<R>::T* __restrict__ x,
-                                                   typename Cx<R>::T* __restrict__ ye) {
-  using C = typename Cx<R>::T;
-  using C2 = typename Cx<R>::T2;
-  constexpr int N = P * (P + 2) * (P + 3) / 2;
+template <int P, typename R>
+__global__ void __launch_bounds__(kBS, fac_waves<R>()) k_eop_fac(
+    int64_t nw, const int32_t* __restrict__ done, const int32_t* __restrict__ wseg, int dstride,
+    const int32_t* __restrict__ edofs, const int32_t* __restrict__ ocode,
+    const R* __restrict__ coef, const R* __restrict__ x, R* __restrict__ ye) {
+  constexpr int N = fac::n_dofs<P>();
+  constexpr int NLE = n_local_entities<P>();
+  if (done && !wseg && *done) return;
+  // XCD-contiguous ranges of slot groups (workgroup b runs on XCD b % 8)
+  const int64_t nb = gridDim.x;
+  int64_t b = blockIdx.x;
+  if (nb % 8 == 0) b = (b % 8) * (nb / 8) + b / 8;
+  const int64_t hw = b * (kBS / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int64_t w = hw >> 1;
+  if (w >= nw) return;
+  // segmented operator: the group's mesh has converged
+  if (wseg && done[(int64_t)__builtin_amdgcn_readfirstlane(wseg[w]) * dstride]) return;
+  const int lane = threadIdx.x % kWave, part = lane & 1;
+  const int l = (int)(hw & 1) * (kWave / 2) + (lane >> 1);
+  // all index and coefficient loads first, then all gathers, unconditionally
+  // (a masked entity reads x[0] and is zeroed after), so that the wave waits
+  // for memory twice rather than once per DOF
+  int f[NLE];
+#pragma unroll
+  for (int la = 0; la < NLE; ++la) f[la] = edofs[(w * NLE + la) * kWave + l];
+  int code = ocode[w * kWave + l];
+  R g[6], h[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    g[c] = coef[(w * 12 + c) * kWave + l];
+    h[c] = coef[(w * 12 + 6 + c) * kWave + l];
+  }
+  R xv[N], y[N], m[N];
+#pragma unroll
+  for (int la = 0; la < NLE; ++la) {
+    const R* xe = x + 2 * (int64_t)(f[la] >= 0 ? f[la] : 0) + part;
+#pragma unroll
+    for (int k = 0; k < loc_nd<P>(la); ++k) xv[loc_off<P>(la) + k] = xe[2 * k];
+  }
+#pragma unroll
+  for (int la = 0; la < NLE; ++la)
+#pragma unroll
+    for (int k = 0; k < loc_nd<P>(la); ++k)
+      xv[loc_off<P>(la) + k] = f[la] >= 0 ? xv[loc_off<P>(la) + k] : R(0);
+  fac::Orient<P, R>(code).in(xv);
+  fac::mass_product<P, R>(xv, g, m);
+  const R sg = part ? R(1) : R(-1);
+#pragma unroll
+  for (int i = 0; i < N; ++i) m[i] = sg * swap_pair(m[i]);
+  __builtin_amdgcn_sched_barrier(0);  // one product's intermediates at a time
+  fac::curl_product<P, R>(xv, h, y);
+#pragma unroll
+  for (int i = 0; i < N; ++i) y[i] += m[i];
+  asm("" : "+v"(code));  // the coefficients again, not kept through the products
+  fac::Orient<P, R>(code).out(y);
+#pragma unroll
+  for (int i = 0; i < N; ++i) ye[((w * N + i) * kWave + l) * 2 + part] = y[i];
+}
+
+// ---------------------------------------------------------------------------
+// local products, p = 3 in complex64: one lane per element, 64 elements of one
+// orientation combination per wave, so every table value is a wave-uniform
+// (scalar) load.  tab[combo][...]: the table components of the pairs k = (i,
+// j >= i) (row-major upper triangle; per pair c < 6 mass, c >= 6 curl-curl),
+// structural zeros left out.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(kWave) k_eop_local3(int64_t nw, const int32_t* __restrict__ done,
+                                                      const int32_t* __restrict__ wseg,
+                                                      int dstride,
+                                                      const int32_t* __restrict__ wcombo,
+                                                      const int32_t* __restrict__ edofs,
+                                                      const float* __restrict__ coef,
+                                                      const float* __restrict__ tab,
+                                                      const float2* __restrict__ x,
+                                                      float2* __restrict__ ye) {
+  using R = float;
+  using C = float2;
+  constexpr int P = 3, N = 45;
   constexpr int NLE = n_local_entities<P>();
   static_assert(N == loc_off<P>(NLE - 1) + loc_nd<P>(NLE - 1), "entity DOFs");
   if (done && !wseg && *done) return;
   // XCD-contiguous ranges of waves (workgroup b runs on XCD b % 8)
   const int64_t nb = gridDim.x;
-  int64_t b = blockIdx.x;
-  if (nb % 8 == 0) b = (b % 8) * (nb / 8) + b / 8;
-  const int64_t w =
-      b * (local_bs<R>() / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  int64_t w = blockIdx.x;
+  if (nb % 8 == 0) w = (w % 8) * (nb / 8) + w / 8;
   if (w >= nw) return;
   // segmented operator: the wave's mesh has converged
   if (wseg && done[(int64_t)__builtin_amdgcn_readfirstlane(wseg[w]) * dstride]) return;
@@ -208,20 +240,6 @@ __global__ void __launch_bounds__(local_bs<R>(), (min_waves<P, R>())) k_eop_loca
   const int combo = __builtin_amdgcn_readfirstlane(wcombo[w]);
   constexpr int NTS = table_stride<P>();  // constant-evaluated, not a loop at run time
   const R* __restrict__ t = tab + (int64_t)combo * NTS;
-  // first batch of table values (scalar loads) in flight during the gathers;
-  // p = 3 (1035 entry pairs, a 17 600-instruction body) keeps the compiler's
-  // own schedule
-  constexpr bool kPipe = P <= 2;
-  constexpr int KB = sizeof(R) == 8 ? 16 : 32;
-  R tb[2][KB];
-  if constexpr (kPipe) {
-#pragma unroll
-    for (int k = 0; k < KB; ++k) tb[0][k] = t[k];
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  // all index and coefficient loads first, then all gathers, unconditionally
-  // (a masked entity reads x[0] and is zeroed after), so that the wave waits
-  // for memory twice rather than once per DOF
   int fv[NLE];
 #pragma unroll
   for (int la = 0; la < NLE; ++la) fv[la] = edofs[(w * NLE + la) * kWave + lane];
@@ -232,14 +250,8 @@ __global__ void __launch_bounds__(local_bs<R>(), (min_waves<P, R>())) k_eop_loca
 #pragma unroll
   for (int la = 0; la < NLE; ++la) {
     const int f = fv[la] >= 0 ? fv[la] : 0;
-    if (P == 2 && PAIR) {
-      const C2 v = *reinterpret_cast<const C2*>(x + f);
-      xv[2 * la] = C{v.x, v.y};
-      xv[2 * la + 1] = C{v.z, v.w};
-    } else {
 #pragma unroll
-      for (int k = 0; k < loc_nd<P>(la); ++k) xv[loc_off<P>(la) + k] = x[f + k];
-    }
+    for (int k = 0; k < loc_nd<P>(la); ++k) xv[loc_off<P>(la) + k] = x[f + k];
   }
 #pragma unroll
   for (int la = 0; la < NLE; ++la)
@@ -262,7 +274,7 @@ __global__ void __launch_bounds__(local_bs<R>(), (min_waves<P, R>())) k_eop_loca
 #pragma unroll
       for (int c = 0; c < 6; ++c)
         if (!((zm >> c) & 1)) {
-          const R tv = kPipe ? tab_next<KB, NTS>(t, tb, off) : t[off];
+          const R tv = t[off];
           im = has_im ? fma(cf[c], tv, im) : cf[c] * tv;
           has_im = true;
           ++off;
@@ -270,7 +282,7 @@ __global__ void __launch_bounds__(local_bs<R>(), (min_waves<P, R>())) k_eop_loca
 #pragma unroll
       for (int c = 6; c < 12; ++c)
         if (!((zm >> c) & 1)) {
-          const R tv = kPipe ? tab_next<KB, NTS>(t, tb, off) : t[off];
+          const R tv = t[off];
           re = has_re ? fma(cf[c], tv, re) : cf[c] * tv;
           has_re = true;
           ++off;
@@ -626,7 +638,6 @@ __global__ void k_eop_coef(int64_t nslot, const int32_t* __restrict__ perm,
 
 struct ElemOp {
   int p = 0, N = 0, D = 1;
-  bool even_entities = false;  // every entity's first DOF even: paired gathers allowed
   int64_t E = 0, ndof = 0, nent = 0, nw = 0;
   int ncombo = 0, grid = 1;
   int32_t* wcombo = nullptr;
@@ -679,49 +690,47 @@ bool eop_supports(const ElemOp* op, bool complex128) {
 }
 int64_t eop_ndof(const ElemOp* op) { return op->ndof; }
 
-// element products of waves [w0, w0 + nwr) (all waves: 0, op->nw)
+// element products of slot groups [w0, w0 + nwr) (all groups: 0, op->nw)
 template <typename R>
 static void launch_local(const ElemOp* op, const int32_t* done, const int32_t* wseg, int dstride,
                          const typename eop::Cx<R>::T* x, typename eop::Cx<R>::T* ye,
                          const R* coef, const R* tab, hipStream_t st, int64_t w0 = 0,
                          int64_t nwr = -1) {
-  using C = typename eop::Cx<R>::T;
   if (nwr < 0) nwr = op->nw;
   if (nwr <= 0) return;
   const int nle = op->p == 1 ? 6 : (op->p == 2 ? 10 : 11);
-  const int32_t* wc = op->wcombo + w0;
   const int32_t* ed = op->edofs + w0 * nle * kWave;
   const int32_t* ws = wseg ? wseg + w0 : nullptr;
   coef += w0 * 12 * kWave;
   ye += w0 * op->N * kWave;
-  const int wpb = eop::local_bs<R>() / kWave;
-  int64_t nbl = (nwr + wpb - 1) / wpb;
-  if (nbl >= 64) nbl = (nbl + 7) / 8 * 8;
-  const dim3 gl((unsigned)nbl), bll(wpb * kWave);
-  const bool pair_ok =
-      op->even_entities && reinterpret_cast<uintptr_t>(x) % (2 * sizeof(C)) == 0;
-  if (op->p == 1) {
-    hipLaunchKernelGGL((eop::k_eop_local<1, R, false>), gl, bll, 0, st, nwr, done, ws, dstride,
-                       wc, ed, coef, tab, x, ye);
-  } else if (op->p == 3) {
-    // complex64: one lane per element; complex128: the matrix-core kernel (the
-    // values of x and of the products do not fit one lane)
-    if constexpr (sizeof(R) == 4) {
-      hipLaunchKernelGGL((eop::k_eop_local<3, R, false>), gl, bll, 0, st, nwr, done, ws,
-                         dstride, wc, ed, coef, tab, x, ye);
-    } else {
-      int64_t nbm = nwr;
-      if (nbm >= 64) nbm = (nbm + 7) / 8 * 8;
-      hipLaunchKernelGGL(eop::k_eop_mfma3, dim3((unsigned)nbm), dim3(kWave), 0, st, nwr, done,
-                         ws, dstride, wc, ed, coef, op->afrag, op->kcol, op->nks, x, ye);
-    }
-  } else if (pair_ok) {
-    hipLaunchKernelGGL((eop::k_eop_local<2, R, true>), gl, bll, 0, st, nwr, done, ws, dstride,
-                       wc, ed, coef, tab, x, ye);
-  } else {
-    hipLaunchKernelGGL((eop::k_eop_local<2, R, false>), gl, bll, 0, st, nwr, done, ws, dstride,
-                       wc, ed, coef, tab, x, ye);
+  if (op->p <= 2) {
+    const int gpb = eop::kBS / (2 * kWave);  // slot groups per workgroup, two waves each
+    int64_t nbl = (nwr + gpb - 1) / gpb;
+    if (nbl >= 64) nbl = (nbl + 7) / 8 * 8;
+    const dim3 g((unsigned)nbl), b(eop::kBS);
+    const int32_t* oc = op->ocode + w0 * kWave;
+    const R* xr = reinterpret_cast<const R*>(x);
+    R* yr = reinterpret_cast<R*>(ye);
+    if (op->p == 1)
+      hipLaunchKernelGGL((eop::k_eop_fac<1, R>), g, b, 0, st, nwr, done, ws, dstride, ed, oc,
+                         coef, xr, yr);
+    else
+      hipLaunchKernelGGL((eop::k_eop_fac<2, R>), g, b, 0, st, nwr, done, ws, dstride, ed, oc,
+                         coef, xr, yr);
+    return;
   }
+  // p = 3: one wave per slot group.  complex64: one lane per element; complex128:
+  // the matrix-core kernel (the values of x and of the products do not fit one lane)
+  int64_t nbl = nwr;
+  if (nbl >= 64) nbl = (nbl + 7) / 8 * 8;
+  const dim3 g((unsigned)nbl), b(kWave);
+  const int32_t* wc = op->wcombo + w0;
+  if constexpr (sizeof(R) == 4)
+    hipLaunchKernelGGL(eop::k_eop_local3, g, b, 0, st, nwr, done, ws, dstride, wc, ed, coef, tab,
+                       x, ye);
+  else
+    hipLaunchKernelGGL(eop::k_eop_mfma3, g, b, 0, st, nwr, done, ws, dstride, wc, ed, coef,
+                       op->afrag, op->kcol, op->nks, x, ye);
 }
 
 template <typename R>
@@ -921,11 +930,12 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   } else {
     std::iota(pos.begin(), pos.end(), 0);
   }
-  // orientation combinations
+  // orientation combinations (p = 3, whose waves hold one combination each; at
+  // p <= 2 the products take any orientation per lane)
   std::map<int, int> cid;
   std::vector<int> combos;
-  std::vector<int32_t> ec(E);
-  for (int64_t e = 0; e < E; ++e) {
+  std::vector<int32_t> ec(E, 0);
+  for (int64_t e = 0; p == 3 && e < E; ++e) {
     auto it = cid.find(hor[e]);
     if (it == cid.end()) {
       it = cid.emplace(hor[e], (int)combos.size()).first;
@@ -933,8 +943,8 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     }
     ec[e] = it->second;
   }
-  // element order: by segment (multi-mesh operator), by combination, then by
-  // the earliest schedule position of the element's entities (spatial order
+  // element order: by segment (multi-mesh operator), by combination (p = 3), then
+  // by the earliest schedule position of the element's entities (spatial order
   // when the schedule is)
   std::vector<int64_t> key(E);
   std::vector<int32_t> es(E, 0);
@@ -958,7 +968,7 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   std::stable_sort(sorted.begin(), sorted.end(), [&](int64_t a, int64_t b) {
     return es[a] != es[b] ? es[a] < es[b] : key[a] < key[b];
   });
-  // waves of 64 elements of one combination (and one segment)
+  // slot groups of 64 elements of one segment (p = 3: and one combination)
   std::vector<int32_t> wcombo, perm, wsg;
   for (int64_t k = 0; k < E;) {
     const int c = ec[sorted[k]], sg = es[sorted[k]];
@@ -1013,45 +1023,42 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     const int64_t g = order ? order[i] : i;
     gm[i] = make_int4(bp[g], bp[g + 1] - bp[g], (int)start[i], (int)start[i + 1]);
   }
-  // per-combination tables of the upper triangle without the structural zeros
-  // (which must vanish here too: a stale mask would drop real terms)
-  const int V = n_variants(p), nc = (int)combos.size();
-  const int NT = p == 1   ? eop::n_table_entries<1>()
-                 : p == 2 ? eop::n_table_entries<2>()
-                          : eop::n_table_entries<3>();
-  const int NTS = p == 1   ? eop::table_stride<1>()
-                  : p == 2 ? eop::table_stride<2>()
-                           : eop::table_stride<3>();
-  std::vector<double> T((size_t)V * V * 12);
-  int rc = pg_tables_host(p, T.data(), (int64_t)T.size());
-  if (rc != PG_OK) return rc;
-  double tmax = 0.0;
-  for (double v : T) tmax = std::max(tmax, std::fabs(v));
+  // p = 3: per-combination tables of the upper triangle without the structural
+  // zeros (which must vanish here too: a stale mask would drop real terms)
+  const int nc = (int)combos.size();
+  const int NT = eop::n_table_entries<3>(), NTS = eop::table_stride<3>();
+  int rc = PG_OK;
   std::vector<double> tab((size_t)nc * NTS, 0.0);
-  std::vector<int> var(N);
-  for (int c = 0; c < nc; ++c) {
-    for (int la = 0; la < nle; ++la)
-      for (int k = 0; k < entity_ndof(la, p); ++k)
-        var[entity_local_offset(la, p) + k] =
-            entity_variant_base(la, orient_of(combos[c], la), p) + k;
-    int k = 0;
-    size_t o = (size_t)c * NTS;
-    for (int i = 0; i < N; ++i)
-      for (int j = i; j < N; ++j, ++k) {
-        const unsigned zm = p == 1   ? eop::zero_mask<1>(k)
-                            : p == 2 ? eop::zero_mask<2>(k)
-                                     : eop::zero_mask<3>(k);
-        for (int q = 0; q < 12; ++q) {
-          const double v = T[((size_t)var[i] * V + var[j]) * 12 + q];
-          if ((zm >> q) & 1) {
-            if (std::fabs(v) > 1e-15 * tmax)
-              PG_FAIL(PG_ERR_UNSUPPORTED, "element table entry (%d, %d, %d) is not zero", i, j, q);
-          } else {
-            tab[o++] = v;
+  if (p == 3) {
+    const int V = n_variants(p);
+    std::vector<double> T((size_t)V * V * 12);
+    if ((rc = pg_tables_host(p, T.data(), (int64_t)T.size())) != PG_OK) return rc;
+    double tmax = 0.0;
+    for (double v : T) tmax = std::max(tmax, std::fabs(v));
+    std::vector<int> var(N);
+    for (int c = 0; c < nc; ++c) {
+      for (int la = 0; la < nle; ++la)
+        for (int k = 0; k < entity_ndof(la, p); ++k)
+          var[entity_local_offset(la, p) + k] =
+              entity_variant_base(la, orient_of(combos[c], la), p) + k;
+      int k = 0;
+      size_t o = (size_t)c * NTS;
+      for (int i = 0; i < N; ++i)
+        for (int j = i; j < N; ++j, ++k) {
+          const unsigned zm = eop::zero_mask<3>(k);
+          for (int q = 0; q < 12; ++q) {
+            const double v = T[((size_t)var[i] * V + var[j]) * 12 + q];
+            if ((zm >> q) & 1) {
+              if (std::fabs(v) > 1e-15 * tmax)
+                PG_FAIL(PG_ERR_UNSUPPORTED, "element table entry (%d, %d, %d) is not zero", i, j,
+                        q);
+            } else {
+              tab[o++] = v;
+            }
           }
         }
-      }
-    if (o != (size_t)c * NTS + NT) PG_FAIL(PG_ERR_UNSUPPORTED, "element table size mismatch");
+      if (o != (size_t)c * NTS + NT) PG_FAIL(PG_ERR_UNSUPPORTED, "element table size mismatch");
+    }
   }
   std::vector<float> tab32(tab.begin(), tab.end());
   // p = 3: matrix-core fragments.  kcol = the (c, j) columns of Tf that are not
@@ -1097,9 +1104,6 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   op->p = p;
   op->N = N;
   op->D = maxd;
-  op->even_entities = true;
-  for (int64_t g = 0; g < nblocks; ++g)
-    if (bp[g] % 2) op->even_entities = false;
   op->E = E;
   op->ndof = ndof;
   op->nent = nblocks;

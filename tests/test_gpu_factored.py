@@ -62,3 +62,23 @@ def test_batch_products_on_arbitrary_orientations(p, n, nrhs, precision):
     err = float((X - ref).abs().max() / ref.abs().max())
     print(f"batch p={p} n={n} R={nrhs} {precision}: {err:.2e}", flush=True)
     assert err <= 1e-7
+
+
+@pytest.mark.parametrize("p,n,keep", [(1, 2, 1), (1, 3, 65), (2, 2, 31), (2, 2, 33), (2, 3, 64),
+                                      (2, 4, 129), (2, 4, None)])
+def test_products_on_arbitrary_orientations(p, n, keep):
+    """y = A x on the operator against the assembled CSR: element counts around the
+    32 elements of a wave, the 64 of a slot group and the 128 of a workgroup, in
+    both precisions and, for complex128, x at an address that is not a
+    multiple of 32 bytes.  Bars as for the structured grids: 1e-12 and 1e-5."""
+    T, mesh, asm, _ = _free(n, p, seed=n, keep=keep)
+    omega = core.omega_of(0.5)
+    vals = asm.assemble(omega)
+    eop = core.ElementOperator(asm, omega, None, mesh.entity_order())
+    g = torch.Generator(DEV).manual_seed(n)
+    xb = torch.randn((T.ndof + 1, 2), dtype=torch.float64, device=DEV, generator=g)
+    for x in (xb[:-1], xb[1:]):
+        ref = core.spmv(asm.plan, vals, x.contiguous())
+        err = float((eop.apply(x) - ref).abs().max() / ref.abs().max())
+        err32 = float((eop.apply(x.float()).double() - ref).abs().max() / ref.abs().max())
+        assert err <= 1e-12 and err32 <= 1e-5, (err, err32)
