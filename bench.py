@@ -44,32 +44,10 @@ def spmv_bytes(nnz, n, bv):
 
 
 def eop_flops(n_elems, p):
-    """Flops of one element-by-element product.  p = 1, 2: the additions and
-    multiplications of the factored product (csrc/pg_factor.h) for one real
-    vector (orientation, curl, mass, their sum), twice per element.  p = 3: per
-    element and upper-triangle pair (i, j >= i): the mass part of the entry from its m
-    nonzero table components (one MUL + m-1 FMA = 2m-1 flops), the curl-curl
-    part likewise, then each nonzero part applied to x_j (2 FMA = 4 flops) and,
-    off the diagonal, to x_i (4 more).  The components that vanish for every
-    orientation (csrc/pg_eop_mask.h) are not computed and not counted."""
-    import re
-    if p <= 2:
-        return n_elems * 2 * (162 if p == 1 else 822)
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "petgem_amd", "csrc",
-                        "pg_eop_mask.h")
-    body = re.search(r"kZero%d\[\d+\] = \{([^}]*)\}" % p, open(path).read()).group(1)
-    masks = [int(v, 16) for v in re.findall(r"0x[0-9a-f]+", body)]
-    n = p * (p + 2) * (p + 3) // 2
-    total, k = 0, 0
-    for i in range(n):
-        for j in range(i, n):
-            z = masks[k]
-            k += 1
-            for part in (z & 0x3F, (z >> 6) & 0x3F):
-                m = 6 - bin(part).count("1")
-                if m:
-                    total += 2 * m - 1 + (4 if j == i else 8)
-    return n_elems * total
+    """Flops of one element-by-element product: the additions and multiplications
+    of the factored product (csrc/pg_factor.h) for one real vector
+    (orientation, curl, mass, their sum), twice per element."""
+    return n_elems * 2 * {1: 162, 2: 822, 3: 3199}[p]
 
 
 def spmv_key(code, dmax, vt, p=2):
@@ -77,8 +55,6 @@ def spmv_key(code, dmax, vt, p=2):
     solver's configuration code kind*1000 + G*10 + U."""
     kind, g, u = code // 1000, (code % 1000) // 10, code % 10
     if kind == 3:  # element products
-        if p == 3:  # complex128: the matrix-core kernel
-            return "k_eop_local3" if vt == "float2" else "k_eop_mfma3"
         return "k_eop_fac<{},{}>".format(p, "float" if vt == "float2" else "double")
     if kind == 2:
         return f"k_spmv_er2<{g},{u},1,{vt},{vt}>"

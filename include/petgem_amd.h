@@ -311,11 +311,10 @@ int pg_solver_profile(void *solver, int reps, double *ms64, double *ms32, int32_
 /* ------------------------------------------------------------------------
  * Element-by-element operator: y = A x for A = sum_e (K_e - i omega mu0 M_e)
  * with the PEC rows and columns replaced by the identity, without the
- * assembled matrix (the element matrices are recomputed from the geometry
- * workspace and the reference tables at every product).  The same product as
+ * assembled matrix (each element's K x and M x are formed from its geometry
+ * coefficients at every product).  The same product as
  * MatMult on the assembled system (petgem/solver.py:584-590, inside KSPSolve),
- * to rounding.  Orders p = 1, 2 and 3, complex128 and complex64 (the p = 3
- * complex128 products on the FP64 matrix cores).
+ * to rounding.  Orders p = 1, 2 and 3, complex128 and complex64.
  *   ws        pg_element_geometry workspace (read at creation and refresh)
  *   dofs      device (E, n) element DOFs, as for the assembly plan
  *   block_ptr host (nblocks+1) DOF ranges of the mesh entities

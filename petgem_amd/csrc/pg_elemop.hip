@@ -4,36 +4,30 @@
 //
 // The element matrices are never stored.  The product is split in two kernels:
 //
-//  k_eop_fac    p = 1, 2: two lanes per element (real and imaginary part), any
+//  k_eop_fac    two lanes per element (real and imaginary part), any
 //               orientation, K_e x and M_e x from 12 geometric coefficients by
 //               expanding field and curl in Bernstein monomials (pg_factor.h):
-//               820 operations per real vector and no table at p = 2; writes
-//               the element's n local results y_e = A_e x_e (slot layout
-//               [group][i][element of 64]).
-//  k_eop_local3, k_eop_mfma3   p = 3 (complex64, complex128): 64 elements of one
-//               orientation combination per wave, entries from the
-//               combination's reference table.
+//               no table, 820 operations per real vector at p = 2 and 3 200 at
+//               p = 3; writes the element's n local results y_e = A_e x_e (slot
+//               layout [group][i][element of 64]).
 //  k_eop_sum    one thread per mesh entity (edge, face), in the entity
 //               schedule: sums the entity's local results over its elements
 //               in a fixed order (atomic-free, bitwise reproducible), and
 //               fuses the COCG dot product or the residual.
 //
-// Orders p = 1, 2 and 3 (n = 6, 20, 45), complex128 and complex64; the p = 3
-// complex128 products run on the FP64 matrix cores (k_eop_mfma3).  The
-// summation order differs from the assembled CSR's, so results agree with the
-// CSR SpMV to rounding.
+// Orders p = 1, 2 and 3 (n = 6, 20, 45), complex128 and complex64.  The summation
+// order differs from the assembled CSR's, so results agree with the CSR SpMV to
+// rounding.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
-#include <map>
 #include <numeric>
 #include <vector>
 
 #include "pg_basis.h"
 #include "pg_common.h"
 #include "pg_eop.h"
-#include "pg_eop_mask.h"
 #include "pg_factor.h"
 
 namespace pg {
@@ -42,11 +36,10 @@ namespace eop {
 
 constexpr int kBS = 256;
 constexpr int kMaxGrid = 2048;
-// waves per SIMD the factored products are compiled for: three in complex128
-// (at most 168 registers), six in complex64
-template <typename R>
+// waves per SIMD the element products are compiled for
+template <int P, typename R>
 constexpr int fac_waves() {
-  return sizeof(R) == 8 ? 3 : 6;
+  return P == 3 ? (sizeof(R) == 8 ? 1 : 2) : (sizeof(R) == 8 ? 3 : 6);
 }
 constexpr double kMu0 = 4.0 * 3.14159265358979323846 * 1e-7;  // petgem/solver.py:175
 
@@ -74,28 +67,6 @@ constexpr int loc_off(int la) {
 template <int P>
 constexpr int loc_nd(int la) {
   return la < 6 ? P : (la < 10 ? P * (P - 1) : P * (P - 1) * (P - 2) / 2);
-}
-
-// table components kept per orientation combination: those that are not
-// structural zeros (zero_mask); the kernel skips the zeros at compile time
-constexpr int popcount12(unsigned m) {
-  int n = 0;
-  for (int c = 0; c < 12; ++c) n += (m >> c) & 1;
-  return n;
-}
-template <int P>
-constexpr int n_table_entries() {
-  constexpr int N = P * (P + 2) * (P + 3) / 2;
-  int n = 0;
-  for (int k = 0; k < N * (N + 1) / 2; ++k) n += 12 - popcount12(zero_mask<P>(k));
-  return n;
-}
-// per-combination table stride: the entries zero-padded to a multiple of 32
-// values, so that the element products load whole batches unconditionally
-constexpr int kTabPad = 32;
-template <int P>
-constexpr int table_stride() {
-  return (n_table_entries<P>() + kTabPad - 1) / kTabPad * kTabPad;
 }
 
 __device__ inline double2 to_d(double2 v) { return v; }
@@ -132,8 +103,7 @@ __device__ inline void write_partials(double (&v)[NV], double* part) {
 }
 
 // ---------------------------------------------------------------------------
-// local products, p = 1 and 2, in factored form (pg_factor.h).  Slots: group w
-// of 64 elements, element l of the group; edofs[w][la][l] = first global DOF of
+// local products in factored form (pg_factor.h).  Slots: group w of 64 elements, element l of the group; edofs[w][la][l] = first global DOF of
 // local entity la, -1 for a PEC entity or an empty slot (its x is taken as 0);
 // ocode[w][l] the packed orientation; coef[w][c][l]: c < 6 the mass
 // coefficients times -omega mu0, c >= 6 the curl-curl coefficients.  Two
@@ -142,14 +112,17 @@ __device__ inline void write_partials(double (&v)[NV], double* part) {
 // giving the other M x (y_re = K x_re - M' x_im, y_im = K x_im + M' x_re), so
 // a wave holds 32 elements and the registers of one real vector each.
 // Bound: memory, about 220 MB of indices, coefficients, x and local results in
-// 48 us at 384 000 elements in complex128 (4.6 TB/s; a copy reaches 5.1).  With
-// one lane per element of one orientation combination per wave, entries formed
+// 48 us at 384 000 elements, p = 2, complex128 (4.6 TB/s; a copy reaches 5.1).
+// One lane per element of one orientation combination per wave, entries formed
 // from scalar table loads (two waves per SIMD, waiting for the scalar cache),
-// it took 107 us; on a mesh of 55 566 elements with arbitrary orientations, one
-// element per wave, 420 us against 12 us now.
+// took 107 us; on a mesh of 55 566 elements with arbitrary orientations, one
+// element per wave, 420 us against 12 us now.  p = 3, 82 944 elements: 20 us in
+// complex64 against 151 us from tables, 34 us in complex128 (302 registers, one
+// wave per SIMD; two waves with 256 are no faster) against 326 us as a dense
+// product with the tables on the FP64 matrix cores.
 // ---------------------------------------------------------------------------
 template <int P, typename R>
-__global__ void __launch_bounds__(kBS, fac_waves<R>()) k_eop_fac(
+__global__ void __launch_bounds__(kBS, (fac_waves<P, R>())) k_eop_fac(
     int64_t nw, const int32_t* __restrict__ done, const int32_t* __restrict__ wseg, int dstride,
     const int32_t* __restrict__ edofs, const int32_t* __restrict__ ocode,
     const R* __restrict__ coef, const R* __restrict__ x, R* __restrict__ ye) {
@@ -180,7 +153,7 @@ __global__ void __launch_bounds__(kBS, fac_waves<R>()) k_eop_fac(
     g[c] = coef[(w * 12 + c) * kWave + l];
     h[c] = coef[(w * 12 + 6 + c) * kWave + l];
   }
-  R xv[N], y[N], m[N];
+  R xv[N], y[N];
 #pragma unroll
   for (int la = 0; la < NLE; ++la) {
     const R* xe = x + 2 * (int64_t)(f[la] >= 0 ? f[la] : 0) + part;
@@ -192,234 +165,15 @@ __global__ void __launch_bounds__(kBS, fac_waves<R>()) k_eop_fac(
 #pragma unroll
     for (int k = 0; k < loc_nd<P>(la); ++k)
       xv[loc_off<P>(la) + k] = f[la] >= 0 ? xv[loc_off<P>(la) + k] : R(0);
-  fac::Orient<P, R>(code).in(xv);
-  fac::mass_product<P, R>(xv, g, m);
+  fac::orient_in<P>(code, xv);
   const R sg = part ? R(1) : R(-1);
-#pragma unroll
-  for (int i = 0; i < N; ++i) m[i] = sg * swap_pair(m[i]);
+  fac::mass_product<P, R>(xv, g, [&](int i, R v) { y[i] = sg * swap_pair(v); });
   __builtin_amdgcn_sched_barrier(0);  // one product's intermediates at a time
-  fac::curl_product<P, R>(xv, h, y);
-#pragma unroll
-  for (int i = 0; i < N; ++i) y[i] += m[i];
+  fac::curl_product<P, R>(xv, h, [&](int i, R v) { y[i] += v; });
   asm("" : "+v"(code));  // the coefficients again, not kept through the products
-  fac::Orient<P, R>(code).out(y);
+  fac::orient_out<P>(code, y);
 #pragma unroll
   for (int i = 0; i < N; ++i) ye[((w * N + i) * kWave + l) * 2 + part] = y[i];
-}
-
-// ---------------------------------------------------------------------------
-// local products, p = 3 in complex64: one lane per element, 64 elements of one
-// orientation combination per wave, so every table value is a wave-uniform
-// (scalar) load.  tab[combo][...]: the table components of the pairs k = (i,
-// j >= i) (row-major upper triangle; per pair c < 6 mass, c >= 6 curl-curl),
-// structural zeros left out.
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kWave) k_eop_local3(int64_t nw, const int32_t* __restrict__ done,
-                                                      const int32_t* __restrict__ wseg,
-                                                      int dstride,
-                                                      const int32_t* __restrict__ wcombo,
-                                                      const int32_t* __restrict__ edofs,
-                                                      const float* __restrict__ coef,
-                                                      const float* __restrict__ tab,
-                                                      const float2* __restrict__ x,
-                                                      float2* __restrict__ ye) {
-  using R = float;
-  using C = float2;
-  constexpr int P = 3, N = 45;
-  constexpr int NLE = n_local_entities<P>();
-  static_assert(N == loc_off<P>(NLE - 1) + loc_nd<P>(NLE - 1), "entity DOFs");
-  if (done && !wseg && *done) return;
-  // XCD-contiguous ranges of waves (workgroup b runs on XCD b % 8)
-  const int64_t nb = gridDim.x;
-  int64_t w = blockIdx.x;
-  if (nb % 8 == 0) w = (w % 8) * (nb / 8) + w / 8;
-  if (w >= nw) return;
-  // segmented operator: the wave's mesh has converged
-  if (wseg && done[(int64_t)__builtin_amdgcn_readfirstlane(wseg[w]) * dstride]) return;
-  const int lane = threadIdx.x % kWave;
-  const int combo = __builtin_amdgcn_readfirstlane(wcombo[w]);
-  constexpr int NTS = table_stride<P>();  // constant-evaluated, not a loop at run time
-  const R* __restrict__ t = tab + (int64_t)combo * NTS;
-  int fv[NLE];
-#pragma unroll
-  for (int la = 0; la < NLE; ++la) fv[la] = edofs[(w * NLE + la) * kWave + lane];
-  R cf[12];
-#pragma unroll
-  for (int c = 0; c < 12; ++c) cf[c] = coef[(w * 12 + c) * kWave + lane];
-  C xv[N];
-#pragma unroll
-  for (int la = 0; la < NLE; ++la) {
-    const int f = fv[la] >= 0 ? fv[la] : 0;
-#pragma unroll
-    for (int k = 0; k < loc_nd<P>(la); ++k) xv[loc_off<P>(la) + k] = x[f + k];
-  }
-#pragma unroll
-  for (int la = 0; la < NLE; ++la)
-    if (fv[la] < 0)
-#pragma unroll
-      for (int k = 0; k < loc_nd<P>(la); ++k) xv[loc_off<P>(la) + k] = C{0, 0};
-  C y[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) y[i] = C{0, 0};
-  // fully unrolled: the masks, the presence flags and the table offset are
-  // compile-time constants, so only the nonzero terms are emitted
-  int off = 0;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-#pragma unroll
-    for (int j = i; j < N; ++j) {
-      const unsigned zm = zero_mask<P>(i * N - (i * (i - 1)) / 2 + (j - i));
-      R im = 0, re = 0;
-      bool has_im = false, has_re = false;
-#pragma unroll
-      for (int c = 0; c < 6; ++c)
-        if (!((zm >> c) & 1)) {
-          const R tv = t[off];
-          im = has_im ? fma(cf[c], tv, im) : cf[c] * tv;
-          has_im = true;
-          ++off;
-        }
-#pragma unroll
-      for (int c = 6; c < 12; ++c)
-        if (!((zm >> c) & 1)) {
-          const R tv = t[off];
-          re = has_re ? fma(cf[c], tv, re) : cf[c] * tv;
-          has_re = true;
-          ++off;
-        }
-      if (has_re) {
-        y[i].x = fma(re, xv[j].x, y[i].x);
-        y[i].y = fma(re, xv[j].y, y[i].y);
-        if (j != i) {
-          y[j].x = fma(re, xv[i].x, y[j].x);
-          y[j].y = fma(re, xv[i].y, y[j].y);
-        }
-      }
-      if (has_im) {
-        y[i].x = fma(-im, xv[j].y, y[i].x);
-        y[i].y = fma(im, xv[j].x, y[i].y);
-        if (j != i) {
-          y[j].x = fma(-im, xv[i].y, y[j].x);
-          y[j].y = fma(im, xv[i].x, y[j].y);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < N; ++i) ye[(w * N + i) * kWave + lane] = y[i];
-}
-
-// ---------------------------------------------------------------------------
-// p = 3 complex128 element products on the FP64 matrix cores.  With 45 DOFs
-// the values of x and of the products take 360 registers per lane in
-// complex128, so the lane-per-element kernel above does not fit; here one
-// wave takes one slot group w (64 elements of one combination) and forms
-//     Y (48 x 128) = Tf (48 x K) * B (K x 128)
-// with v_mfma_f64_16x16x4f64: column n < 64 of Y is element n's real part,
-// column 64 + n its imaginary part (rows 45..47 padding); column k = (c, j)
-// of Tf is table component c of the pairs (i, j) (both triangles), and
-//     B[(c, j)][n]      = cf_n[c] re x_n[j]   (c curl-curl) or -cf_n[c] im x_n[j] (c mass)
-//     B[(c, j)][64 + n] = cf_n[c] im x_n[j]   (c curl-curl) or  cf_n[c] re x_n[j] (c mass)
-// (mass coefficients carry -omega mu0, as in k_eop_local).  Only the columns
-// (c, j) that are not zero for every orientation are kept (kcol, padded to a
-// multiple of 4 with -1).  The element's x and coefficients are staged in LDS
-// (52 KB per wave); the fragments of Tf are per combination in fragment order
-// afrag[combo][ks][m-tile][lane] (L2-resident).  Operand layout of the
-// instruction (measured): A lane l = (row l % 16, k l / 16), B lane l =
-// (k l / 16, column l % 16), D lane l, value r = (row 4 r + l / 16, column l % 16).
-// ---------------------------------------------------------------------------
-typedef double mfma_d4 __attribute__((ext_vector_type(4)));
-constexpr int kMfmaXStride = 46;  // complex values per element row in LDS (45 + 1 pad)
-
-__global__ void __launch_bounds__(kWave) k_eop_mfma3(int64_t nw, const int32_t* __restrict__ done,
-                                                     const int32_t* __restrict__ wseg, int dstride,
-                                                     const int32_t* __restrict__ wcombo,
-                                                     const int32_t* __restrict__ edofs,
-                                                     const double* __restrict__ coef,
-                                                     const double* __restrict__ afrag,
-                                                     const int32_t* __restrict__ kcol, int nks,
-                                                     const double2* __restrict__ x,
-                                                     double2* __restrict__ ye) {
-  constexpr int P = 3, N = 45, NLE = n_local_entities<P>();
-  __shared__ double2 xs[kWave * kMfmaXStride];
-  __shared__ double cfs[kWave * 12];
-  if (done && !wseg && *done) return;
-  const int64_t nb = gridDim.x;
-  int64_t w = blockIdx.x;
-  if (nb % 8 == 0) w = (w % 8) * (nb / 8) + w / 8;  // XCD-contiguous ranges of slot groups
-  if (w >= nw) return;
-  if (wseg && done[(int64_t)wseg[w] * dstride]) return;  // segmented: the mesh has converged
-  const int lane = threadIdx.x;
-  const int combo = __builtin_amdgcn_readfirstlane(wcombo[w]);
-  // stage this lane's element: coefficients and x (zero for PEC / empty)
-#pragma unroll
-  for (int c = 0; c < 12; ++c) cfs[lane * 12 + c] = coef[(w * 12 + c) * kWave + lane];
-#pragma unroll
-  for (int la = 0; la < NLE; ++la) {
-    const int f = edofs[(w * NLE + la) * kWave + lane];
-#pragma unroll
-    for (int k = 0; k < loc_nd<P>(la); ++k)
-      xs[lane * kMfmaXStride + loc_off<P>(la) + k] = f >= 0 ? x[f + k] : double2{0.0, 0.0};
-  }
-  __syncthreads();
-  mfma_d4 acc[3][8];
-#pragma unroll
-  for (int mt = 0; mt < 3; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) acc[mt][nt] = mfma_d4{0.0, 0.0, 0.0, 0.0};
-  const double* __restrict__ af = afrag + (int64_t)combo * nks * 3 * kWave;
-  const int kr = lane / 16, en = lane % 16;
-  // the fragments of Tf and the column of step ks + 1 are loaded during step ks
-  double na0 = af[lane], na1 = af[kWave + lane], na2 = af[2 * kWave + lane];
-  int nkc = kcol[kr];
-  for (int ks = 0; ks < nks; ++ks) {
-    const double a0 = na0, a1 = na1, a2 = na2;
-    const int kc = nkc;
-    if (ks + 1 < nks) {
-      na0 = af[((ks + 1) * 3 + 0) * kWave + lane];
-      na1 = af[((ks + 1) * 3 + 1) * kWave + lane];
-      na2 = af[((ks + 1) * 3 + 2) * kWave + lane];
-      nkc = kcol[(ks + 1) * 4 + kr];
-    }
-    double bre[4], bim[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) bre[q] = bim[q] = 0.0;
-    if (kc >= 0) {
-      const int c = kc >> 8, j = kc & 255;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int e = q * 16 + en;
-        const double2 xv = xs[e * kMfmaXStride + j];
-        const double cv = cfs[e * 12 + c];
-        if (c >= 6) {
-          bre[q] = cv * xv.x;
-          bim[q] = cv * xv.y;
-        } else {
-          bre[q] = -(cv * xv.y);
-          bim[q] = cv * xv.x;
-        }
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      acc[0][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, bre[q], acc[0][q], 0, 0, 0);
-      acc[1][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, bre[q], acc[1][q], 0, 0, 0);
-      acc[2][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a2, bre[q], acc[2][q], 0, 0, 0);
-      acc[0][q + 4] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, bim[q], acc[0][q + 4], 0, 0, 0);
-      acc[1][q + 4] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, bim[q], acc[1][q + 4], 0, 0, 0);
-      acc[2][q + 4] = __builtin_amdgcn_mfma_f64_16x16x4f64(a2, bim[q], acc[2][q + 4], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int mt = 0; mt < 3; ++mt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = mt * 16 + 4 * r + kr;
-      if (i < N)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          ye[((int64_t)w * N + i) * kWave + q * 16 + en] = double2{acc[mt][q][r], acc[mt][q + 4][r]};
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -580,21 +334,17 @@ __global__ void __launch_bounds__(512, 3) k_meop_local(
       g[c] = coefm[(w * 12 + c) * kWave + l];
       h[c] = coefm[(w * 12 + 6 + c) * kWave + l];
     }
-    double xv[N], y[N], m[N];
+    double xv[N], y[N];
 #pragma unroll
     for (int la = 0; la < NLE; ++la)
 #pragma unroll
       for (int k = 0; k < loc_nd<P>(la); ++k)
         xv[loc_off<P>(la) + k] = f[la] >= 0 ? (double)x[(f[la] + k) * ld + t] : 0.0;
     int code = ocode[w * kWave + l];
-    fac::Orient<P, double>(code).in(xv);
-    fac::mass_product<P, double>(xv, g, m);
-#pragma unroll
-    for (int i = 0; i < N; ++i) m[i] = om * swap_pair(m[i]);
-    __builtin_amdgcn_sched_barrier(0);  // one part's intermediates at a time
-    fac::curl_product<P, double>(xv, h, y);
-#pragma unroll
-    for (int i = 0; i < N; ++i) y[i] += m[i];
+    fac::orient_in<P>(code, xv);
+    fac::mass_product<P, double>(xv, g, [&](int i, double v) { y[i] = om * swap_pair(v); });
+    __builtin_amdgcn_sched_barrier(0);  // one product's intermediates at a time
+    fac::curl_product<P, double>(xv, h, [&](int i, double v) { y[i] += v; });
     // x^T y is the same in the code-0 functions
 #pragma unroll
     for (int i = 0; i < N; ++i) {
@@ -602,7 +352,7 @@ __global__ void __launch_bounds__(512, 3) k_meop_local(
       dim += xv[i] * swap_pair(y[i]);
     }
     asm("" : "+s"(code));  // the coefficients again, not kept through the products
-    fac::Orient<P, double>(code).out(y);
+    fac::orient_out<P>(code, y);
 #pragma unroll
     for (int i = 0; i < N; ++i) ye[((w * N + i) * kWave + l) * ld + t] = (R)y[i];
   }
@@ -639,16 +389,13 @@ __global__ void k_eop_coef(int64_t nslot, const int32_t* __restrict__ perm,
 struct ElemOp {
   int p = 0, N = 0, D = 1;
   int64_t E = 0, ndof = 0, nent = 0, nw = 0;
-  int ncombo = 0, grid = 1;
-  int32_t* wcombo = nullptr;
+  int grid = 1;
   int32_t* edofs = nullptr;
   int32_t* perm = nullptr;
   int4* gm = nullptr;
   int32_t* gslot = nullptr;
   double* coef64 = nullptr;
   float* coef32 = nullptr;
-  double* tab64 = nullptr;
-  float* tab32 = nullptr;
   double2* ye64 = nullptr;
   float2* ye32 = nullptr;
   // packed element orientation per slot (orient_of)
@@ -656,11 +403,6 @@ struct ElemOp {
   // multi-right-hand-side products (eop_multi_prepare): raw coefficients in
   // slot order (mass part without -omega mu0)
   double* coefm = nullptr;
-  // p = 3 complex128 products on the matrix cores (k_eop_mfma3): Tf fragments
-  // per combination and the kept (c, j) columns
-  double* afrag = nullptr;
-  int32_t* kcol = nullptr;
-  int nks = 0;
   // multi-mesh operator (pg_eop_create_multi): segment of every wave, omega mu0
   // of every segment, first schedule position of every segment (nseg + 1)
   int nseg = 0;
@@ -685,61 +427,42 @@ struct ElemOp {
 };
 
 int eop_grid(const ElemOp* op) { return op->grid; }
-bool eop_supports(const ElemOp* op, bool complex128) {
-  return !(complex128 && op->p == 3 && !op->afrag);
-}
 int64_t eop_ndof(const ElemOp* op) { return op->ndof; }
 
 // element products of slot groups [w0, w0 + nwr) (all groups: 0, op->nw)
 template <typename R>
 static void launch_local(const ElemOp* op, const int32_t* done, const int32_t* wseg, int dstride,
                          const typename eop::Cx<R>::T* x, typename eop::Cx<R>::T* ye,
-                         const R* coef, const R* tab, hipStream_t st, int64_t w0 = 0,
-                         int64_t nwr = -1) {
+                         const R* coef, hipStream_t st, int64_t w0 = 0, int64_t nwr = -1) {
   if (nwr < 0) nwr = op->nw;
   if (nwr <= 0) return;
   const int nle = op->p == 1 ? 6 : (op->p == 2 ? 10 : 11);
-  const int32_t* ed = op->edofs + w0 * nle * kWave;
-  const int32_t* ws = wseg ? wseg + w0 : nullptr;
-  coef += w0 * 12 * kWave;
-  ye += w0 * op->N * kWave;
-  if (op->p <= 2) {
-    const int gpb = eop::kBS / (2 * kWave);  // slot groups per workgroup, two waves each
-    int64_t nbl = (nwr + gpb - 1) / gpb;
-    if (nbl >= 64) nbl = (nbl + 7) / 8 * 8;
-    const dim3 g((unsigned)nbl), b(eop::kBS);
-    const int32_t* oc = op->ocode + w0 * kWave;
-    const R* xr = reinterpret_cast<const R*>(x);
-    R* yr = reinterpret_cast<R*>(ye);
-    if (op->p == 1)
-      hipLaunchKernelGGL((eop::k_eop_fac<1, R>), g, b, 0, st, nwr, done, ws, dstride, ed, oc,
-                         coef, xr, yr);
-    else
-      hipLaunchKernelGGL((eop::k_eop_fac<2, R>), g, b, 0, st, nwr, done, ws, dstride, ed, oc,
-                         coef, xr, yr);
-    return;
-  }
-  // p = 3: one wave per slot group.  complex64: one lane per element; complex128:
-  // the matrix-core kernel (the values of x and of the products do not fit one lane)
-  int64_t nbl = nwr;
+  const int gpb = eop::kBS / (2 * kWave);  // slot groups per workgroup, two waves each
+  int64_t nbl = (nwr + gpb - 1) / gpb;
   if (nbl >= 64) nbl = (nbl + 7) / 8 * 8;
-  const dim3 g((unsigned)nbl), b(kWave);
-  const int32_t* wc = op->wcombo + w0;
-  if constexpr (sizeof(R) == 4)
-    hipLaunchKernelGGL(eop::k_eop_local3, g, b, 0, st, nwr, done, ws, dstride, wc, ed, coef, tab,
-                       x, ye);
-  else
-    hipLaunchKernelGGL(eop::k_eop_mfma3, g, b, 0, st, nwr, done, ws, dstride, wc, ed, coef,
-                       op->afrag, op->kcol, op->nks, x, ye);
+  const dim3 g((unsigned)nbl), b(eop::kBS);
+  const int32_t* ed = op->edofs + w0 * nle * kWave;
+  const int32_t* oc = op->ocode + w0 * kWave;
+  const int32_t* ws = wseg ? wseg + w0 : nullptr;
+  const R* xr = reinterpret_cast<const R*>(x);
+  R* yr = reinterpret_cast<R*>(ye + w0 * op->N * kWave);
+  coef += w0 * 12 * kWave;
+#define PG_FAC(P)                                                                               \
+  hipLaunchKernelGGL((eop::k_eop_fac<P, R>), g, b, 0, st, nwr, done, ws, dstride, ed, oc, coef, \
+                     xr, yr)
+  if (op->p == 1) PG_FAC(1);
+  else if (op->p == 2) PG_FAC(2);
+  else PG_FAC(3);
+#undef PG_FAC
 }
 
 template <typename R>
 static void launch_impl(const ElemOp* op, int mode, const int32_t* done,
                         const typename eop::Cx<R>::T* x, typename eop::Cx<R>::T* y,
                         const double2* b, double* part, hipStream_t st, hipEvent_t mid,
-                        typename eop::Cx<R>::T* ye, const R* coef, const R* tab) {
+                        typename eop::Cx<R>::T* ye, const R* coef) {
   using C = typename eop::Cx<R>::T;
-  launch_local<R>(op, done, nullptr, 0, x, ye, coef, tab, st);
+  launch_local<R>(op, done, nullptr, 0, x, ye, coef, st);
   // a failed record only loses this timing sample (the elapsed-time query fails)
   if (mid) (void)hipEventRecord(mid, st);
   const dim3 g(op->grid), bl(eop::kBS);
@@ -764,11 +487,11 @@ static void launch_impl(const ElemOp* op, int mode, const int32_t* done,
 
 void eop_launch(const ElemOp* op, int mode, const int32_t* done, const double2* x, double2* y,
                 const double2* b, double* part, hipStream_t st, hipEvent_t mid) {
-  launch_impl<double>(op, mode, done, x, y, b, part, st, mid, op->ye64, op->coef64, op->tab64);
+  launch_impl<double>(op, mode, done, x, y, b, part, st, mid, op->ye64, op->coef64);
 }
 void eop_launch(const ElemOp* op, int mode, const int32_t* done, const float2* x, float2* y,
                 const double2* b, double* part, hipStream_t st, hipEvent_t mid) {
-  launch_impl<float>(op, mode, done, x, y, b, part, st, mid, op->ye32, op->coef32, op->tab32);
+  launch_impl<float>(op, mode, done, x, y, b, part, st, mid, op->ye32, op->coef32);
 }
 
 static int eop_refresh(ElemOp* op, const void* ws, double omega, hipStream_t st) {
@@ -817,14 +540,14 @@ int eop_segments(const ElemOp* op, const int64_t** seg_pos, const int64_t** seg_
 const double2* eop_local_segments(const ElemOp* op, const int32_t* done, int dstride,
                                   const double2* x, hipStream_t st, int64_t w0, int64_t w1) {
   if (w1 < 0) w1 = op->nw;
-  launch_local<double>(op, done, op->wseg, dstride, x, op->ye64, op->coef64, op->tab64, st, w0,
+  launch_local<double>(op, done, op->wseg, dstride, x, op->ye64, op->coef64, st, w0,
                        w1 - w0);
   return op->ye64;
 }
 const float2* eop_local_segments(const ElemOp* op, const int32_t* done, int dstride,
                                  const float2* x, hipStream_t st, int64_t w0, int64_t w1) {
   if (w1 < 0) w1 = op->nw;
-  launch_local<float>(op, done, op->wseg, dstride, x, op->ye32, op->coef32, op->tab32, st, w0,
+  launch_local<float>(op, done, op->wseg, dstride, x, op->ye32, op->coef32, st, w0,
                       w1 - w0);
   return op->ye32;
 }
@@ -930,23 +653,9 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   } else {
     std::iota(pos.begin(), pos.end(), 0);
   }
-  // orientation combinations (p = 3, whose waves hold one combination each; at
-  // p <= 2 the products take any orientation per lane)
-  std::map<int, int> cid;
-  std::vector<int> combos;
-  std::vector<int32_t> ec(E, 0);
-  for (int64_t e = 0; p == 3 && e < E; ++e) {
-    auto it = cid.find(hor[e]);
-    if (it == cid.end()) {
-      it = cid.emplace(hor[e], (int)combos.size()).first;
-      combos.push_back(hor[e]);
-    }
-    ec[e] = it->second;
-  }
-  // element order: by segment (multi-mesh operator), by combination (p = 3), then
-  // by the earliest schedule position of the element's entities (spatial order
-  // when the schedule is)
-  std::vector<int64_t> key(E);
+  // element order: by segment (multi-mesh operator), then by the earliest schedule
+  // position of the element's entities (spatial order when the schedule is)
+  std::vector<int32_t> key(E);
   std::vector<int32_t> es(E, 0);
   for (int64_t e = 0; e < E; ++e) {
     int32_t m = pos[eg[e * nle]], mx = m;
@@ -954,7 +663,7 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
       m = std::min(m, pos[eg[e * nle + la]]);
       mx = std::max(mx, pos[eg[e * nle + la]]);
     }
-    key[e] = ((int64_t)ec[e] << 32) | (uint32_t)m;
+    key[e] = m;
     if (seg) {
       const auto& sp = seg->pos;
       const int sm = (int)(std::upper_bound(sp.begin(), sp.end(), (int64_t)m) - sp.begin()) - 1;
@@ -968,20 +677,19 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   std::stable_sort(sorted.begin(), sorted.end(), [&](int64_t a, int64_t b) {
     return es[a] != es[b] ? es[a] < es[b] : key[a] < key[b];
   });
-  // slot groups of 64 elements of one segment (p = 3: and one combination)
-  std::vector<int32_t> wcombo, perm, wsg;
+  // slot groups of 64 elements of one segment
+  std::vector<int32_t> perm, wsg;
   for (int64_t k = 0; k < E;) {
-    const int c = ec[sorted[k]], sg = es[sorted[k]];
+    const int sg = es[sorted[k]];
     int64_t k1 = k;
-    while (k1 < E && ec[sorted[k1]] == c && es[sorted[k1]] == sg) ++k1;
+    while (k1 < E && es[sorted[k1]] == sg) ++k1;
     for (int64_t a = k; a < k1; a += kWave) {
-      wcombo.push_back(c);
       wsg.push_back(sg);
       for (int l = 0; l < kWave; ++l) perm.push_back(a + l < k1 ? (int32_t)sorted[a + l] : -1);
     }
     k = k1;
   }
-  const int64_t nw = (int64_t)wcombo.size(), nslot = nw * kWave;
+  const int64_t nw = (int64_t)wsg.size(), nslot = nw * kWave;
   if (nslot * N >= (1LL << 31)) PG_FAIL(PG_ERR_UNSUPPORTED, "too many elements");
   std::vector<int32_t> hoc(nslot, 0);  // orientation per slot
   for (int64_t s = 0; s < nslot; ++s)
@@ -1023,83 +731,7 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     const int64_t g = order ? order[i] : i;
     gm[i] = make_int4(bp[g], bp[g + 1] - bp[g], (int)start[i], (int)start[i + 1]);
   }
-  // p = 3: per-combination tables of the upper triangle without the structural
-  // zeros (which must vanish here too: a stale mask would drop real terms)
-  const int nc = (int)combos.size();
-  const int NT = eop::n_table_entries<3>(), NTS = eop::table_stride<3>();
   int rc = PG_OK;
-  std::vector<double> tab((size_t)nc * NTS, 0.0);
-  if (p == 3) {
-    const int V = n_variants(p);
-    std::vector<double> T((size_t)V * V * 12);
-    if ((rc = pg_tables_host(p, T.data(), (int64_t)T.size())) != PG_OK) return rc;
-    double tmax = 0.0;
-    for (double v : T) tmax = std::max(tmax, std::fabs(v));
-    std::vector<int> var(N);
-    for (int c = 0; c < nc; ++c) {
-      for (int la = 0; la < nle; ++la)
-        for (int k = 0; k < entity_ndof(la, p); ++k)
-          var[entity_local_offset(la, p) + k] =
-              entity_variant_base(la, orient_of(combos[c], la), p) + k;
-      int k = 0;
-      size_t o = (size_t)c * NTS;
-      for (int i = 0; i < N; ++i)
-        for (int j = i; j < N; ++j, ++k) {
-          const unsigned zm = eop::zero_mask<3>(k);
-          for (int q = 0; q < 12; ++q) {
-            const double v = T[((size_t)var[i] * V + var[j]) * 12 + q];
-            if ((zm >> q) & 1) {
-              if (std::fabs(v) > 1e-15 * tmax)
-                PG_FAIL(PG_ERR_UNSUPPORTED, "element table entry (%d, %d, %d) is not zero", i, j,
-                        q);
-            } else {
-              tab[o++] = v;
-            }
-          }
-        }
-      if (o != (size_t)c * NTS + NT) PG_FAIL(PG_ERR_UNSUPPORTED, "element table size mismatch");
-    }
-  }
-  std::vector<float> tab32(tab.begin(), tab.end());
-  // p = 3: matrix-core fragments.  kcol = the (c, j) columns of Tf that are not
-  // zero for every orientation (c << 8 | j), padded to a multiple of 4 with -1;
-  // afrag[combo][ks][mt][lane] = Tf[mt * 16 + lane % 16][kcol[4 ks + lane / 16]]
-  std::vector<int32_t> kcol;
-  std::vector<double> afrag;
-  int nks = 0;
-  if (p == 3) {
-    const int NPp = N * (N + 1) / 2;
-    std::vector<int> poff(NPp + 1, 0);
-    for (int k = 0; k < NPp; ++k) poff[k + 1] = poff[k] + 12 - eop::popcount12(eop::zero_mask<3>(k));
-    auto pair_of = [&](int i, int j) {
-      const int a = std::min(i, j), b2 = std::max(i, j);
-      return a * N - (a * (a - 1)) / 2 + (b2 - a);
-    };
-    for (int c = 0; c < 12; ++c)
-      for (int j = 0; j < N; ++j) {
-        bool any = false;
-        for (int i = 0; i < N && !any; ++i) any = !((eop::zero_mask<3>(pair_of(i, j)) >> c) & 1);
-        if (any) kcol.push_back((c << 8) | j);
-      }
-    while (kcol.size() % 4) kcol.push_back(-1);
-    nks = (int)kcol.size() / 4;
-    afrag.assign((size_t)nc * nks * 3 * kWave, 0.0);
-    for (int cb = 0; cb < nc; ++cb)
-      for (int ks = 0; ks < nks; ++ks)
-        for (int mt = 0; mt < 3; ++mt)
-          for (int l = 0; l < kWave; ++l) {
-            const int i = mt * 16 + l % 16, kc = kcol[ks * 4 + l / 16];
-            if (i >= N || kc < 0) continue;
-            const int c = kc >> 8, j = kc & 255, k = pair_of(i, j);
-            const unsigned zm = eop::zero_mask<3>(k);
-            if ((zm >> c) & 1) continue;
-            int rank = 0;  // position of component c among the pair's kept components
-            for (int q = 0; q < c; ++q) rank += !((zm >> q) & 1);
-            afrag[(((size_t)cb * nks + ks) * 3 + mt) * kWave + l] =
-                tab[(size_t)cb * NTS + poff[k] + rank];
-          }
-  }
-
   ElemOp* op = new ElemOp();
   op->p = p;
   op->N = N;
@@ -1108,7 +740,6 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   op->ndof = ndof;
   op->nent = nblocks;
   op->nw = nw;
-  op->ncombo = nc;
   {
     int64_t g = (nblocks + eop::kBS - 1) / eop::kBS;
     g = std::min<int64_t>(g, eop::kMaxGrid);
@@ -1120,7 +751,6 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     delete op;                                    \
     return rc;                                    \
   }
-  PG_A(op->wcombo, nw);
   PG_A(op->edofs, hed.size());
   PG_A(op->perm, nslot);
   PG_A(op->ocode, nslot);
@@ -1128,15 +758,8 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   PG_A(op->gslot, gslot.size());
   PG_A(op->coef64, nslot * 12);
   PG_A(op->coef32, nslot * 12);
-  PG_A(op->tab64, tab.size());
-  PG_A(op->tab32, tab.size());
   PG_A(op->ye64, nslot * N);
   PG_A(op->ye32, nslot * N);
-  if (p == 3) {
-    PG_A(op->afrag, afrag.size());
-    PG_A(op->kcol, kcol.size());
-    op->nks = nks;
-  }
   std::vector<double> womu;
   if (seg) {
     op->nseg = seg->nseg;
@@ -1154,16 +777,11 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     void* dst;
     const void* src;
     size_t bytes;
-  } up[] = {{op->wcombo, wcombo.data(), wcombo.size() * sizeof(int32_t)},
-            {op->edofs, hed.data(), hed.size() * sizeof(int32_t)},
+  } up[] = {{op->edofs, hed.data(), hed.size() * sizeof(int32_t)},
             {op->perm, perm.data(), perm.size() * sizeof(int32_t)},
             {op->ocode, hoc.data(), hoc.size() * sizeof(int32_t)},
             {op->gm, gm.data(), gm.size() * sizeof(int4)},
             {op->gslot, gslot.data(), gslot.size() * sizeof(int32_t)},
-            {op->tab64, tab.data(), tab.size() * sizeof(double)},
-            {op->tab32, tab32.data(), tab32.size() * sizeof(float)},
-            {op->afrag, afrag.data(), afrag.size() * sizeof(double)},
-            {op->kcol, kcol.data(), kcol.size() * sizeof(int32_t)},
             {op->wseg, wsg.data(), op->wseg ? wsg.size() * sizeof(int32_t) : 0},
             {op->womu, womu.data(), womu.size() * sizeof(double)}};
   for (const auto& u : up)
@@ -1308,8 +926,6 @@ int pg_eop_refresh(void* op, const void* ws, double omega, void* stream) {
 
 int pg_eop_apply_z(const void* op, const double* x, double* y, void* stream) {
   if (!op || !x || !y) PG_FAIL(PG_ERR_ARG, "bad arguments");
-  if (!eop_supports(static_cast<const ElemOp*>(op), true))
-    PG_FAIL(PG_ERR_UNSUPPORTED, "element-by-element operator without a complex128 product");
   eop_launch(static_cast<const ElemOp*>(op), 0, nullptr, reinterpret_cast<const double2*>(x),
              reinterpret_cast<double2*>(y), nullptr, nullptr, as_stream(stream));
   PG_CHECK_LAUNCH();

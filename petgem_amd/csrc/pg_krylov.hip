@@ -1649,10 +1649,8 @@ static int autotune(Solver* S, hipStream_t st) {
     const Solver* L = static_cast<const Solver*>(S->o.like);
     if (L->n != S->n || L->nnz != S->nnz || L->er_ok != S->er_ok || L->pairs_ok != S->pairs_ok)
       PG_FAIL(PG_ERR_ARG, "`like` is a solver of another system or layout");
-    const auto usable = [&](const SpmvCfg& c, bool c128) {
-      return c.kind != 3 || (S->eop && eop_supports(S->eop, c128));
-    };
-    if (!usable(L->c64, true) || (mixed && !usable(L->c32, false)))
+    const auto usable = [&](const SpmvCfg& c) { return c.kind != 3 || S->eop; };
+    if (!usable(L->c64) || (mixed && !usable(L->c32)))
       PG_FAIL(PG_ERR_ARG, "`like` uses an element operator this solver does not have");
     if (mixed && L->o.precision != PG_PREC_MIXED)
       PG_FAIL(PG_ERR_ARG, "`like` has no complex64 configuration");
@@ -1703,14 +1701,9 @@ static int autotune(Solver* S, hipStream_t st) {
   ce.G = ce.U = 0;
   if (S->eop) ce.grid = eop_grid(S->eop);
   S->c64 = S->cres;
-  // (an operator without a complex128 product, p = 3, serves complex64 only;
-  // the FP64 recursion then keeps the CSR kernel)
-  const bool eop64 = S->eop && eop_supports(S->eop, true);
-  if (only_eop && !eop64 && !mixed)
-    PG_FAIL(PG_ERR_UNSUPPORTED, "the element operator at p = 3 has no complex128 product");
-  if (only_eop && eop64) {
+  if (only_eop) {
     S->c64 = ce;
-  } else if (eop64 && S->o.spmv == PG_SPMV_AUTO) {
+  } else if (S->eop && S->o.spmv == PG_SPMV_AUTO) {
     const float t_csr = time_spmv<double2, double2>(S, S->cres, st, S->vals, S->r64, S->q, 20);
     const float t_eop = time_spmv<double2, double2>(S, ce, st, S->vals, S->r64, S->q, 20);
     if (t_eop < t_csr) S->c64 = ce;

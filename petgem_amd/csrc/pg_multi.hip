@@ -1235,8 +1235,6 @@ int pg_multi_set_element_operator(void* batch, void* op, void* stream) {
   if (nseg != B->nseg)
     PG_FAIL(PG_ERR_ARG, "element operator of %d meshes for a batch of %d", nseg, B->nseg);
   if (eop_ndof(E) != B->n) PG_FAIL(PG_ERR_ARG, "element operator and batch differ in size");
-  if (!eop_supports(E, true))
-    PG_FAIL(PG_ERR_UNSUPPORTED, "element operator without a complex128 product");
   const EopSchedule es = eop_schedule(E);
   const int64_t nent = es.nent;
   hipStream_t cst = as_stream(stream);

@@ -1,14 +1,15 @@
 """Generate ``csrc/pg_eop_mask.h``: the structural zeros of the element tables.
 
-For order p, the element products use, per pair (i, j >= i) of local DOFs, the
-12 table components T_c[v_i][v_j] (6 mass, 6 curl-curl) of the two DOFs'
+For order p, an element entry of the pair (i, j >= i) of local DOFs is a sum of
+the 12 table components T_c[v_i][v_j] (6 mass, 6 curl-curl) of the two DOFs'
 orientation variants.  Some components vanish for every orientation of the
 element (the quadrature sums cancel exactly; the computed values are rounding
 noise below 1e-16 of the largest entry).  This script evaluates the tables of
 the built library (``pg_tables_host``) over all 2^6 * 6^4 orientation
 combinations and writes, per pair, a 12-bit mask of the components that are
-zero in every one of them; the element-product kernel skips those terms at
-compile time, and ``pg_eop_create`` checks them against the tables it builds.
+zero in every one of them: the terms that an entry formed from the tables can
+leave out.  (The element products form no entries, csrc/pg_factor.h; the masks
+pin the tables' structure in the tests.)
 
 Usage (after ``python -m petgem_amd.build``)::
 
