@@ -186,8 +186,8 @@ int pg_adjoint_rhs(int p, int64_t n_points, const double *points, const int32_t 
                    const double *coords, const int32_t *elems_nodes, const int32_t *elems_edges,
                    const int32_t *edges_nodes, const int32_t *faces_edges, const int32_t *dofs,
                    const double *coef, double *f, void *stream);
-/* g[e] += sum_r -omega_r*mu0 * Im(lam_e^T M_e(sigma) x_e), with M_e
- * recomputed from the tables and a filled geometry workspace; x, lam are
+/* g[e] += sum_r -omega_r*mu0 * Im(lam_e^T M_e(sigma) x_e), with M_e x_e
+ * formed from a filled geometry workspace; x, lam are
  * (nrhs, ndof) complex128, omega (nrhs) host array. */
 int pg_adjoint_gradient(const void *tables, int64_t n_elems, const void *workspace,
                         const int32_t *dofs, int nrhs, int64_t ndof, const double *x,
@@ -196,15 +196,13 @@ int pg_adjoint_gradient(const void *tables, int64_t n_elems, const void *workspa
 int pg_adjoint_gradient_rows(const void *tables, int64_t n_elems, const void *workspace,
                              const int32_t *dofs, int nrhs, int64_t ndof, const double *x,
                              const double *lam, const double *omega, double *g, void *stream);
-/* pg_adjoint_gradient without any allocation.  No counterpart in the
- * reference: for callers that cannot allocate device memory (code under HIP
- * graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
- * per-right-hand-side omega*mu0 values are staged in a fixed 32 KB device
- * array (one per GPU, kept until the process ends) instead of a stream-ordered
- * allocation, so nrhs is at most 4096 (larger: PG_ERR_ARG).  Same arguments,
- * kernel and results as pg_adjoint_gradient; the call returns once the stream
- * has drained.  Every call on a GPU shares that GPU's staging array: calls that
- * overlap on one GPU (from several host threads) race. */
+/* pg_adjoint_gradient for callers that need the guarantee that nothing is
+ * allocated (tight serving loops, harnesses that forbid hipMalloc).  No
+ * counterpart in the reference.  Same arguments, kernel and results as
+ * pg_adjoint_gradient, which allocates nothing either: the per-right-hand-side
+ * omega*mu0 values travel with the launches, 32 at a time.  nrhs is at most 4096
+ * (larger: PG_ERR_ARG), as for pg_adjoint_gradient; the call returns once the
+ * stream has drained. */
 int pg_adjoint_gradient_noalloc(const void *tables, int64_t n_elems, const void *workspace,
                                 const int32_t *dofs, int nrhs, int64_t ndof, const double *x,
                                 const double *lam, const double *omega, double *g,

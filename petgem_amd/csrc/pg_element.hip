@@ -16,9 +16,9 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <mutex>
 #include <vector>
 
+#include "pg_adjoint.h"
 #include "pg_basis.h"
 #include "pg_common.h"
 #include "pg_rowasm.h"
@@ -821,98 +821,9 @@ __global__ void k_adjoint_rhs(int64_t npts, const double* __restrict__ pts,
   }
 }
 
-// g[e] += sum_r -omega_r*mu0 * Im(lam_e^T M_e x_e), M_e recomputed from the tables.
-// One thread per element.  Column r of x and lam holds DOF d at d*sd + r*sr
-// ((nrhs, N) layout: sd = 1, sr = N; (N, nrhs) layout: sd = nrhs, sr = 1).  Each
-// M_ij is contracted once per chunk of RC columns.
-template <int P>
-__global__ void __launch_bounds__(256) k_adjoint_grad(
-    int64_t E, const double* __restrict__ T, const double* __restrict__ coef,
-    const int32_t* __restrict__ orient, const int32_t* __restrict__ dofs, int nrhs, int64_t sd,
-    int64_t sr, const double2* __restrict__ x, const double2* __restrict__ lam,
-    const double* __restrict__ omega_mu, double* __restrict__ g) {
-  constexpr int n = P * (P + 2) * (P + 3) / 2;
-  constexpr int V = 12 * P + 24 * P * (P - 1) + P * (P - 1) * (P - 2) / 2;
-  constexpr int RC = 8;
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= E) return;
-  const int pk = orient[e];
-  const double* cf = coef + 12 * e;
-  const int32_t* de = dofs + e * n;
-  double acc_g = 0.0;
-  for (int r0 = 0; r0 < nrhs; r0 += RC) {
-    const int nr = nrhs - r0 < RC ? nrhs - r0 : RC;
-    double sim[RC];
-#pragma unroll
-    for (int t = 0; t < RC; ++t) sim[t] = 0.0;
-    for (int i = 0; i < n; ++i) {
-      int la, ka;
-      dof_entity<P>(i, la, ka);
-      const int va = entity_variant_base(la, orient_of(pk, la), P) + ka;
-      double are[RC], aim[RC];
-#pragma unroll
-      for (int t = 0; t < RC; ++t) are[t] = aim[t] = 0.0;
-      for (int j = 0; j < n; ++j) {
-        int lb, kb;
-        dof_entity<P>(j, lb, kb);
-        const int vb = entity_variant_base(lb, orient_of(pk, lb), P) + kb;
-        double m, kk;
-        contract(T + ((size_t)va * V + vb) * 12, cf, &m, &kk);
-        const double2* xj = x + (int64_t)de[j] * sd + (int64_t)r0 * sr;
-#pragma unroll
-        for (int t = 0; t < RC; ++t)
-          if (t < nr) {
-            const double2 v = xj[t * sr];
-            are[t] += m * v.x;
-            aim[t] += m * v.y;
-          }
-      }
-      const double2* li = lam + (int64_t)de[i] * sd + (int64_t)r0 * sr;
-#pragma unroll
-      for (int t = 0; t < RC; ++t)
-        if (t < nr) {
-          const double2 l = li[t * sr];
-          sim[t] += l.x * aim[t] + l.y * are[t];
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < RC; ++t)
-      if (t < nr) acc_g += -omega_mu[r0 + t] * sim[t];
-  }
-  g[e] += acc_g;
-}
-
 static inline unsigned nblocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-// ---------------------------------------------------------------------------
-// Staging of the adjoint gradient's per-right-hand-side omega*mu0 for the
-// entry point that allocates nothing (pg_adjoint_gradient_noalloc).  Every
-// device holds its own copy of `scratch`, at its own address; in host code the
-// name is only a stand-in, so the address is resolved once per device with
-// hipGetSymbolAddress (that device current) and only that address is used.
-// Each call overwrites the first nrhs entries before its kernel reads them;
-// calls that overlap on one device (several host threads) race on it.
-// ---------------------------------------------------------------------------
 constexpr int kAdjointMaxRhs = 4096;
-static __device__ __align__(256) double scratch[kAdjointMaxRhs];
-
-static std::mutex g_scratch_mu;
-static std::vector<double*> g_scratch_ptr;  // by device ordinal; nullptr = not resolved yet
-
-static int scratch_address(double** out) {
-  int dev = 0;
-  PG_HIP(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  if ((int)g_scratch_ptr.size() <= dev) g_scratch_ptr.resize(dev + 1, nullptr);
-  if (!g_scratch_ptr[dev]) {
-    void* p = nullptr;
-    PG_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-    if (!p) PG_FAIL(PG_ERR_HIP, "hipGetSymbolAddress returned a null staging address");
-    g_scratch_ptr[dev] = static_cast<double*>(p);
-  }
-  *out = g_scratch_ptr[dev];
-  return PG_OK;
-}
 
 }  // namespace pg
 
@@ -1185,12 +1096,9 @@ int pg_adjoint_rhs(int p, int64_t npts, const double* pts, const int32_t* elem,
   return PG_OK;
 }
 
-// static_staging: stage omega*mu0 in the file-scope device array instead of a
-// stream-ordered allocation (pg_adjoint_gradient_noalloc)
 static int adjoint_gradient(const void* tables, int64_t E, const void* ws, const int32_t* dofs,
                             int nrhs, int64_t ndof, int64_t sd, int64_t sr, const double* x,
-                            const double* lam, const double* omega, double* g, void* stream,
-                            bool static_staging = false) {
+                            const double* lam, const double* omega, double* g, void* stream) {
   if (!tables || !ws || !dofs || nrhs <= 0 || ndof <= 0 || !x || !lam || !omega || !g || E <= 0)
     PG_FAIL(PG_ERR_ARG, "bad arguments");
   if (nrhs > kAdjointMaxRhs)
@@ -1198,28 +1106,13 @@ static int adjoint_gradient(const void* tables, int64_t E, const void* ws, const
   const Tables* t = static_cast<const Tables*>(tables);
   double om[kAdjointMaxRhs];
   for (int r = 0; r < nrhs; ++r) om[r] = omega[r] * kMu0;
-  double* d_om = nullptr;
   hipStream_t s = as_stream(stream);
-  if (static_staging) {
-    const int rc = scratch_address(&d_om);
-    if (rc != PG_OK) return rc;
-  } else {
-    PG_HIP(hipMallocAsync(reinterpret_cast<void**>(&d_om), nrhs * sizeof(double), s));
-  }
-  PG_HIP(hipMemcpyAsync(d_om, om, nrhs * sizeof(double), hipMemcpyHostToDevice, s));
   void* w = const_cast<void*>(ws);
-  const dim3 gr(nblocks(E, 256)), bl(256);
-  const double2* xx = reinterpret_cast<const double2*>(x);
-  const double2* ll = reinterpret_cast<const double2*>(lam);
-  switch (t->p) {
-    case 1: hipLaunchKernelGGL(k_adjoint_grad<1>, gr, bl, 0, s, E, t->d_T, ws_coef(w), ws_orient(w, E), dofs, nrhs, sd, sr, xx, ll, d_om, g); break;
-    case 2: hipLaunchKernelGGL(k_adjoint_grad<2>, gr, bl, 0, s, E, t->d_T, ws_coef(w), ws_orient(w, E), dofs, nrhs, sd, sr, xx, ll, d_om, g); break;
-    case 3: hipLaunchKernelGGL(k_adjoint_grad<3>, gr, bl, 0, s, E, t->d_T, ws_coef(w), ws_orient(w, E), dofs, nrhs, sd, sr, xx, ll, d_om, g); break;
-  }
+  launch_adjoint_grad(t->p, E, ws_coef(w), ws_orient(w, E), dofs, ndof, nrhs, sd, sr,
+                      reinterpret_cast<const double2*>(x), reinterpret_cast<const double2*>(lam),
+                      om, g, s);
   PG_CHECK_LAUNCH();
-  // the host copy above is synchronous with respect to `om` only once the stream drains
   PG_HIP(hipStreamSynchronize(s));
-  if (!static_staging) PG_HIP(hipFreeAsync(d_om, s));
   return PG_OK;
 }
 
@@ -1239,8 +1132,7 @@ int pg_adjoint_gradient_noalloc(const void* tables, int64_t E, const void* ws,
                                 const int32_t* dofs, int nrhs, int64_t ndof, const double* x,
                                 const double* lam, const double* omega, double* g,
                                 void* stream) {
-  return adjoint_gradient(tables, E, ws, dofs, nrhs, ndof, 1, ndof, x, lam, omega, g, stream,
-                          true);
+  return adjoint_gradient(tables, E, ws, dofs, nrhs, ndof, 1, ndof, x, lam, omega, g, stream);
 }
 
 }  // extern "C"

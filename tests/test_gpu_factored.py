@@ -83,3 +83,35 @@ def test_products_on_arbitrary_orientations(p, n, keep):
         err = float((eop.apply(x) - ref).abs().max() / ref.abs().max())
         err32 = float((eop.apply(x.float()).double() - ref).abs().max() / ref.abs().max())
         assert err <= 1e-12 and err32 <= 1e-5, (err, err32)
+
+
+@pytest.mark.parametrize("p,n,keep,nrhs", [(1, 2, 1, 1), (1, 3, None, 33), (2, 2, 127, 2),
+                                           (2, 3, 129, 65), (3, 2, 47, 3)])
+@pytest.mark.parametrize("rows", [False, True])
+def test_adjoint_gradient_on_arbitrary_orientations(p, n, keep, nrhs, rows):
+    """-omega mu0 Im(lam^T M_e x) with the element matrices of pg_element_matrices in
+    64 bits, both column layouts, right-hand sides below, at and past the 32 of
+    one launch.  n^2 products of 1e-16 each, summed over the columns: 1e-12 of
+    the largest entry."""
+    import ctypes
+
+    from petgem_amd import _native as nat
+    T, mesh, asm, _ = _free(n, p, seed=n, keep=keep)
+    gen = torch.Generator(DEV).manual_seed(nrhs)
+    x, lam = (torch.randn((nrhs, T.ndof, 2), dtype=torch.float64, device=DEV, generator=gen)
+              for _ in range(2))
+    omega = np.linspace(1.0, 9.0, nrhs)
+    M, _ = asm.element_matrices()
+    d = torch.from_numpy(T.dofs).to(DEV)
+    xe, le = torch.view_as_complex(x)[:, d], torch.view_as_complex(lam)[:, d]
+    y = (M[None] * xe.real[:, :, None]).sum(-1) + 1j * (M[None] * xe.imag[:, :, None]).sum(-1)
+    w = torch.from_numpy(omega).to(DEV) * (4e-7 * np.pi)
+    ref = -(w[:, None] * (le * y).sum(-1).imag).sum(0)
+    if rows:
+        x, lam = (v.transpose(0, 1).contiguous() for v in (x, lam))
+    g = torch.zeros(T.n_elems, dtype=torch.float64, device=DEV)
+    fn = nat.lib().pg_adjoint_gradient_rows if rows else nat.lib().pg_adjoint_gradient
+    nat.check(fn(asm.tables.handle, mesh.n_elems, nat.ptr(asm.workspace), nat.ptr(mesh.dofs),
+                 nrhs, ctypes.c_int64(T.ndof), nat.ptr(x), nat.ptr(lam), nat.ptr(omega),
+                 nat.ptr(g), nat.stream_handle()))
+    assert float((g - ref).abs().max()) <= 1e-12 * float(ref.abs().max())
