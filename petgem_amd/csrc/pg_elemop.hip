@@ -128,7 +128,8 @@ __global__ void __launch_bounds__(kBS, (fac_waves<P, R>())) k_eop_fac(
     const R* __restrict__ coef, const R* __restrict__ x, R* __restrict__ ye) {
   constexpr int N = fac::n_dofs<P>();
   constexpr int NLE = n_local_entities<P>();
-  if (done && !wseg && *done) return;
+  // looked at below, with the first loads under way
+  const int32_t stop = done && !wseg ? *done : 0;
   // XCD-contiguous ranges of slot groups (workgroup b runs on XCD b % 8)
   const int64_t nb = gridDim.x;
   int64_t b = blockIdx.x;
@@ -153,6 +154,7 @@ __global__ void __launch_bounds__(kBS, (fac_waves<P, R>())) k_eop_fac(
     g[c] = coef[(w * 12 + c) * kWave + l];
     h[c] = coef[(w * 12 + 6 + c) * kWave + l];
   }
+  if (stop) return;
   R xv[N], y[N];
 #pragma unroll
   for (int la = 0; la < NLE; ++la) {
@@ -189,7 +191,7 @@ __global__ void __launch_bounds__(kBS) k_eop_sum(int64_t nent, const int32_t* __
                                                  const C* __restrict__ ye, const C* __restrict__ x,
                                                  C* __restrict__ y, const double2* __restrict__ b,
                                                  double* part) {
-  if (done && *done) return;
+  const int32_t stop = done ? *done : 0;
   const int64_t blk = blockIdx.x, nb = gridDim.x;
   int64_t first = blk * kBS, end = nent, stride = nb * kBS;
   if (nb % 8 == 0) {
@@ -199,8 +201,13 @@ __global__ void __launch_bounds__(kBS) k_eop_sum(int64_t nent, const int32_t* __
     stride = nbx * kBS;
   }
   double red[2] = {0.0, 0.0};
-  for (int64_t ent = first + threadIdx.x; ent < end; ent += stride) {
-    const int4 m = gm[ent];
+  int64_t ent = first + threadIdx.x;
+  int4 mn = make_int4(0, 0, 0, 0);
+  if (ent < end) mn = gm[ent];
+  if (stop) return;
+  for (; ent < end; ent += stride) {
+    const int4 m = mn;
+    if (ent + stride < end) mn = gm[ent + stride];
     const int r0 = m.x, d = m.y, s0 = m.z, s1 = m.w;
     // x at the entity's rows (identity rows; the MODE 1 dot product), loaded
     // before the sums so that its latency overlaps theirs

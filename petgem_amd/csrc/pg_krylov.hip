@@ -10,18 +10,19 @@
 //
 // Device organisation:
 //  * one HIP stream; a COCG iteration is
-//      p = z + beta p | q = A p (+ partials of p^T q) | finish mu, alpha |
-//      x += alpha p, r -= alpha q, z = P r (+ partials of r^T z, |r|^2) |
-//      finish rho, beta, convergence
+//      beta from r^T z of the last iteration; x += alpha p, p = z + beta p |
+//      q = A p (+ partials of p^T q) |
+//      alpha from them; r -= alpha q, z = P r (+ partials of r^T z, |r|^2)
 //    with every scalar in device memory;
 //  * reductions: each workgroup writes its partial sums with plain stores and
-//    a one-workgroup "finish" kernel adds them in a fixed order (bitwise
+//    the workgroups of the next kernel add them in a fixed order (bitwise
 //    reproducible).  The kernel boundary makes the partials visible, so no
 //    workgroup issues a device-scope fence (those force L2 write-backs
 //    across the XCDs and cost ~0.2 ms per kernel at this size);
-//  * every kernel returns immediately once the device-side `done` flag is
-//    set, so the host enqueues batches of iterations and reads the flags only
-//    between batches;
+//  * every kernel returns once the device-side `done` flag is set (read first,
+//    looked at when its first loads are under way: the flag comes from memory,
+//    about 1 us on a kernel that takes 4), so the host enqueues batches of
+//    iterations and reads the flags only between batches;
 //  * each XCD owns a contiguous eighth of the rows; in the SpMV its
 //    workgroups sweep that eighth together (row-interleaved) so that the
 //    gathers of x stay in the XCD's L2, in the vector kernels each workgroup
@@ -54,15 +55,22 @@ constexpr int kMaxGrid = 2048;
 constexpr int kMaxBlock = 8;
 constexpr int kMaxRestart = 128;
 
-struct Scal {
-  double2 rho, mu, alpha, beta;
-  double res2, bnorm2, tol2, ref2;
-  double res64;
-  int32_t iter, maxit, done, status;
+// what one iteration hands to the next; two records, so that a kernel whose
+// workgroups all read the last iteration's can write the next one's
+struct Rec {
+  double2 rho;
   // stagnation watch of the complex64 recursion (mixed precision): best |r|^2
   // of the current round and the iteration of its last 10 % improvement
   double best2;
-  int32_t last_imp, stall_limit, stalled, pad;
+  int32_t iter, last_imp;
+};
+struct Scal {
+  double2 mu, alpha, beta;
+  Rec rec[2];
+  double res2, bnorm2, tol2, ref2;
+  double res64;
+  int32_t iter, maxit, done, status;
+  int32_t stall_limit, stalled;
 };
 
 // a complex64 round whose best residual norm has not improved by 10 % for
@@ -161,23 +169,29 @@ __device__ inline void write_partials(double (&v)[NV], double* part) {
     for (int k = 0; k < NV; ++k) part[(int64_t)k * gridDim.x + blockIdx.x] = v[k];
 }
 
-// in a one-workgroup finish kernel: fixed-order totals of np partials; all threads
+// fixed-order totals of np partials, in every thread of the workgroup; two calls
+// in one kernel need a barrier between them
 template <int NV>
 __device__ inline void sum_partials(const double* part, int np, double (&tot)[NV]) {
-  double acc[NV];
+  __shared__ double sm[NV][kBS / kWave];
 #pragma unroll
-  for (int k = 0; k < NV; ++k) acc[k] = 0.0;
+  for (int k = 0; k < NV; ++k) tot[k] = 0.0;
   for (int i = threadIdx.x; i < np; i += kBS)
 #pragma unroll
-    for (int k = 0; k < NV; ++k) acc[k] += part[(int64_t)k * np + i];
-  block_reduce<NV>(acc);
-  __shared__ double res[NV];
-  if (threadIdx.x == 0)
+    for (int k = 0; k < NV; ++k) tot[k] += part[(int64_t)k * np + i];
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
 #pragma unroll
-    for (int k = 0; k < NV; ++k) res[k] = acc[k];
+  for (int k = 0; k < NV; ++k) tot[k] = wave_sum(tot[k]);
+  if (lane == 0)
+#pragma unroll
+    for (int k = 0; k < NV; ++k) sm[k][w] = tot[k];
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < NV; ++k) tot[k] = res[k];
+  for (int k = 0; k < NV; ++k) {
+    tot[k] = 0.0;
+#pragma unroll
+    for (int i = 0; i < kBS / kWave; ++i) tot[k] += sm[k][i];
+  }
 }
 
 // Matrix loads.  (Non-temporal loads were measured slower here: without L2
@@ -219,7 +233,7 @@ __global__ void __launch_bounds__(kBS) k_spmv(const Scal* __restrict__ s, int64_
                                               const VT* __restrict__ vals,
                                               const XT* __restrict__ x, XT* __restrict__ y,
                                               const double2* __restrict__ b, double* part) {
-  if (MODE != 0 && s->done) return;
+  const int32_t done = MODE != 0 ? s->done : 0;
   constexpr int RPB = kBS / G;
   const Sweep sw = xcd_sweep(n, RPB);
   const int lane = threadIdx.x % G;
@@ -230,6 +244,7 @@ __global__ void __launch_bounds__(kBS) k_spmv(const Scal* __restrict__ s, int64_
     s0n = rowptr[row];
     s1n = rowptr[row + 1];
   }
+  if (done) return;
   for (; row < sw.end; row += sw.stride) {
     const int s0 = s0n, s1 = s1n;
     const int64_t nx = row + sw.stride;
@@ -273,7 +288,7 @@ __global__ void __launch_bounds__(kBS) k_spmv_er(const Scal* __restrict__ s, int
                                                  const VT* __restrict__ vals,
                                                  const XT* __restrict__ x, XT* __restrict__ y,
                                                  const double2* __restrict__ b, double* part) {
-  if (MODE != 0 && s->done) return;
+  const int32_t done = MODE != 0 ? s->done : 0;
   constexpr int EPB = kBS / G;
   const Sweep sw = xcd_sweep(nent, EPB);
   const int lane = threadIdx.x % G;
@@ -281,6 +296,7 @@ __global__ void __launch_bounds__(kBS) k_spmv_er(const Scal* __restrict__ s, int
   int64_t ent = sw.first + threadIdx.x / G;
   int4 mn = make_int4(0, 0, 0, 0);
   if (ent < sw.end) mn = emeta[ent];
+  if (done) return;
   for (; ent < sw.end; ent += sw.stride) {
     const int r0 = mn.x, d = mn.y & 0xff, L = mn.y >> 8, cbase = mn.z, vbase = mn.w;
     const int64_t nx = ent + sw.stride;
@@ -347,7 +363,7 @@ __global__ void __launch_bounds__(kBS) k_spmv_er2(const Scal* __restrict__ s, in
                                                   const double2* __restrict__ b, double* part) {
   using VP = typename PairOf<VT>::type;
   using XP = typename PairOf<XT>::type;
-  if (MODE != 0 && s->done) return;
+  const int32_t done = MODE != 0 ? s->done : 0;
   constexpr int EPB = kBS / G;
   const Sweep sw = xcd_sweep(nent, EPB);
   const int lane = threadIdx.x % G;
@@ -355,6 +371,7 @@ __global__ void __launch_bounds__(kBS) k_spmv_er2(const Scal* __restrict__ s, in
   int64_t ent = sw.first + threadIdx.x / G;
   int4 mn = make_int4(0, 0, 0, 0);
   if (ent < sw.end) mn = emeta[ent];
+  if (done) return;
   for (; ent < sw.end; ent += sw.stride) {
     const int r0 = mn.x, L = mn.y >> 8, c2 = mn.z >> 1, vbase = mn.w;
     const int L2 = L >> 1;
@@ -448,23 +465,76 @@ __global__ void __launch_bounds__(kBS) k_sched_vals(int64_t nent, const int4* __
   for (int t = threadIdx.x % G; t < len; t += G) vals_s[m.w + t] = from_d<VT>(vals[base + t]);
 }
 
-// finish mu = p^T q, alpha = rho / mu
-__global__ void __launch_bounds__(kBS) k_fin_mu(Scal* __restrict__ s, const double* part,
-                                                int np) {
-  if (s->done) return;
-  double tot[2];
-  sum_partials<2>(part, np, tot);
-  if (threadIdx.x != 0) return;
-  const double2 mu = make_double2(tot[0], tot[1]);
+// ---------------------------------------------------------------------------
+// The two scalar steps of an iteration (alpha from p^T q; rho, beta and the
+// convergence decision from r^T z and |r|^2) are part of the kernels that need
+// their results: every workgroup adds all partials itself, in the same order,
+// and workgroup 0 stores the scalars.  As one-workgroup kernels of their own they
+// took 2.4 to 4 us each whatever the size; reading at most 2048 partials in every
+// workgroup costs less at all sizes: an iteration (element products, FP64, block
+// Jacobi) 30.3 -> 26.5 us at 91 000 DOFs, 46.4 -> 42.8 at 321 000, 214 -> 211 at
+// 2 480 000.  Only the last iteration before a host check is finished by a kernel
+// of its own (k_fin_update).
+// ---------------------------------------------------------------------------
+// alpha = rho / mu; false on a breakdown
+__device__ inline bool step_alpha(double2 rho, double2 mu, double2* alpha) {
+  *alpha = zdiv(rho, mu);
+  return (mu.x != 0.0 || mu.y != 0.0) && isfinite(alpha->x) && isfinite(alpha->y);
+}
+__device__ inline void store_alpha(Scal* s, double2 mu, double2 alpha, bool ok) {
   s->mu = mu;
-  const double2 al = zdiv(s->rho, mu);
-  if (!(mu.x != 0.0 || mu.y != 0.0) || !isfinite(al.x) || !isfinite(al.y)) {
+  s->alpha = ok ? alpha : make_double2(0.0, 0.0);
+  if (!ok) {
     s->status = PG_ERR_BREAKDOWN;
     s->done = 1;
-    s->alpha = make_double2(0.0, 0.0);
-  } else {
-    s->alpha = al;
   }
+}
+
+// rho, beta, |r|^2 and the convergence / pause decision; tot = r^T z, |r|^2
+struct Step {
+  double2 beta;
+  Rec rec;
+  bool broken, stalled, stop;
+};
+__device__ inline Step step_update(const Scal* s, const Rec& old, const double (&tot)[3]) {
+  Step t;
+  t.rec = old;
+  t.rec.rho = make_double2(tot[0], tot[1]);
+  t.beta = zdiv(t.rec.rho, old.rho);
+  t.rec.iter = old.iter + 1;
+  t.broken = !isfinite(tot[2]) || !isfinite(t.beta.x) || !isfinite(t.beta.y);
+  t.stalled = false;
+  // converged recursion, refinement point, or iteration limit
+  t.stop = t.broken || tot[2] <= s->tol2 * s->bnorm2 || tot[2] <= s->ref2 ||
+           t.rec.iter >= s->maxit;
+  if (!t.stop && s->stall_limit > 0) {
+    if (tot[2] < 0.81 * old.best2) {
+      t.rec.best2 = tot[2];
+      t.rec.last_imp = t.rec.iter;
+    } else if (t.rec.iter - old.last_imp >= s->stall_limit) {
+      t.stalled = t.stop = true;  // stagnated round
+    }
+  }
+  return t;
+}
+__device__ inline void store_step(Scal* s, Rec* to, const Step& t, double res2) {
+  s->beta = t.beta;
+  s->res2 = res2;
+  s->iter = t.rec.iter;
+  *to = t.rec;
+  if (t.broken) s->status = PG_ERR_BREAKDOWN;
+  if (t.stalled) s->stalled = 1;
+  if (t.stop) s->done = 1;
+}
+
+// alpha from the product's partials; false = return (a breakdown)
+__device__ inline bool get_alpha(Scal* s, const double* part, int np, int slot, double2* al) {
+  double tot[2];
+  sum_partials<2>(part, np, tot);
+  const double2 mu = make_double2(tot[0], tot[1]);
+  const bool ok = step_alpha(s->rec[slot].rho, mu, al);
+  if (blockIdx.x == 0 && threadIdx.x == 0) store_alpha(s, mu, *al, ok);
+  return ok;
 }
 
 // finish |b - A x|^2
@@ -483,25 +553,41 @@ __global__ void __launch_bounds__(kBS) k_fin_res64(Scal* __restrict__ s, const d
 // of the same iteration is taken by the next k_pupdate (which reads p anyway)
 // or, once the recursion pauses, by k_xstep.
 template <typename XT>
-__global__ void __launch_bounds__(kBS) k_update(const Scal* __restrict__ s, int64_t n,
-                                                XT* __restrict__ r, const XT* __restrict__ q,
-                                                const XT* __restrict__ dinv,
-                                                XT* __restrict__ z, double* part) {
-  if (s->done) return;
-  const double2 al = s->alpha;
-  const XT na = from_d<XT>(make_double2(-al.x, -al.y));
+__global__ void __launch_bounds__(kBS) k_update(Scal* s, int64_t n, XT* __restrict__ r,
+                                                const XT* __restrict__ q,
+                                                const XT* __restrict__ dinv, XT* __restrict__ z,
+                                                const double* pin, int np, int slot,
+                                                double* part) {
+  const int32_t done = s->done;
   int64_t lo, hi;
   chunk(n, kBS, &lo, &hi);
+  int64_t i = lo + threadIdx.x;
+  // the first elements are loaded before the scalars are finished
+  XT qv{}, rv{}, dv{};
+  const auto load = [&] {
+    if (i < hi) {
+      qv = q[i];
+      rv = r[i];
+      dv = dinv[i];
+    }
+  };
+  load();
+  if (done) return;
+  double2 al;
+  if (!get_alpha(s, pin, np, slot, &al)) return;
+  const XT na = from_d<XT>(make_double2(-al.x, -al.y));
   double red[3] = {0.0, 0.0, 0.0};
-  for (int64_t i = lo + threadIdx.x; i < hi; i += kBS) {
-    const XT ri = cfma(na, q[i], r[i]);
+  while (i < hi) {
+    const XT ri = cfma(na, qv, rv);
     r[i] = ri;
-    const XT zi = cm(dinv[i], ri);
+    const XT zi = cm(dv, ri);
     z[i] = zi;
     const double2 rd = to_d(ri), zd = to_d(zi);
     red[0] += rd.x * zd.x - rd.y * zd.y;
     red[1] += rd.x * zd.y + rd.y * zd.x;
     red[2] += rd.x * rd.x + rd.y * rd.y;
+    i += kBS;
+    load();
   }
   write_partials<3>(red, part);
 }
@@ -509,11 +595,12 @@ __global__ void __launch_bounds__(kBS) k_update(const Scal* __restrict__ s, int6
 // same with the entity-block preconditioner: one thread per block
 template <typename XT>
 __global__ void __launch_bounds__(kBS) k_update_blk(
-    const Scal* __restrict__ s, int64_t nb, const int32_t* __restrict__ bptr,
-    const int32_t* __restrict__ boff, XT* __restrict__ r, const XT* __restrict__ q,
-    const XT* __restrict__ binv, XT* __restrict__ z, double* part) {
+    Scal* s, int64_t nb, const int32_t* __restrict__ bptr, const int32_t* __restrict__ boff,
+    XT* __restrict__ r, const XT* __restrict__ q, const XT* __restrict__ binv,
+    XT* __restrict__ z, const double* pin, int np, int slot, double* part) {
   if (s->done) return;
-  const double2 al = s->alpha;
+  double2 al;
+  if (!get_alpha(s, pin, np, slot, &al)) return;
   const XT na = from_d<XT>(make_double2(-al.x, -al.y));
   int64_t lo, hi;
   chunk(nb, kBS, &lo, &hi);
@@ -550,24 +637,37 @@ __global__ void __launch_bounds__(kBS) k_update_blk(
 // 2k+1 and its inverse the four entries at 4k): one 16-byte (complex64) or
 // 32-byte (complex128) access per vector and block, and no block index reads.
 template <typename XT>
-__global__ void __launch_bounds__(kBS) k_update_blk2(const Scal* __restrict__ s, int64_t nb,
-                                                     XT* __restrict__ r,
+__global__ void __launch_bounds__(kBS) k_update_blk2(Scal* s, int64_t nb, XT* __restrict__ r,
                                                      const XT* __restrict__ q,
                                                      const XT* __restrict__ binv,
-                                                     XT* __restrict__ z, double* part) {
+                                                     XT* __restrict__ z, const double* pin,
+                                                     int np, int slot, double* part) {
   using V = typename PairOf<XT>::type;
-  if (s->done) return;
-  const double2 al = s->alpha;
-  const XT na = from_d<XT>(make_double2(-al.x, -al.y));
+  const int32_t done = s->done;
   int64_t lo, hi;
   chunk(nb, kBS, &lo, &hi);
-  double red[3] = {0.0, 0.0, 0.0};
   V* r2 = reinterpret_cast<V*>(r);
   V* z2 = reinterpret_cast<V*>(z);
   const V* q2 = reinterpret_cast<const V*>(q);
   const V* b2 = reinterpret_cast<const V*>(binv);
-  for (int64_t k = lo + threadIdx.x; k < hi; k += kBS) {
-    const V rv = r2[k], qv = q2[k], B0 = b2[2 * k], B1 = b2[2 * k + 1];
+  int64_t k = lo + threadIdx.x;
+  // the first blocks are loaded before the scalars are finished
+  V rv{}, qv{}, B0{}, B1{};
+  const auto load = [&] {
+    if (k < hi) {
+      rv = r2[k];
+      qv = q2[k];
+      B0 = b2[2 * k];
+      B1 = b2[2 * k + 1];
+    }
+  };
+  load();
+  if (done) return;
+  double2 al;
+  if (!get_alpha(s, pin, np, slot, &al)) return;
+  const XT na = from_d<XT>(make_double2(-al.x, -al.y));
+  double red[3] = {0.0, 0.0, 0.0};
+  while (k < hi) {
     const XT ra = cfma(na, XT{qv.x, qv.y}, XT{rv.x, rv.y});
     const XT rb = cfma(na, XT{qv.z, qv.w}, XT{rv.z, rv.w});
     r2[k] = V{ra.x, ra.y, rb.x, rb.y};
@@ -582,54 +682,62 @@ __global__ void __launch_bounds__(kBS) k_update_blk2(const Scal* __restrict__ s,
     red[0] += r1.x * z1.x - r1.y * z1.y;
     red[1] += r1.x * z1.y + r1.y * z1.x;
     red[2] += r1.x * r1.x + r1.y * r1.y;
+    k += kBS;
+    load();
   }
   write_partials<3>(red, part);
 }
 
 // finish rho, beta, |r|^2 and the convergence / pause decision
 __global__ void __launch_bounds__(kBS) k_fin_update(Scal* __restrict__ s, const double* part,
-                                                    int np) {
+                                                    int np, int from, int to) {
   if (s->done) return;
   double tot[3];
   sum_partials<3>(part, np, tot);
   if (threadIdx.x != 0) return;
-  const double2 rho_new = make_double2(tot[0], tot[1]);
-  const double2 beta = zdiv(rho_new, s->rho);
-  s->beta = beta;
-  s->rho = rho_new;
-  s->res2 = tot[2];
-  s->iter += 1;
-  if (!isfinite(tot[2]) || !isfinite(beta.x) || !isfinite(beta.y)) {
-    s->status = PG_ERR_BREAKDOWN;
-    s->done = 1;
-  } else if (tot[2] <= s->tol2 * s->bnorm2 || tot[2] <= s->ref2 || s->iter >= s->maxit) {
-    s->done = 1;  // converged recursion, refinement point, or iteration limit
-  } else if (s->stall_limit > 0) {
-    if (tot[2] < 0.81 * s->best2) {
-      s->best2 = tot[2];
-      s->last_imp = s->iter;
-    } else if (s->iter - s->last_imp >= s->stall_limit) {
-      s->stalled = 1;  // stagnated round
-      s->done = 1;
-    }
-  }
+  const Rec old = s->rec[from];
+  store_step(s, &s->rec[to], step_update(s, old, tot), tot[2]);
 }
 
 // x += alpha p (the previous iteration's step: alpha is still that iteration's,
-// and after a (re)start p = 0), then p = z + beta p
-template <typename XT>
-__global__ void __launch_bounds__(kBS) k_pupdate(const Scal* __restrict__ s, int64_t n,
-                                                 const XT* __restrict__ z, XT* __restrict__ p,
-                                                 XT* __restrict__ x) {
-  if (s->done) return;
-  const XT a = from_d<XT>(s->alpha);
-  const XT be = from_d<XT>(s->beta);
+// and after a (re)start p = 0), then p = z + beta p.  FUSE: the previous
+// iteration's k_fin_update first, from the record `from` to the other one `to`.
+template <typename XT, bool FUSE>
+__global__ void __launch_bounds__(kBS) k_pupdate(Scal* s, int64_t n, const XT* __restrict__ z,
+                                                 XT* __restrict__ p, XT* __restrict__ x,
+                                                 const double* pin, int np, int from, int to) {
+  const int32_t done = s->done;
   int64_t lo, hi;
   chunk(n, kBS, &lo, &hi);
-  for (int64_t i = lo + threadIdx.x; i < hi; i += kBS) {
-    const XT pv = p[i];
-    x[i] = cfma(a, pv, x[i]);
-    p[i] = cfma(be, pv, z[i]);
+  int64_t i = lo + threadIdx.x;
+  XT pv{}, xv{}, zv{};
+  const auto load = [&] {
+    if (i < hi) {
+      pv = p[i];
+      xv = x[i];
+      zv = z[i];
+    }
+  };
+  load();
+  if (done) return;
+  double2 beta;
+  if (FUSE) {
+    double tot[3];
+    sum_partials<3>(pin, np, tot);
+    const Step t = step_update(s, s->rec[from], tot);
+    if (blockIdx.x == 0 && threadIdx.x == 0) store_step(s, &s->rec[to], t, tot[2]);
+    if (t.stop) return;  // every workgroup decides the same
+    beta = t.beta;
+  } else {
+    beta = s->beta;
+  }
+  const XT a = from_d<XT>(s->alpha);
+  const XT be = from_d<XT>(beta);
+  while (i < hi) {
+    x[i] = cfma(a, pv, xv);
+    p[i] = cfma(be, pv, zv);
+    i += kBS;
+    load();
   }
 }
 
@@ -721,12 +829,10 @@ __global__ void __launch_bounds__(kBS) k_fin_reset(Scal* __restrict__ s, const d
   double tot[4];
   sum_partials<4>(part, np, tot);
   if (threadIdx.x != 0) return;
-  s->rho = make_double2(tot[0], tot[1]);
+  s->rec[0] = Rec{make_double2(tot[0], tot[1]), tot[2], s->iter, s->iter};
   s->beta = make_double2(0.0, 0.0);
   s->res2 = tot[2];
   if (has_b) s->bnorm2 = tot[3];
-  s->best2 = tot[2];
-  s->last_imp = s->iter;
   s->stalled = 0;
   s->done = 0;
 }
@@ -938,6 +1044,7 @@ __global__ void __launch_bounds__(kBS) k_reorth_test(const double* before, const
                                                      int np, int32_t* skip) {
   double b[1], a[1];
   sum_partials<1>(before, np, b);
+  __syncthreads();
   sum_partials<1>(after, np, a);
   if (threadIdx.x == 0) *skip = (a[0] > 0.5 * b[0]) ? 1 : 0;
 }
@@ -1078,6 +1185,7 @@ struct Solver {
   Scal* s = nullptr;
   Scal* h = nullptr;  // pinned host mirror
   double* part = nullptr;
+  double* part2 = nullptr;  // partials of the update (part: of the product)
   double2 *r = nullptr, *p = nullptr, *q = nullptr, *z = nullptr, *dinv = nullptr, *r64 = nullptr;
   float2 *r32 = nullptr, *p32 = nullptr, *q32 = nullptr, *z32 = nullptr, *x32 = nullptr,
          *dinv32 = nullptr;
@@ -1229,31 +1337,37 @@ static void launch_reset(Solver* S, hipStream_t st, XT* r, const XT* dinv, const
   hipLaunchKernelGGL(k_fin_reset, dim3(1), dim3(kBS), 0, st, S->s, S->part, np, b ? 1 : 0);
 }
 
+// iteration k of a batch of `count` between two host checks, with the records
+// rec[k & 1]; the batch begins from rec[0] and its k_fin_update ends there
 template <typename VT, typename XT>
 static void launch_iteration(Solver* S, hipStream_t st, const SpmvCfg& c, const VT* vals, XT* x,
-                             XT* r, XT* p, XT* q, const XT* dinv, const XT* binv, XT* z,
-                             bool sample) {
-  hipLaunchKernelGGL(k_pupdate<XT>, dim3(S->gv), dim3(kBS), 0, st, S->s, S->n, z, p, x);
+                             XT* r, XT* p, XT* q, const XT* dinv, const XT* binv, XT* z, int k,
+                             int count) {
+  const bool blk = S->o.pc == PG_PC_BJACOBI, sample = k == 0;
+  const int gu = blk ? S->gb : S->gv;  // workgroups (and partials) of the update
+  const int slot = k & 1;
+  const dim3 b(kBS);
+  if (k > 0)
+    hipLaunchKernelGGL((k_pupdate<XT, true>), dim3(S->gv), b, 0, st, S->s, S->n, z, p, x,
+                       S->part2, gu, slot ^ 1, slot);
+  else
+    hipLaunchKernelGGL((k_pupdate<XT, false>), dim3(S->gv), b, 0, st, S->s, S->n, z, p, x,
+                       nullptr, 0, 0, 0);
   // a failed record only loses this timing sample (the elapsed-time query fails)
   if (sample) (void)hipEventRecord(S->ev[0], st);
   spmv<1, VT, XT>(S, c, st, vals, p, q, nullptr, sample && c.kind == 3 ? S->ev[2] : nullptr);
   if (sample) (void)hipEventRecord(S->ev[1], st);
-  hipLaunchKernelGGL(k_fin_mu, dim3(1), dim3(kBS), 0, st, S->s, S->part, c.grid);
-  int np;
-  if (S->o.pc == PG_PC_BJACOBI && S->blk2) {  // r, q, z: the solver's own 256-byte aligned buffers
-    hipLaunchKernelGGL(k_update_blk2<XT>, dim3(S->gb), dim3(kBS), 0, st, S->s, S->nblocks, r, q,
-                       binv, z, S->part);
-    np = S->gb;
-  } else if (S->o.pc == PG_PC_BJACOBI) {
-    hipLaunchKernelGGL(k_update_blk<XT>, dim3(S->gb), dim3(kBS), 0, st, S->s, S->nblocks, S->bptr,
-                       S->boff, r, q, binv, z, S->part);
-    np = S->gb;
-  } else {
-    hipLaunchKernelGGL(k_update<XT>, dim3(S->gv), dim3(kBS), 0, st, S->s, S->n, r, q, dinv, z,
-                       S->part);
-    np = S->gv;
-  }
-  hipLaunchKernelGGL(k_fin_update, dim3(1), dim3(kBS), 0, st, S->s, S->part, np);
+  if (blk && S->blk2)  // r, q, z: the solver's own 256-byte aligned buffers
+    hipLaunchKernelGGL(k_update_blk2<XT>, dim3(gu), b, 0, st, S->s, S->nblocks, r, q, binv, z,
+                       S->part, c.grid, slot, S->part2);
+  else if (blk)
+    hipLaunchKernelGGL(k_update_blk<XT>, dim3(gu), b, 0, st, S->s, S->nblocks, S->bptr, S->boff,
+                       r, q, binv, z, S->part, c.grid, slot, S->part2);
+  else
+    hipLaunchKernelGGL(k_update<XT>, dim3(gu), b, 0, st, S->s, S->n, r, q, dinv, z, S->part,
+                       c.grid, slot, S->part2);
+  if (k == count - 1)
+    hipLaunchKernelGGL(k_fin_update, dim3(1), b, 0, st, S->s, S->part2, gu, slot, 0);
 }
 
 static int cocg_solve(Solver* S, const double2* b, double2* x, pg_solve_info* info,
@@ -1311,10 +1425,10 @@ static int cocg_solve(Solver* S, const double2* b, double2* x, pg_solve_info* in
     for (int k = 0; k < check; ++k) {
       if (low)
         launch_iteration<float2, float2>(S, st, S->c32, S->vals32, S->x32, S->r32, S->p32, S->q32,
-                                         S->dinv32, S->binv32, S->z32, k == 0);
+                                         S->dinv32, S->binv32, S->z32, k, check);
       else
         launch_iteration<double2, double2>(S, st, S->c64, S->vals, x, S->r, S->p, S->q, S->dinv,
-                                           S->binv, S->z, k == 0);
+                                           S->binv, S->z, k, check);
     }
     PG_CHECK_LAUNCH();
     PG_TRY(read_scalars(S, st));
@@ -1837,6 +1951,7 @@ int pg_solver_create(int64_t n, int64_t nnz, const int32_t* rowptr, const int32_
   }
   PG_A(S->s, 1);
   PG_A(S->part, 4 * kMaxGrid);
+  PG_A(S->part2, 4 * kMaxGrid);
   PG_A(S->r64, n);
   PG_A(S->q, n);
   PG_A(S->bad, 1);
