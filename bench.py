@@ -54,8 +54,9 @@ def spmv_key(code, dmax, vt, p=2):
     """Kernel name (as the profile summaries print it) of the solve's SpMV from the
     solver's configuration code kind*1000 + G*10 + U."""
     kind, g, u = code // 1000, (code % 1000) // 10, code % 10
-    if kind == 3:  # element products
-        return "k_eop_fac<{},{}>".format(p, "float" if vt == "float2" else "double")
+    if kind == 3:  # element products (p = 3: followed by the per-entity sums)
+        t = "float" if vt == "float2" else "double"
+        return f"k_eop_fac<3,{t}>" if p == 3 else f"k_eop_blk<{p},{t},1>"
     if kind == 2:
         return f"k_spmv_er2<{g},{u},1,{vt},{vt}>"
     if kind == 1:
@@ -68,10 +69,11 @@ def roofline_entry(code, res, standalone_ms, vt, T, plan, dmax, traffic):
     """Roofline of the first kernel of the solve's SpMV.
 
     CSR kinds: HBM-bound, algorithmic bytes = spmv_bytes.  Element-by-element
-    operator (kind 3): its element-product kernel is bound by the vector ALU
-    (FP32 or FP64 FMA issue), so it is priced in algorithmic flops (eop_flops)
-    against the FP32 / FP64 peak; the summation kernel that follows it is
-    HBM-bound and reported beside it with its algorithmic bytes."""
+    operator (kind 3): its element products are priced in flops with every
+    element counted once (eop_flops; at p <= 2 the elements on the border of a
+    workgroup's cluster are computed more than once) against the FP32 / FP64
+    vector peak, with the bytes they cannot do without beside them; at p = 3 the
+    summation kernel that follows is HBM-bound and reported separately."""
     bv = 8 if vt == "float2" else 16
     n, nnz = plan.ndof, plan.nnz
     key = spmv_key(code, dmax, vt, T.p)
@@ -82,15 +84,11 @@ def roofline_entry(code, res, standalone_ms, vt, T, plan, dmax, traffic):
         fl = eop_flops(T.n_elems, T.p)
         peak = FP32_PEAK_TFLOPS if vt == "float2" else FP64_PEAK_TFLOPS
         ach = fl / (ms * 1e-3) / 1e12
-        # summation kernel: 16-byte entity descriptors, one 4-byte slot per
-        # (entity, element) incidence, the n local results of every element,
-        # p read and q written
-        nle = 6 if T.p == 1 else 10
-        nent = T.n_edges + (T.n_faces if T.p >= 2 else 0)
-        sum_bytes = 16 * nent + 4 * T.n_elems * nle + T.n_elems * T.n_dof_elem * bv + 2 * n * bv
-        sum_ms = max(res["spmv_ms"] - ms, 1e-9)
+        nle = {1: 6, 2: 10, 3: 11}[T.p]
+        # coefficients, entities and orientation of every element, p read, q written
+        by = T.n_elems * (12 * bv // 2 + 4 * nle + 4) + 2 * n * bv
         out.update({
-            "bound": "valu", "kernel": f"{key} (element products y_e = A_e p_e)",
+            "bound": "valu", "kernel": f"{key} (element products)",
             "achieved": round(ach, 2), "peak": peak, "unit": "TFLOP/s",
             "frac": round(ach / peak, 4), "traffic": traffic.get(key),
             "algorithmic_flops": fl, "avg_ms": round(ms, 5),
@@ -99,13 +97,21 @@ def roofline_entry(code, res, standalone_ms, vt, T, plan, dmax, traffic):
                      if vt == "float2" else
                      "vector-ALU FP64 FMA kernel (no matrix-core work); peak = MI355X FP64 "
                      "vector rate"),
-            "sum_kernel": {"bound": "hbm", "avg_ms": round(sum_ms, 5),
-                           "algorithmic_bytes": sum_bytes,
-                           "achieved": round(sum_bytes / (sum_ms * 1e-3) / 1e9, 1),
-                           "unit": "GB/s", "peak": HBM_PEAK_GBS,
-                           "frac": round(sum_bytes / (sum_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)},
+            "algorithmic_bytes": by,
             "csr_equivalent_bytes": spmv_bytes(nnz, n, bv),
         })
+        if T.p == 3:
+            # 16-byte entity descriptors, one 4-byte slot per (entity, element)
+            # incidence, the n local results of every element, p read, q written
+            nent = T.n_edges + T.n_faces + T.n_elems
+            sum_bytes = (16 * nent + 4 * T.n_elems * nle + T.n_elems * T.n_dof_elem * bv
+                         + 2 * n * bv)
+            sum_ms = max(res["spmv_ms"] - ms, 1e-9)
+            sum_gbs = sum_bytes / (sum_ms * 1e-3) / 1e9
+            out["sum_kernel"] = {"bound": "hbm", "avg_ms": round(sum_ms, 5),
+                                 "algorithmic_bytes": sum_bytes, "achieved": round(sum_gbs, 1),
+                                 "unit": "GB/s", "peak": HBM_PEAK_GBS,
+                                 "frac": round(sum_gbs / HBM_PEAK_GBS, 4)}
     else:
         ms = res["spmv_ms"]
         by = spmv_bytes(nnz, n, bv)

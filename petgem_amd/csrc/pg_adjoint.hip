@@ -48,6 +48,12 @@ __global__ void __launch_bounds__(kBS, (P == 1 ? 3 : (P == 2 ? 2 : 1))) k_adjoin
     const double* __restrict__ x, const double* __restrict__ lam, const Omegas om,
     double* __restrict__ g) {
   constexpr int N = fac::n_dofs<P>();
+  __shared__ double faces[fac::face_table_size<P>()];
+  if constexpr (P > 1) {
+    constexpr auto t = fac::kFaces<P>;
+    for (int i = threadIdx.x; i < fac::face_table_size<P>(); i += kBS) faces[i] = t.v[i];
+    __syncthreads();
+  }
   const int64_t nb = gridDim.x;
   int64_t b = blockIdx.x;
   if (nb % 8 == 0) b = (b % 8) * (nb / 8) + b / 8;  // XCD-contiguous ranges of elements
@@ -68,12 +74,12 @@ __global__ void __launch_bounds__(kBS, (P == 1 ? 3 : (P == 2 ? 2 : 1))) k_adjoin
     double xv[N], m[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) xv[i] = at(xr, off[i]);
-    fac::orient_in<P>(pk, xv);
+    fac::orient_in<P>(pk, faces, xv);
     fac::mass_product<P, double>(xv, cf, [&](int i, double v) { m[i] = v; });
     // p = 3: lam is loaded once the intermediates are gone (it would spill);
     // p = 2: during them
     if (P == 3) __builtin_amdgcn_sched_barrier(0);
-    fac::orient_out<P>(pk, m);
+    fac::orient_out<P>(pk, faces, m);
     double s = 0.0;
 #pragma unroll
     for (int i = 0; i < N; ++i) s += at(lr, off[i]) * m[i];

@@ -2,14 +2,15 @@
 //     A = sum_e P_e^T (K_e - i omega mu0 M_e) P_e,   PEC rows and columns -> identity,
 // for gfx950, as an alternative to the CSR SpMV inside the Krylov solver.
 //
-// The element matrices are never stored.  The product is split in two kernels:
+// The element matrices are never stored: two lanes take one element (real and
+// imaginary part), any orientation, and form K_e x and M_e x from 12 geometric
+// coefficients by expanding field and curl in Bernstein monomials (pg_factor.h).
+// Two forms:
 //
-//  k_eop_fac    two lanes per element (real and imaginary part), any
-//               orientation, K_e x and M_e x from 12 geometric coefficients by
-//               expanding field and curl in Bernstein monomials (pg_factor.h):
-//               no table, 820 operations per real vector at p = 2 and 3 200 at
-//               p = 3; writes the element's n local results y_e = A_e x_e (slot
-//               layout [group][i][element of 64]).
+//  k_eop_blk    p <= 2: one kernel; a workgroup owns a cluster of entities,
+//               computes every element around them and sums their results in LDS.
+//  k_eop_fac    the element products alone, writing the elements' n local results
+//               (slot layout [group][i][element of 64]), and
 //  k_eop_sum    one thread per mesh entity (edge, face), in the entity
 //               schedule: sums the entity's local results over its elements
 //               in a fixed order (atomic-free, bitwise reproducible), and
@@ -39,7 +40,7 @@ constexpr int kMaxGrid = 2048;
 // waves per SIMD the element products are compiled for
 template <int P, typename R>
 constexpr int fac_waves() {
-  return P == 3 ? (sizeof(R) == 8 ? 1 : 2) : (sizeof(R) == 8 ? 3 : 6);
+  return P == 3 ? (sizeof(R) == 8 ? 1 : 2) : (sizeof(R) == 8 ? 3 : 5);
 }
 constexpr double kMu0 = 4.0 * 3.14159265358979323846 * 1e-7;  // petgem/solver.py:175
 
@@ -83,6 +84,16 @@ __device__ inline double swap_pair(double v) {
   return __hiloint2double(swap_pair(__double2hiint(v)), swap_pair(__double2loint(v)));
 }
 
+// the face coefficients of the factored products, to LDS; all threads
+template <int P, typename R>
+__device__ inline void fac_fill(R* faces) {
+  if constexpr (P > 1) {
+    constexpr auto t = fac::kFaces<P>;
+    for (int i = threadIdx.x; i < fac::face_table_size<P>(); i += blockDim.x) faces[i] = (R)t.v[i];
+    __syncthreads();
+  }
+}
+
 template <int NV>
 __device__ inline void write_partials(double (&v)[NV], double* part) {
   __shared__ double sm[NV][kBS / kWave];
@@ -103,8 +114,8 @@ __device__ inline void write_partials(double (&v)[NV], double* part) {
 }
 
 // ---------------------------------------------------------------------------
-// local products in factored form (pg_factor.h).  Slots: group w of 64 elements, element l of the group; edofs[w][la][l] = first global DOF of
-// local entity la, -1 for a PEC entity or an empty slot (its x is taken as 0);
+// local products in factored form (pg_factor.h).  Slots: group w of 64 elements,
+// element l of the group; edofs[w][la][l] = first global DOF of local entity la, -1 for a PEC entity or an empty slot (its x is taken as 0);
 // ocode[w][l] the packed orientation; coef[w][c][l]: c < 6 the mass
 // coefficients times -omega mu0, c >= 6 the curl-curl coefficients.  Two
 // neighbouring lanes take one element: lane 2 i the real part of x, lane
@@ -128,6 +139,8 @@ __global__ void __launch_bounds__(kBS, (fac_waves<P, R>())) k_eop_fac(
     const R* __restrict__ coef, const R* __restrict__ x, R* __restrict__ ye) {
   constexpr int N = fac::n_dofs<P>();
   constexpr int NLE = n_local_entities<P>();
+  __shared__ R faces[fac::face_table_size<P>()];
+  fac_fill<P>(faces);
   // looked at below, with the first loads under way
   const int32_t stop = done && !wseg ? *done : 0;
   // XCD-contiguous ranges of slot groups (workgroup b runs on XCD b % 8)
@@ -167,13 +180,13 @@ __global__ void __launch_bounds__(kBS, (fac_waves<P, R>())) k_eop_fac(
 #pragma unroll
     for (int k = 0; k < loc_nd<P>(la); ++k)
       xv[loc_off<P>(la) + k] = f[la] >= 0 ? xv[loc_off<P>(la) + k] : R(0);
-  fac::orient_in<P>(code, xv);
+  fac::orient_in<P>(code, faces, xv);
   const R sg = part ? R(1) : R(-1);
   fac::mass_product<P, R>(xv, g, [&](int i, R v) { y[i] = sg * swap_pair(v); });
   __builtin_amdgcn_sched_barrier(0);  // one product's intermediates at a time
   fac::curl_product<P, R>(xv, h, [&](int i, R v) { y[i] += v; });
   asm("" : "+v"(code));  // the coefficients again, not kept through the products
-  fac::orient_out<P>(code, y);
+  fac::orient_out<P>(code, faces, y);
 #pragma unroll
   for (int i = 0; i < N; ++i) ye[((w * N + i) * kWave + l) * 2 + part] = y[i];
 }
@@ -281,6 +294,151 @@ __global__ void __launch_bounds__(kBS) k_eop_sum(int64_t nent, const int32_t* __
 }
 
 // ---------------------------------------------------------------------------
+// The whole product in one kernel: a workgroup owns a run of scheduled entities
+// (a spatial cluster when the schedule is spatial), computes every element that
+// touches them (128 elements, two lanes each, as k_eop_fac), keeps the local
+// results of its own entities in LDS and sums each entity there in the slot
+// order of k_eop_sum (bitwise the two-kernel result), so the local results never
+// reach memory.  Elements on the border of a cluster are computed by every
+// workgroup that owns one of their entities.
+//   bmeta[b]      {first schedule position, entities, first element group, groups}
+//   bslot[g][l]   slot of element l < 128 of group g, -1 empty
+//   bcode, bdofs  its orientation and entities (as ocode, edofs)
+//   bpos[g][q][l] LDS places of its local entities 2 q and 2 q + 1 (16 bits each,
+//                 in complex values; 0xFFFF = not owned here)
+//   em[i]         {first DOF, place | incidences << 16 | DOFs << 28} of entity i
+// MODE as k_eop_sum.
+// Bound: FP64 / FP32 issue (900 vector instructions per wave of 32 elements, each
+// element 1.8 to 2.1 times) next to 180 MB of indices, coefficients, x and y.
+// Against the two kernels: 384 000 elements, p = 2: 71 us (complex128, 98 before)
+// and 53 us (complex64, 54; 85 against 105 inside the solve, where nothing of the
+// local results is in cache); 13 182 elements 10.9 against 13.2 us, one launch
+// less.  Loading the next block's indices ahead of the sums was slower (the
+// registers spill or cost a wave per SIMD).
+// ---------------------------------------------------------------------------
+constexpr int kGroup = kBS / 2;  // elements per pass of a workgroup
+
+template <int P, typename R, int MODE>
+__global__ void __launch_bounds__(kBS, (fac_waves<P, R>())) k_eop_blk(
+    int64_t nblk, const int32_t* __restrict__ done, const int4* __restrict__ bmeta,
+    const int32_t* __restrict__ bslot, const int32_t* __restrict__ bcode,
+    const int32_t* __restrict__ bdofs, const uint32_t* __restrict__ bpos,
+    const int2* __restrict__ em, const R* __restrict__ coef, const R* __restrict__ x,
+    typename Cx<R>::T* __restrict__ y, const double2* __restrict__ rhs, double* part) {
+  using C = typename Cx<R>::T;
+  constexpr int N = fac::n_dofs<P>();
+  constexpr int NLE = n_local_entities<P>();
+  constexpr int NQ = (NLE + 1) / 2;
+  static_assert(P <= 2, "entities of up to two DOFs");
+  constexpr int D = P;  // DOFs of an entity
+  extern __shared__ __align__(16) char smem[];
+  __shared__ R faces[fac::face_table_size<P>()];
+  const int32_t stop = done ? *done : 0;
+  const int tid = threadIdx.x, el = tid >> 1, part_ = tid & 1;
+  // XCD x (workgroup b runs on XCD b % 8) takes the x-th eighth of the blocks
+  const int64_t nb = gridDim.x;
+  int64_t b = blockIdx.x, end = nblk, stride = nb;
+  if (nb % 8 == 0) {
+    const int64_t xc = b % 8;
+    b = nblk * xc / 8 + b / 8;
+    end = nblk * (xc + 1) / 8;
+    stride = nb / 8;
+  }
+  int4 bm{0, 0, 0, 0};
+  if (b < end) bm = bmeta[b];
+  fac_fill<P>(faces);
+  if (stop) return;
+  double red[2] = {0.0, 0.0};
+  while (b < end) {
+    R* acc = reinterpret_cast<R*>(smem);
+    for (int64_t g = bm.z; g < bm.z + bm.w; ++g) {
+      const int slot = bslot[g * kGroup + el];
+      int code = bcode[g * kGroup + el];
+      int f[NLE];
+#pragma unroll
+      for (int la = 0; la < NLE; ++la) f[la] = bdofs[(g * NLE + la) * kGroup + el];
+      uint32_t pos[NQ];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) pos[q] = bpos[(g * NQ + q) * kGroup + el];
+      const R* cf = coef + 12 * (int64_t)(slot >= 0 ? slot : 0);
+      R gm[6], h[6];
+#pragma unroll
+      for (int c = 0; c < 6; ++c) {
+        gm[c] = cf[c];
+        h[c] = cf[6 + c];
+      }
+      R xv[N], yv[N];
+      bool pec = false;
+#pragma unroll
+      for (int la = 0; la < NLE; ++la) {
+        pec |= f[la] < 0;
+        const R* xe = x + 2 * (int64_t)(f[la] >= 0 ? f[la] : 0) + part_;
+#pragma unroll
+        for (int k = 0; k < loc_nd<P>(la); ++k) xv[loc_off<P>(la) + k] = xe[2 * k];
+      }
+      if (__any(pec)) {  // few waves hold a PEC entity or an empty place
+#pragma unroll
+        for (int la = 0; la < NLE; ++la)
+#pragma unroll
+          for (int k = 0; k < loc_nd<P>(la); ++k)
+            xv[loc_off<P>(la) + k] = f[la] >= 0 ? xv[loc_off<P>(la) + k] : R(0);
+      }
+      fac::orient_in<P>(code, faces, xv);
+      const R sg = part_ ? R(1) : R(-1);
+      fac::mass_product<P, R>(xv, gm, [&](int i, R v) { yv[i] = sg * swap_pair(v); });
+      __builtin_amdgcn_sched_barrier(0);  // one product's intermediates at a time
+      fac::curl_product<P, R>(xv, h, [&](int i, R v) { yv[i] += v; });
+      asm("" : "+v"(code));  // the coefficients again, not kept through the products
+      fac::orient_out<P>(code, faces, yv);
+#pragma unroll
+      for (int la = 0; la < NLE; ++la) {
+        const uint32_t at = (la & 1) ? pos[la / 2] >> 16 : pos[la / 2] & 0xFFFFu;
+        if (at != 0xFFFFu)
+#pragma unroll
+          for (int k = 0; k < loc_nd<P>(la); ++k)
+            acc[2 * (at + k) + part_] = yv[loc_off<P>(la) + k];
+      }
+    }
+    const int4 cm = bm;
+    b += stride;
+    if (b < end) bm = bmeta[b];
+    __syncthreads();
+    for (int i = tid; i < cm.y * D; i += kBS) {
+      const int2 e = em[cm.x + i / D];
+      const int t = i % D, d = (uint32_t)e.y >> 28, n = (e.y >> 16) & 0xFFF, row = e.x + t;
+      if (t >= d) continue;
+      C s{0, 0}, xr{0, 0};
+      if (MODE == 1 || n == 0) xr = reinterpret_cast<const C*>(x)[row];
+      if (n == 0) s = xr;  // PEC: identity row
+      const C* v = reinterpret_cast<const C*>(smem) + (e.y & 0xFFFF) + t;
+      for (int q = 0; q < n; ++q) {
+        s.x += v[q * d].x;
+        s.y += v[q * d].y;
+      }
+      if (MODE == 2) {
+        const double2 bb = rhs[row];
+        const double2 rr = make_double2(bb.x - (double)s.x, bb.y - (double)s.y);
+        store(y + row, rr);
+        red[0] += rr.x * rr.x + rr.y * rr.y;
+      } else {
+        y[row] = s;
+        if (MODE == 1) {
+          const double2 pv = to_d(xr), qv = to_d(s);
+          red[0] += pv.x * qv.x - pv.y * qv.y;
+          red[1] += pv.x * qv.y + pv.y * qv.x;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (MODE == 1) write_partials<2>(red, part);
+  if (MODE == 2) {
+    double r1[1] = {red[0]};
+    write_partials<1>(r1, part);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // multi-right-hand-side local products for the batched solver: column r of the
 // (ndof, R) row-major block x gets y_e,r = (K_e - i omega_r mu0 M_e) x_e,r.
 // One workgroup of 2 R threads (thread 2 r + part = the real or imaginary part
@@ -314,6 +472,8 @@ __global__ void __launch_bounds__(512, 3) k_meop_local(
     R* __restrict__ ye, double* __restrict__ dpart) {
   constexpr int N = fac::n_dofs<P>();
   constexpr int NLE = n_local_entities<P>();
+  __shared__ double faces[fac::face_table_size<P>()];
+  fac_fill<P>(faces);
   if (done && *done) return;
   const int64_t nb = gridDim.x;
   int64_t b = blockIdx.x;
@@ -348,7 +508,7 @@ __global__ void __launch_bounds__(512, 3) k_meop_local(
       for (int k = 0; k < loc_nd<P>(la); ++k)
         xv[loc_off<P>(la) + k] = f[la] >= 0 ? (double)x[(f[la] + k) * ld + t] : 0.0;
     int code = ocode[w * kWave + l];
-    fac::orient_in<P>(code, xv);
+    fac::orient_in<P>(code, faces, xv);
     fac::mass_product<P, double>(xv, g, [&](int i, double v) { y[i] = om * swap_pair(v); });
     __builtin_amdgcn_sched_barrier(0);  // one product's intermediates at a time
     fac::curl_product<P, double>(xv, h, [&](int i, double v) { y[i] += v; });
@@ -359,7 +519,7 @@ __global__ void __launch_bounds__(512, 3) k_meop_local(
       dim += xv[i] * swap_pair(y[i]);
     }
     asm("" : "+s"(code));  // the coefficients again, not kept through the products
-    fac::orient_out<P>(code, y);
+    fac::orient_out<P>(code, faces, y);
 #pragma unroll
     for (int i = 0; i < N; ++i) ye[((w * N + i) * kWave + l) * ld + t] = (R)y[i];
   }
@@ -372,12 +532,13 @@ __global__ void __launch_bounds__(512, 3) k_meop_local(
 }
 
 // coefficients in slot order: mass part times -omega mu0, then curl-curl part
-// (multi-mesh operator: omega mu0 of the wave's segment, womu[wseg[w]])
+// (multi-mesh operator: omega mu0 of the wave's segment, womu[wseg[w]]); the 12 of
+// a slot together (by_slot) or [group][c][element of 64]
 template <typename R>
 __global__ void k_eop_coef(int64_t nslot, const int32_t* __restrict__ perm,
                            const double* __restrict__ wscoef, double omega_mu,
                            const int32_t* __restrict__ wseg, const double* __restrict__ womu,
-                           R* __restrict__ coef) {
+                           int by_slot, R* __restrict__ coef) {
   const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nslot) return;
   const int64_t w = s / kWave, lane = s % kWave;
@@ -387,7 +548,7 @@ __global__ void k_eop_coef(int64_t nslot, const int32_t* __restrict__ perm,
   for (int c = 0; c < 12; ++c) {
     double v = e >= 0 ? wscoef[12 * e + c] : 0.0;
     if (c < 6) v = -(om * v);
-    coef[(w * 12 + c) * kWave + lane] = (R)v;
+    coef[by_slot ? s * 12 + c : (w * 12 + c) * kWave + lane] = (R)v;
   }
 }
 
@@ -410,6 +571,15 @@ struct ElemOp {
   // multi-right-hand-side products (eop_multi_prepare): raw coefficients in
   // slot order (mass part without -omega mu0)
   double* coefm = nullptr;
+  // one-kernel product (k_eop_blk) of a one-mesh operator, p <= 2; nblk = 0: the
+  // two kernels (p = 3, multi-mesh operators, and meshes with an entity of more
+  // elements than a workgroup takes)
+  int64_t nblk = 0;
+  int lds_values = 0;  // complex values of LDS per workgroup
+  int4* bmeta = nullptr;
+  int32_t *bslot = nullptr, *bcode = nullptr, *bdofs = nullptr;
+  uint32_t* bpos = nullptr;
+  int2* em = nullptr;
   // multi-mesh operator (pg_eop_create_multi): segment of every wave, omega mu0
   // of every segment, first schedule position of every segment (nseg + 1)
   int nseg = 0;
@@ -469,27 +639,55 @@ static void launch_impl(const ElemOp* op, int mode, const int32_t* done,
                         const double2* b, double* part, hipStream_t st, hipEvent_t mid,
                         typename eop::Cx<R>::T* ye, const R* coef) {
   using C = typename eop::Cx<R>::T;
-  launch_local<R>(op, done, nullptr, 0, x, ye, coef, st);
-  // a failed record only loses this timing sample (the elapsed-time query fails)
-  if (mid) (void)hipEventRecord(mid, st);
   const dim3 g(op->grid), bl(eop::kBS);
+#define PG_MODES(CALL) \
+  if (mode == 0) {     \
+    CALL(0);           \
+  } else if (mode == 1) { \
+    CALL(1);           \
+  } else {             \
+    CALL(2);           \
+  }
+  if (op->nblk > 0) {
+    const R* xr = reinterpret_cast<const R*>(x);
+#define PG_BLK(P, MM)                                                                           \
+  hipLaunchKernelGGL((eop::k_eop_blk<P, R, MM>), g, bl, op->lds_values * sizeof(C), st, op->nblk, \
+                     done, op->bmeta, op->bslot, op->bcode, op->bdofs, op->bpos, op->em, coef, xr, \
+                     y, b, part)
+#define PG_BLK1(MM) PG_BLK(1, MM)
+#define PG_BLK2(MM) PG_BLK(2, MM)
+    if (op->p == 1) {
+      PG_MODES(PG_BLK1)
+    } else {
+      PG_MODES(PG_BLK2)
+    }
+#undef PG_BLK1
+#undef PG_BLK2
+#undef PG_BLK
+    // a failed record only loses this timing sample (the elapsed-time query fails)
+    if (mid) (void)hipEventRecord(mid, st);
+    return;
+  }
+  launch_local<R>(op, done, nullptr, 0, x, ye, coef, st);
+  if (mid) (void)hipEventRecord(mid, st);
 #define PG_SUM(DD, MM)                                                                        \
   hipLaunchKernelGGL((eop::k_eop_sum<DD, MM, C>), g, bl, 0, st, op->nent, done, op->gm,       \
                      op->gslot, (const C*)ye, x, y, b, part)
+#define PG_SUM1(MM) PG_SUM(1, MM)
+#define PG_SUM2(MM) PG_SUM(2, MM)
+#define PG_SUM6(MM) PG_SUM(6, MM)
   if (op->D == 1) {
-    if (mode == 0) PG_SUM(1, 0);
-    else if (mode == 1) PG_SUM(1, 1);
-    else PG_SUM(1, 2);
+    PG_MODES(PG_SUM1)
   } else if (op->D == 2) {
-    if (mode == 0) PG_SUM(2, 0);
-    else if (mode == 1) PG_SUM(2, 1);
-    else PG_SUM(2, 2);
+    PG_MODES(PG_SUM2)
   } else {
-    if (mode == 0) PG_SUM(6, 0);
-    else if (mode == 1) PG_SUM(6, 1);
-    else PG_SUM(6, 2);
+    PG_MODES(PG_SUM6)
   }
+#undef PG_SUM1
+#undef PG_SUM2
+#undef PG_SUM6
 #undef PG_SUM
+#undef PG_MODES
 }
 
 void eop_launch(const ElemOp* op, int mode, const int32_t* done, const double2* x, double2* y,
@@ -507,13 +705,13 @@ static int eop_refresh(ElemOp* op, const void* ws, double omega, hipStream_t st)
   const double om = omega * eop::kMu0;
   const dim3 g((unsigned)((nslot + 255) / 256)), b(256);
   hipLaunchKernelGGL(eop::k_eop_coef<double>, g, b, 0, st, nslot, op->perm, wscoef, om,
-                     op->wseg, op->womu, op->coef64);
+                     op->wseg, op->womu, op->nblk > 0, op->coef64);
   hipLaunchKernelGGL(eop::k_eop_coef<float>, g, b, 0, st, nslot, op->perm, wscoef, om,
-                     op->wseg, op->womu, op->coef32);
+                     op->wseg, op->womu, op->nblk > 0, op->coef32);
   // raw coefficients: -(-1 * v) = v exactly
   if (op->coefm)
     hipLaunchKernelGGL(eop::k_eop_coef<double>, g, b, 0, st, nslot, op->perm, wscoef, -1.0,
-                       nullptr, nullptr, op->coefm);
+                       nullptr, nullptr, 0, op->coefm);
   PG_CHECK_LAUNCH();
   return PG_OK;
 }
@@ -529,7 +727,7 @@ int eop_multi_prepare(ElemOp* op, const void* ws, hipStream_t st) {
   const int64_t nslot = op->nw * kWave;
   const dim3 g((unsigned)((nslot + 255) / 256)), b(256);
   hipLaunchKernelGGL(eop::k_eop_coef<double>, g, b, 0, st, nslot, op->perm,
-                     reinterpret_cast<const double*>(ws), -1.0, nullptr, nullptr, op->coefm);
+                     reinterpret_cast<const double*>(ws), -1.0, nullptr, nullptr, 0, op->coefm);
   PG_CHECK_LAUNCH();
   return PG_OK;
 }
@@ -615,6 +813,75 @@ static int check_block_ptr(int p, const int32_t* bp, int64_t nblocks, int64_t nd
   return PG_OK;
 }
 
+// Blocks of k_eop_blk from the schedule (gm, and per incidence its slot and local
+// entity), each slot's orientation and entities: entities are taken in schedule
+// order while the elements around them fit `passes` groups and their local results
+// the LDS budget.  False when one entity alone does not fit.
+struct Blocks {
+  std::vector<int4> meta;
+  std::vector<int32_t> slot, code, dofs;
+  std::vector<uint32_t> pos;
+  std::vector<int2> em;
+  int lds_values = 1;
+};
+static bool make_blocks(int nle, int passes, const std::vector<int4>& gm,
+                        const std::vector<int32_t>& islot, const std::vector<uint8_t>& ila,
+                        const std::vector<int32_t>& hoc, const std::vector<int32_t>& hed,
+                        Blocks* B) {
+  constexpr int G = eop::kGroup;
+  constexpr int kMaxEnt = 1024;     // entities per block (PEC entities have no elements)
+  constexpr int kMaxValues = 3072;  // complex128 values of LDS: 48 KB, three workgroups
+  const int64_t nent = (int64_t)gm.size();
+  const int nq = (nle + 1) / 2;
+  std::vector<int32_t> stamp(hoc.size(), -1);  // block that last took the slot
+  std::vector<int32_t> place(hoc.size());      // and its element number there
+  const size_t ng0 = hoc.size() / G * 5 / 2 + 1;  // each element about twice
+  B->slot.reserve(ng0 * G);
+  B->code.reserve(ng0 * G);
+  B->dofs.reserve(ng0 * G * nle);
+  B->pos.reserve(ng0 * G * nq);
+  B->em.resize(nent);
+  for (int64_t i = 0; i < nent;) {
+    const int32_t b = (int32_t)B->meta.size();
+    const int64_t i0 = i, g0 = (int64_t)B->slot.size() / G;
+    int ne = 0, nv = 0;
+    for (; i < nent && i - i0 < kMaxEnt; ++i) {
+      const int4 m = gm[i];
+      const int n = m.w - m.z;
+      int fresh = 0;
+      for (int k = m.z; k < m.w; ++k) fresh += stamp[islot[k]] != b;
+      if (n > 0xFFF || ne + fresh > passes * G || nv + n * m.y > kMaxValues) break;
+      B->em[i] = make_int2(m.x, (int)((uint32_t)nv | (uint32_t)n << 16 | (uint32_t)m.y << 28));
+      for (int k = m.z; k < m.w; ++k) {
+        const int64_t s = islot[k];
+        if (stamp[s] != b) {
+          stamp[s] = b;
+          place[s] = ne++;
+          const int64_t g = g0 + place[s] / G, e = place[s] % G;
+          if (e == 0) {
+            B->slot.resize((g + 1) * G, -1);
+            B->code.resize((g + 1) * G, 0);
+            B->dofs.resize((g + 1) * G * nle, -1);
+            B->pos.resize((g + 1) * G * nq, 0xFFFFFFFFu);
+          }
+          B->slot[g * G + e] = (int32_t)s;
+          B->code[g * G + e] = hoc[s];
+          for (int la = 0; la < nle; ++la)
+            B->dofs[(g * nle + la) * G + e] = hed[(s / kWave * nle + la) * kWave + s % kWave];
+        }
+        const int la = ila[k];
+        uint32_t& at = B->pos[((g0 + place[s] / G) * nq + la / 2) * G + place[s] % G];
+        at = (la & 1) ? (at & 0xFFFFu) | (uint32_t)nv << 16 : (at & 0xFFFF0000u) | (uint32_t)nv;
+        nv += m.y;
+      }
+    }
+    if (i == i0) return false;
+    B->meta.push_back(make_int4((int)i0, (int)(i - i0), (int)g0, (ne + G - 1) / G));
+    B->lds_values = std::max(B->lds_values, nv);
+  }
+  return true;
+}
+
 static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32_t* bp,
                      int64_t nblocks, const int32_t* order, const std::vector<int32_t>& hd,
                      const std::vector<int32_t>& hor, const std::vector<uint8_t>& hbc,
@@ -679,11 +946,12 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
       es[e] = sm;
     }
   }
-  std::vector<int64_t> sorted(E);
-  std::iota(sorted.begin(), sorted.end(), 0);
-  std::stable_sort(sorted.begin(), sorted.end(), [&](int64_t a, int64_t b) {
-    return es[a] != es[b] ? es[a] < es[b] : key[a] < key[b];
-  });
+  // (stable counting sort; a segment's schedule positions are consecutive, so the
+  // position alone also orders the segments)
+  std::vector<int32_t> first(nblocks + 1, 0), sorted(E);
+  for (int64_t e = 0; e < E; ++e) first[key[e] + 1]++;
+  for (int64_t i = 0; i < nblocks; ++i) first[i + 1] += first[i];
+  for (int64_t e = 0; e < E; ++e) sorted[first[key[e]]++] = (int32_t)e;
   // slot groups of 64 elements of one segment
   std::vector<int32_t> perm, wsg;
   for (int64_t k = 0; k < E;) {
@@ -692,7 +960,7 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     while (k1 < E && es[sorted[k1]] == sg) ++k1;
     for (int64_t a = k; a < k1; a += kWave) {
       wsg.push_back(sg);
-      for (int l = 0; l < kWave; ++l) perm.push_back(a + l < k1 ? (int32_t)sorted[a + l] : -1);
+      for (int l = 0; l < kWave; ++l) perm.push_back(a + l < k1 ? sorted[a + l] : -1);
     }
     k = k1;
   }
@@ -720,7 +988,8 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     start[i + 1] = start[i] + (hbc[g] ? 0 : cnt[g]);
   }
   if (start[nblocks] >= (1LL << 31)) PG_FAIL(PG_ERR_UNSUPPORTED, "too many incidences");
-  std::vector<int32_t> gslot(start[nblocks]);
+  std::vector<int32_t> gslot(start[nblocks]), islot(start[nblocks]);  // local result, slot
+  std::vector<uint8_t> ila(start[nblocks]);                           // local entity
   std::vector<int64_t> cur(nblocks);
   for (int64_t g = 0; g < nblocks; ++g) cur[g] = start[pos[g]];
   for (int64_t s = 0; s < nslot; ++s) {
@@ -730,7 +999,10 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     for (int la = 0; la < nle; ++la) {
       const int g = eg[e * nle + la];
       if (hbc[g]) continue;
-      gslot[cur[g]++] = (int32_t)((w * N + entity_local_offset(la, p)) * kWave + l);
+      const int64_t c = cur[g]++;
+      gslot[c] = (int32_t)((w * N + entity_local_offset(la, p)) * kWave + l);
+      islot[c] = (int32_t)s;
+      ila[c] = (uint8_t)la;
     }
   }
   std::vector<int4> gm(nblocks);
@@ -738,6 +1010,17 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     const int64_t g = order ? order[i] : i;
     gm[i] = make_int4(bp[g], bp[g + 1] - bp[g], (int)start[i], (int)start[i + 1]);
   }
+  // The one-kernel product at p <= 2.  Two groups per block from 131 072 elements:
+  // fewer elements are computed twice (1.8 against 2.1 times each, p = 2), but a
+  // block takes two passes, which pays once the blocks fill the chip several
+  // times (us per FP64 iteration with one / two: 40.4 / 46.8 at 48 000 elements,
+  // 66.7 / 64.6 at 105 000, 92 / 90 at 162 000, 196 / 182 at 384 000; mixed
+  // precision 50.2 / 53.8 at 105 000, 73 / 70 at 162 000, 116 / 106 at 384 000).
+  // At p = 3 an element costs four times as much and the two kernels are faster
+  // (product at 82 944 elements 58 against 80 us, at 10 000 the same).
+  Blocks B;
+  const int passes = E >= (1 << 17) ? 2 : 1;
+  if (seg || p > 2 || !make_blocks(nle, passes, gm, islot, ila, hoc, hed, &B)) B = Blocks();
   int rc = PG_OK;
   ElemOp* op = new ElemOp();
   op->p = p;
@@ -748,7 +1031,9 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   op->nent = nblocks;
   op->nw = nw;
   {
-    int64_t g = (nblocks + eop::kBS - 1) / eop::kBS;
+    op->nblk = (int64_t)B.meta.size();
+    op->lds_values = B.lds_values;
+    int64_t g = op->nblk > 0 ? op->nblk : (nblocks + eop::kBS - 1) / eop::kBS;
     g = std::min<int64_t>(g, eop::kMaxGrid);
     if (g >= 64) g = (g / 8) * 8;
     op->grid = (int)std::max<int64_t>(g, 1);
@@ -765,8 +1050,17 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   PG_A(op->gslot, gslot.size());
   PG_A(op->coef64, nslot * 12);
   PG_A(op->coef32, nslot * 12);
-  PG_A(op->ye64, nslot * N);
-  PG_A(op->ye32, nslot * N);
+  if (op->nblk > 0) {
+    PG_A(op->bmeta, B.meta.size());
+    PG_A(op->bslot, B.slot.size());
+    PG_A(op->bcode, B.code.size());
+    PG_A(op->bdofs, B.dofs.size());
+    PG_A(op->bpos, B.pos.size());
+    PG_A(op->em, B.em.size());
+  } else {
+    PG_A(op->ye64, nslot * N);
+    PG_A(op->ye32, nslot * N);
+  }
   std::vector<double> womu;
   if (seg) {
     op->nseg = seg->nseg;
@@ -789,6 +1083,12 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
             {op->ocode, hoc.data(), hoc.size() * sizeof(int32_t)},
             {op->gm, gm.data(), gm.size() * sizeof(int4)},
             {op->gslot, gslot.data(), gslot.size() * sizeof(int32_t)},
+            {op->bmeta, B.meta.data(), B.meta.size() * sizeof(int4)},
+            {op->bslot, B.slot.data(), op->nblk ? B.slot.size() * sizeof(int32_t) : 0},
+            {op->bcode, B.code.data(), op->nblk ? B.code.size() * sizeof(int32_t) : 0},
+            {op->bdofs, B.dofs.data(), op->nblk ? B.dofs.size() * sizeof(int32_t) : 0},
+            {op->bpos, B.pos.data(), op->nblk ? B.pos.size() * sizeof(uint32_t) : 0},
+            {op->em, B.em.data(), op->nblk ? B.em.size() * sizeof(int2) : 0},
             {op->wseg, wsg.data(), op->wseg ? wsg.size() * sizeof(int32_t) : 0},
             {op->womu, womu.data(), womu.size() * sizeof(double)}};
   for (const auto& u : up)

@@ -79,24 +79,49 @@ PG_HD constexpr int mono(int i, int j) {
 // so with c the coefficients of f_0, f_1, f_2 from the pair's two, c_j =
 // sum_m e[j][m] x_m, the code-0 coefficients are c_0, c_1 plus c_2 times f_2's.
 // ---------------------------------------------------------------------------
-struct FacePerm {
-  int e[3][2];  // in {0, +-1}
-  int s;        // -1 for codes 3..5
-  PG_HD FacePerm(int packed, int f) {
-    // f_m of code o is +-f_j of code 0: j, and the sign, two bits per code
-    constexpr int v[6][6] = {{1, 0, 0, 0, -1, 0}, {0, 0, 1, 0, 0, -1}, {0, 1, 0, 0, 0, -1},
-                             {1, 0, 0, -1, 0, 0}, {0, 0, 1, -1, 0, 0}, {0, 1, 0, 0, -1, 0}};
-    const int sh = 30 - 2 * ((packed >> (6 + 3 * f)) & 7);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      unsigned pk = 0;
-#pragma unroll
-      for (int o = 0; o < 6; ++o) pk |= (unsigned)(v[k][o] & 3) << (2 * o);
-      e[k / 2][k % 2] = (int)(pk << sh) >> 30;
-    }
-    s = (packed >> (6 + 3 * f) & 7) >= 3 ? -1 : 1;
-  }
+// The coefficients by code are read from a table of face_entries<P>() values per
+// code, which a kernel keeps in LDS (fill_faces): they differ from lane to lane,
+// and forming them from the code took a fifth of the instructions at p = 2.
+//   p = 2: c_0, c_1 after f_2 = -f_0 - f_1: t[m][j] = e[j][m] - e[2][m]
+//   p = 3: e[j][m], and the sign -1 for codes 3..5
+PG_HD constexpr int face_perm_entry(int o, int j, int m) {
+  // f_m of code o is +-f_j of code 0
+  constexpr int v[6][3][2] = {{{1, 0}, {0, 1}, {0, 0}},   {{0, 0}, {1, 0}, {0, 1}},
+                              {{0, 1}, {0, 0}, {1, 0}},   {{0, 0}, {0, -1}, {-1, 0}},
+                              {{-1, 0}, {0, 0}, {0, -1}}, {{0, -1}, {-1, 0}, {0, 0}}};
+  return v[o][j][m];
+}
+template <int P>
+PG_HD constexpr int face_entries() {
+  return P == 3 ? 8 : 4;
+}
+template <int P>
+PG_HD constexpr int face_table_size() {
+  return P == 1 ? 1 : 8 * face_entries<P>();  // codes 6, 7 do not occur
+}
+template <int P>
+PG_HD constexpr int face_table(int i) {
+  const int o = i / face_entries<P>(), k = i % face_entries<P>();
+  if (P == 1 || o > 5) return 0;
+  if (P == 2) return face_perm_entry(o, k % 2, k / 2) - face_perm_entry(o, 2, k / 2);
+  return k < 6 ? face_perm_entry(o, k / 2, k % 2) : (k == 6 ? (o > 2 ? -1 : 1) : 0);
+}
+template <int P>
+struct FaceTable {
+  int v[face_table_size<P>()];
 };
+template <int P>
+constexpr FaceTable<P> make_face_table() {
+  FaceTable<P> t{};
+  for (int i = 0; i < face_table_size<P>(); ++i) t.v[i] = face_table<P>(i);
+  return t;
+}
+template <int P>
+inline constexpr FaceTable<P> kFaces = make_face_table<P>();
+template <int P, typename R>
+PG_HD const R* face_row(const R* tab, int packed, int f) {
+  return tab + ((packed >> (6 + 3 * f)) & 7) * face_entries<P>();
+}
 // f_2 of face f, kind t (0: phi = lambda_c^2 / 2 - .., 1: phi = (lambda_b -
 // lambda_a) lambda_c): coefficient of function k < 6 of the face, k - 6 of the volume
 PG_HD constexpr double face_third(int f, int t, int k) {
@@ -107,9 +132,9 @@ PG_HD constexpr double face_third(int f, int t, int k) {
                                  {{-0.75, -0.75, -0.75}, {-0.5, -0.5, 0.5}}};
   return k < 6 ? c[t][k] : b[f][t][k - 6];
 }
-// x -> coefficients of the code-0 functions
+// x -> coefficients of the code-0 functions; tab = the table of face coefficients
 template <int P, typename R>
-PG_HD void orient_in(int packed, R* x) {
+PG_HD void orient_in(int packed, const R* tab, R* x) {
 #pragma unroll
   for (int e = 0; e < 6; ++e) {
     const R s = (packed >> e) & 1 ? R(-1) : R(1);
@@ -119,20 +144,20 @@ PG_HD void orient_in(int packed, R* x) {
   if constexpr (P >= 2)
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
-      const FacePerm q(packed, f);
+      const R* q = face_row<P>(tab, packed, f);
       R* xf = x + 6 * P + f * P * (P - 1);
       if constexpr (P == 2) {
         const R a = xf[0], b = xf[1];
-        xf[0] = R(q.e[0][0] - q.e[2][0]) * a + R(q.e[0][1] - q.e[2][1]) * b;
-        xf[1] = R(q.e[1][0] - q.e[2][0]) * a + R(q.e[1][1] - q.e[2][1]) * b;
+        xf[0] = q[0] * a + q[2] * b;
+        xf[1] = q[1] * a + q[3] * b;
       } else {
         R c[3][3];  // [pair][j]
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
           R a = xf[2 * t], b = xf[2 * t + 1];
-          if (t == 2) a = R(q.s) * a, b = R(q.s) * b;
+          if (t == 2) a = q[6] * a, b = q[6] * b;
 #pragma unroll
-          for (int j = 0; j < 3; ++j) c[t][j] = R(q.e[j][0]) * a + R(q.e[j][1]) * b;
+          for (int j = 0; j < 3; ++j) c[t][j] = q[2 * j] * a + q[2 * j + 1] * b;
         }
 #pragma unroll
         for (int k = 0; k < 6; ++k) xf[k] = c[k / 2][k % 2];
@@ -148,7 +173,7 @@ PG_HD void orient_in(int packed, R* x) {
 }
 // moments against the code-0 functions -> against the element's own
 template <int P, typename R>
-PG_HD void orient_out(int packed, R* y) {
+PG_HD void orient_out(int packed, const R* tab, R* y) {
 #pragma unroll
   for (int e = 0; e < 6; ++e) {
     const R s = (packed >> e) & 1 ? R(-1) : R(1);
@@ -158,12 +183,12 @@ PG_HD void orient_out(int packed, R* y) {
   if constexpr (P >= 2)
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
-      const FacePerm q(packed, f);
+      const R* q = face_row<P>(tab, packed, f);
       R* yf = y + 6 * P + f * P * (P - 1);
       if constexpr (P == 2) {
         const R a = yf[0], b = yf[1];
-        yf[0] = R(q.e[0][0] - q.e[2][0]) * a + R(q.e[1][0] - q.e[2][0]) * b;
-        yf[1] = R(q.e[0][1] - q.e[2][1]) * a + R(q.e[1][1] - q.e[2][1]) * b;
+        yf[0] = q[0] * a + q[1] * b;
+        yf[1] = q[2] * a + q[3] * b;
       } else {
         R d[3][3];
 #pragma unroll
@@ -180,8 +205,8 @@ PG_HD void orient_out(int packed, R* y) {
         for (int t = 0; t < 3; ++t)
 #pragma unroll
           for (int m = 0; m < 2; ++m) {
-            const R v = R(q.e[0][m]) * d[t][0] + (R(q.e[1][m]) * d[t][1] + R(q.e[2][m]) * d[t][2]);
-            yf[2 * t + m] = t == 2 ? R(q.s) * v : v;
+            const R v = q[m] * d[t][0] + (q[2 + m] * d[t][1] + q[4 + m] * d[t][2]);
+            yf[2 * t + m] = t == 2 ? q[6] * v : v;
           }
       }
     }

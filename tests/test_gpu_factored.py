@@ -65,13 +65,15 @@ def test_batch_products_on_arbitrary_orientations(p, n, nrhs, precision):
 
 
 @pytest.mark.parametrize("p,n,keep", [(1, 2, 1), (1, 3, 65), (2, 2, 31), (2, 2, 33), (2, 3, 64),
-                                      (2, 4, 129), (2, 4, None), (3, 2, 1), (3, 2, 33),
+                                      (2, 4, 129), (2, 4, None), (1, 28, None), (3, 2, 1),
+                                      (3, 2, 33),
                                       (3, 3, None)])
 def test_products_on_arbitrary_orientations(p, n, keep):
     """y = A x on the operator against the assembled CSR: element counts around the
-    32 elements of a wave, the 64 of a slot group and the 128 of a workgroup, in
-    both precisions and, for complex128, x at an address that is not a
-    multiple of 32 bytes.  Bars as for the structured grids: 1e-12 and 1e-5."""
+    32 elements of a wave, the 64 of a slot group and the 128 of a workgroup, and
+    past the 131 072 from which a workgroup takes two groups, in both precisions
+    and, for complex128, x at an address that is not a multiple of 32 bytes.
+    Bars as for the structured grids: 1e-12 and 1e-5."""
     T, mesh, asm, _ = _free(n, p, seed=n, keep=keep)
     omega = core.omega_of(0.5)
     vals = asm.assemble(omega)
