@@ -94,6 +94,22 @@ __host__ __device__ inline int32_t* ws_orient(void* ws, int64_t E) {
 }
 __host__ __device__ inline int32_t* ws_flag(void* ws, int64_t E) { return ws_orient(ws, E) + E; }
 
+// orientation code of a face from its first two edges g0, g1 and the owner's three
+__device__ inline int face_code(int g0, int g1, const int32_t* fe) {
+  int k1 = 0, k2 = 0;
+  for (int k = 0; k < 3; ++k) {
+    if (g0 == fe[k]) k1 = k + 1;
+    if (g1 == fe[k]) k2 = k + 1;
+  }
+  const int sel = k1 * 10 + k2;
+  if (sel == 31) return 1;
+  if (sel == 23) return 2;
+  if (sel == 32) return 3;
+  if (sel == 13) return 4;
+  if (sel == 21) return 5;
+  return 0;
+}
+
 __device__ inline int element_orientation(const int32_t* en, const int32_t* ee, const int32_t* edn,
                                           const int32_t* fe, int* eo, int* fo) {
   int packed = 0;
@@ -104,20 +120,7 @@ __device__ inline int element_orientation(const int32_t* en, const int32_t* ee, 
     packed |= flag << i;
   }
   for (int f = 0; f < 4; ++f) {
-    const int g0 = ee[face_edge(f, 0)], g1 = ee[face_edge(f, 1)];
-    int k1 = 0, k2 = 0;
-    for (int k = 0; k < 3; ++k) {
-      if (g0 == fe[3 * f + k]) k1 = k + 1;
-      if (g1 == fe[3 * f + k]) k2 = k + 1;
-    }
-    const int sel = k1 * 10 + k2;
-    int code = 0;
-    if (sel == 12) code = 0;
-    else if (sel == 31) code = 1;
-    else if (sel == 23) code = 2;
-    else if (sel == 32) code = 3;
-    else if (sel == 13) code = 4;
-    else if (sel == 21) code = 5;
+    const int code = face_code(ee[face_edge(f, 0)], ee[face_edge(f, 1)], fe + 3 * f);
     fo[f] = code;
     packed |= code << (6 + 3 * f);
   }
@@ -670,8 +673,11 @@ __device__ inline bool barycentric_inside(const double* c, const double* x, doub
   return last >= -tol && last <= 1.0 + tol;
 }
 
-__global__ void k_locate(int64_t E, const double* __restrict__ coords, int64_t npts,
-                         const double* __restrict__ pts, double tol, int32_t* __restrict__ out) {
+// one thread per element and slice of the points (gridDim.y slices); out starts
+// at -1, the largest unsigned value
+__global__ void __launch_bounds__(256) k_locate(int64_t E, const double* __restrict__ coords,
+                                                int64_t npts, const double* __restrict__ pts,
+                                                double tol, int32_t* __restrict__ out) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= E) return;
   const double* c = coords + 12 * e;
@@ -680,13 +686,15 @@ __global__ void k_locate(int64_t E, const double* __restrict__ coords, int64_t n
     lo[k] = fmin(fmin(c[k], c[3 + k]), fmin(c[6 + k], c[9 + k]));
     hi[k] = fmax(fmax(c[k], c[3 + k]), fmax(c[6 + k], c[9 + k]));
   }
-  for (int64_t q = 0; q < npts; ++q) {
+  const double sl = 1e-6 * (hi[0] - lo[0] + hi[1] - lo[1] + hi[2] - lo[2]);
+  const int64_t q1 = npts * (blockIdx.y + 1) / gridDim.y;
+  for (int64_t q = npts * blockIdx.y / gridDim.y; q < q1; ++q) {
     const double* x = pts + 3 * q;
-    const double sl = 1e-6 * (hi[0] - lo[0] + hi[1] - lo[1] + hi[2] - lo[2]);
     if (x[0] < lo[0] - sl || x[0] > hi[0] + sl || x[1] < lo[1] - sl || x[1] > hi[1] + sl ||
         x[2] < lo[2] - sl || x[2] > hi[2] + sl)
       continue;
-    if (barycentric_inside(c, x, tol)) atomicMin(&out[q], (int32_t)e);
+    if (barycentric_inside(c, x, tol))
+      atomicMin(reinterpret_cast<unsigned*>(out + q), (unsigned)e);
   }
 }
 
@@ -694,130 +702,239 @@ __global__ void k_fill_i32(int64_t n, int32_t* p, int32_t v) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-__global__ void k_notfound(int64_t n, int32_t* p) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && p[i] == 0x7fffffff) p[i] = -1;
-}
 
 // -------------------------------------------------------------------------
-// basis at a physical point of one element (source and receivers)
+// basis at a physical point of one element (source, receivers, adjoint source):
+// one thread per local entity of the element that contains the point.  Bound by
+// latency: one thread per point, which held all n functions in scratch memory and
+// formed them one after another, took 12.6 us for 101 receivers and 7.3 us for a
+// source at p = 2; these take 6.0 and 4.0.
 // -------------------------------------------------------------------------
+struct ElemArrays {
+  const double* coords;
+  const int32_t *en, *ee, *edn, *fe, *dofs;
+};
+__device__ inline double pick(const double (&l)[4], int i) {
+  return i == 0 ? l[0] : (i == 1 ? l[1] : (i == 2 ? l[2] : l[3]));
+}
+__device__ inline V3 pick_grad(int i) {
+  return i == 0 ? v3(-1.0, -1.0, -1.0) : v3(i == 1 ? 1.0 : 0.0, i == 2 ? 1.0 : 0.0, i == 3 ? 1.0 : 0.0);
+}
+
+// the functions of local entity la of element e at x (and their curls), in
+// physical space; returns their number
 template <int P>
-__device__ inline void physical_basis(const double* c, const int32_t* en, const int32_t* ee,
-                                      const int32_t* edn, const int32_t* fe, const double* x,
-                                      V3* N, V3* Cu) {
-  constexpr int n = P * (P + 2) * (P + 3) / 2;
+__device__ inline int physical_entity(const ElemArrays& A, int64_t e, int la, const double* x, V3* N,
+                                      V3* Cu) {
   double J[3][3], iJ[3][3], det;
+  const double* c = A.coords + 12 * e;
   jacobian(c, J, iJ, &det);
   // reference coordinates: xi = J^-T (x - x0)
   const double r[3] = {x[0] - c[0], x[1] - c[1], x[2] - c[2]};
   double X[3];
   for (int a = 0; a < 3; ++a) X[a] = r[0] * iJ[0][a] + r[1] * iJ[1][a] + r[2] * iJ[2][a];
-  int eo[6], fo[4];
-  element_orientation(en, ee, edn, fe, eo, fo);
-  V3 S[n], C[n];
-  element_functions(X, eo, fo, P, S, C);
-  for (int i = 0; i < n; ++i) {
-    const V3 s = S[i], u = C[i];
-    N[i] = v3(iJ[0][0] * s.x + iJ[0][1] * s.y + iJ[0][2] * s.z,
-              iJ[1][0] * s.x + iJ[1][1] * s.y + iJ[1][2] * s.z,
-              iJ[2][0] * s.x + iJ[2][1] * s.y + iJ[2][2] * s.z);
-    Cu[i] = v3((J[0][0] * u.x + J[1][0] * u.y + J[2][0] * u.z) / det,
-               (J[0][1] * u.x + J[1][1] * u.y + J[2][1] * u.z) / det,
-               (J[0][2] * u.x + J[1][2] * u.y + J[2][2] * u.z) / det);
+  double lam[4];
+  V3 dlam[4];
+  affine(X, lam, dlam);
+  constexpr int DF = P * (P - 1), MAXD = P == 1 ? 1 : DF;
+  V3 S[MAXD], C[MAXD];
+  int nd;
+  if (la < 6) {
+    const int32_t *en = A.en + 4 * e, *edn = A.edn + 12 * e + 2 * la;
+    int a = edge_vert(la, 0), b = edge_vert(la, 1);
+    if (en[a] == edn[1] && en[b] == edn[0]) {
+      const int t = a;
+      a = b;
+      b = t;
+    }
+    anc_edge(pick(lam, a), pick(lam, b), pick_grad(a), pick_grad(b), P, S, C);
+    nd = P;
+  } else if (P >= 2 && la < 10) {
+    const int f = la - 6;
+    const int32_t *ee = A.ee + 6 * e, *fe = A.fe + 12 * e + 3 * f;
+    const int o = face_code(ee[face_edge(f, 0)], ee[face_edge(f, 1)], fe);
+    int g[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) g[k] = face_vert(f, face_perm(o, k));
+#pragma unroll
+    for (int fam = 0; fam < 2; ++fam) {
+      double s[3];
+      V3 ds[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const int v = g[(fam + k) % 3];
+        s[k] = pick(lam, v);
+        ds[k] = pick_grad(v);
+      }
+      V3 ET[kJ][kJ], CT[kJ][kJ];
+      anc_tri(s, ds, P, ET, CT);
+      int m = fam;
+#pragma unroll
+      for (int k = 1; k < P; ++k)
+#pragma unroll
+        for (int q = 0; q < k; ++q) {
+          S[m] = ET[q][k - q - 1];
+          C[m] = CT[q][k - q - 1];
+          m += 2;
+        }
+    }
+    nd = DF;
+  } else {
+    bubble_functions(lam, dlam, P, S, C);
+    nd = P * (P - 1) * (P - 2) / 2;
   }
+#pragma unroll
+  for (int i = 0; i < MAXD; ++i)
+    if (i < nd) {
+      const V3 s = S[i], u = C[i];
+      N[i] = v3(iJ[0][0] * s.x + iJ[0][1] * s.y + iJ[0][2] * s.z,
+                iJ[1][0] * s.x + iJ[1][1] * s.y + iJ[1][2] * s.z,
+                iJ[2][0] * s.x + iJ[2][1] * s.y + iJ[2][2] * s.z);
+      Cu[i] = v3((J[0][0] * u.x + J[1][0] * u.y + J[2][0] * u.z) / det,
+                 (J[0][1] * u.x + J[1][1] * u.y + J[2][1] * u.z) / det,
+                 (J[0][2] * u.x + J[1][2] * u.y + J[2][2] * u.z) / det);
+    }
+  return nd;
+}
+template <int P>
+__device__ inline int entity_first(int la) {
+  return la < 6 ? la * P : (la < 10 ? 6 * P + (la - 6) * P * (P - 1) : 6 * P + 4 * P * (P - 1));
 }
 
 template <int P>
-__global__ void k_source(int32_t e, const double* __restrict__ coords,
-                         const int32_t* __restrict__ en, const int32_t* __restrict__ ee,
-                         const int32_t* __restrict__ edn, const int32_t* __restrict__ fe,
-                         const int32_t* __restrict__ dofs, const double* __restrict__ pos,
-                         const double* __restrict__ moment, double omega_mu,
-                         double2* __restrict__ b) {
-  constexpr int n = P * (P + 2) * (P + 3) / 2;
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  V3 N[n], Cu[n];
-  const int64_t E = e;
-  physical_basis<P>(coords + 12 * E, en + 4 * E, ee + 6 * E, edn + 12 * E, fe + 12 * E, pos, N,
-                    Cu);
-  for (int i = 0; i < n; ++i) {
+__global__ void __launch_bounds__(64) k_source(int32_t e, ElemArrays A,
+                                               const double* __restrict__ pos,
+                                               const double* __restrict__ moment, double omega_mu,
+                                               double2* __restrict__ b) {
+  constexpr int n = P * (P + 2) * (P + 3) / 2, MAXD = P == 1 ? 1 : P * (P - 1);
+  const int la = threadIdx.x;
+  if (la >= asm_nloc<P>()) return;
+  V3 N[MAXD], Cu[MAXD];
+  const int nd = physical_entity<P>(A, e, la, pos, N, Cu);
+  for (int i = 0; i < nd; ++i) {
     const double v = moment[0] * N[i].x + moment[1] * N[i].y + moment[2] * N[i].z;
-    const int g = dofs[E * n + i];
-    double2 bi = b[g];
-    bi.y += omega_mu * v;
-    b[g] = bi;
+    b[A.dofs[(int64_t)e * n + entity_first<P>(la) + i]].y += omega_mu * v;
   }
 }
 
 template <int P>
-__global__ void k_receivers(int64_t npts, const double* __restrict__ pts,
-                            const int32_t* __restrict__ elem, const double* __restrict__ coords,
-                            const int32_t* __restrict__ en, const int32_t* __restrict__ ee,
-                            const int32_t* __restrict__ edn, const int32_t* __restrict__ fe,
-                            const int32_t* __restrict__ dofs, const double2* __restrict__ x,
-                            double omega_mu, double2* __restrict__ out) {
-  constexpr int n = P * (P + 2) * (P + 3) / 2;
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= npts) return;
-  const int64_t E = elem[q];
-  double2* o = out + 6 * q;
-  if (E < 0) {
-    for (int k = 0; k < 6; ++k) o[k] = make_double2(0.0, 0.0);
-    return;
-  }
-  V3 N[n], Cu[n];
-  physical_basis<P>(coords + 12 * E, en + 4 * E, ee + 6 * E, edn + 12 * E, fe + 12 * E,
-                    pts + 3 * q, N, Cu);
-  double2 f[6];
-  for (int k = 0; k < 6; ++k) f[k] = make_double2(0.0, 0.0);
-  for (int i = 0; i < n; ++i) {
-    const double2 xi = x[dofs[E * n + i]];
-    const double nv[3] = {N[i].x, N[i].y, N[i].z};
-    const double cv[3] = {Cu[i].x, Cu[i].y, Cu[i].z};
-    for (int k = 0; k < 3; ++k) {
-      f[k].x += xi.x * nv[k];
-      f[k].y += xi.y * nv[k];
-      f[3 + k].x += xi.x * cv[k];
-      f[3 + k].y += xi.y * cv[k];
+__global__ void __launch_bounds__(256) k_receivers(int64_t npts, const double* __restrict__ pts,
+                                                   const int32_t* __restrict__ elem, ElemArrays A,
+                                                   const double2* __restrict__ x, double omega_mu,
+                                                   double2* __restrict__ out) {
+  constexpr int n = P * (P + 2) * (P + 3) / 2, MAXD = P == 1 ? 1 : P * (P - 1);
+  constexpr int NL = asm_nloc<P>(), Q = 256 / NL;  // receivers of a workgroup
+  __shared__ double2 part[Q][NL][6];
+  const int t = threadIdx.x, ql = t / NL, la = t % NL;
+  const int64_t q0 = (int64_t)blockIdx.x * Q, q = q0 + ql;
+  if (ql < Q && q < npts) {
+    const int64_t e = elem[q];
+    double2 f[6];
+    for (int k = 0; k < 6; ++k) f[k] = make_double2(0.0, 0.0);
+    if (e >= 0) {
+      V3 N[MAXD], Cu[MAXD];
+      const int nd = physical_entity<P>(A, e, la, pts + 3 * q, N, Cu);
+      for (int i = 0; i < nd; ++i) {
+        const double2 xi = x[A.dofs[e * n + entity_first<P>(la) + i]];
+        const double nv[3] = {N[i].x, N[i].y, N[i].z};
+        const double cv[3] = {Cu[i].x, Cu[i].y, Cu[i].z};
+        for (int k = 0; k < 3; ++k) {
+          f[k].x += xi.x * nv[k];
+          f[k].y += xi.y * nv[k];
+          f[3 + k].x += xi.x * cv[k];
+          f[3 + k].y += xi.y * cv[k];
+        }
+      }
     }
+    for (int k = 0; k < 6; ++k) part[ql][la][k] = f[k];
   }
-  // H = curl E / (i omega mu0): (a + ib) / (i w) = (b - i a) / w
-  for (int k = 0; k < 3; ++k) {
-    o[k] = f[k];
-    o[3 + k] = make_double2(f[3 + k].y / omega_mu, -f[3 + k].x / omega_mu);
+  __syncthreads();
+  if (t < Q * 6 && q0 + t / 6 < npts) {
+    const int k = t % 6;
+    double2 f = make_double2(0.0, 0.0);
+    for (int l = 0; l < NL; ++l) f = zadd(f, part[t / 6][l][k]);
+    // H = curl E / (i omega mu0): (a + ib) / (i w) = (b - i a) / w; zero (not -0)
+    // without an element
+    if (k >= 3)
+      f = elem[q0 + t / 6] >= 0 ? make_double2(f.y / omega_mu, -f.x / omega_mu)
+                                : make_double2(0.0, 0.0);
+    out[6 * q0 + t] = f;
   }
 }
 
+// -------------------------------------------------------------------------
+// Adjoint source: f[dofs_e(r)] += sum_c coef[r][c] * N_c(x_r) for every located
+// receiver r, each DOF's contributions in receiver order.  One workgroup takes Q
+// receivers at a time, a thread per receiver and local entity: the products go to
+// LDS, the DOFs they belong to into a hash table there (in any order: only the
+// place of a DOF depends on it), the table is filled from f, the receivers' products
+// are added to it one receiver after another, and it is stored.  (A single thread
+// taking one receiver after another needed 510 us for 101 receivers at p = 2; this
+// takes @@ us.)
+// -------------------------------------------------------------------------
+constexpr int kAdjThreads = 512, kAdjValues = 1024, kAdjTable = 2048;
 
-// -------------------------------------------------------------------------
-// adjoint: receiver adjoint source and per-element gradient contraction
-// -------------------------------------------------------------------------
-// f[dofs_e(r)] += sum_c coef[r][c] * N_c(x_r) for every located receiver r,
-// accumulated by one thread in receiver order (deterministic).
 template <int P>
-__global__ void k_adjoint_rhs(int64_t npts, const double* __restrict__ pts,
-                              const int32_t* __restrict__ elem, const double* __restrict__ coords,
-                              const int32_t* __restrict__ en, const int32_t* __restrict__ ee,
-                              const int32_t* __restrict__ edn, const int32_t* __restrict__ fe,
-                              const int32_t* __restrict__ dofs, const double2* __restrict__ coef,
-                              double2* __restrict__ f) {
-  constexpr int n = P * (P + 2) * (P + 3) / 2;
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  for (int64_t q = 0; q < npts; ++q) {
-    const int64_t E = elem[q];
-    if (E < 0) continue;
-    V3 N[n], Cu[n];
-    physical_basis<P>(coords + 12 * E, en + 4 * E, ee + 6 * E, edn + 12 * E, fe + 12 * E,
-                      pts + 3 * q, N, Cu);
-    const double2 c0 = coef[3 * q], c1 = coef[3 * q + 1], c2 = coef[3 * q + 2];
-    for (int i = 0; i < n; ++i) {
-      const int g = dofs[E * n + i];
-      double2 v = f[g];
-      v.x += c0.x * N[i].x + c1.x * N[i].y + c2.x * N[i].z;
-      v.y += c0.y * N[i].x + c1.y * N[i].y + c2.y * N[i].z;
-      f[g] = v;
+__global__ void __launch_bounds__(kAdjThreads) k_adjoint_rhs(int64_t npts,
+                                                             const double* __restrict__ pts,
+                                                             const int32_t* __restrict__ elem,
+                                                             ElemArrays A,
+                                                             const double2* __restrict__ coef,
+                                                             double2* __restrict__ f) {
+  constexpr int n = P * (P + 2) * (P + 3) / 2, MAXD = P == 1 ? 1 : P * (P - 1);
+  constexpr int NL = asm_nloc<P>();
+  constexpr int QT = kAdjThreads / NL, QV = kAdjValues / n, Q = QT < QV ? QT : QV;
+  static_assert(2 * kAdjValues <= kAdjTable && n <= 64, "table at most half full");
+  __shared__ int32_t key[kAdjTable];
+  __shared__ double2 sum[kAdjTable];
+  __shared__ double2 val[kAdjValues];
+  __shared__ int16_t place[kAdjValues];
+  const int t = threadIdx.x, ql = t / NL, la = t % NL;
+  for (int64_t q0 = 0; q0 < npts; q0 += Q) {
+    for (int i = t; i < kAdjTable; i += kAdjThreads) key[i] = -1;
+    __syncthreads();
+    const int64_t q = q0 + ql;
+    if (ql < Q && q < npts) {
+      const int64_t e = elem[q];
+      V3 N[MAXD], Cu[MAXD];
+      const double2 c0 = coef[3 * q], c1 = coef[3 * q + 1], c2 = coef[3 * q + 2];
+      const int o = ql * n + entity_first<P>(la);
+      if (e >= 0) {
+        const int nd = physical_entity<P>(A, e, la, pts + 3 * q, N, Cu);
+        for (int i = 0; i < nd; ++i) {
+          val[o + i] = make_double2(c0.x * N[i].x + c1.x * N[i].y + c2.x * N[i].z,
+                                    c0.y * N[i].x + c1.y * N[i].y + c2.y * N[i].z);
+          const int g = A.dofs[e * n + entity_first<P>(la) + i];
+          int h = (int)(((uint32_t)g * 2654435761u) >> 21);  // 11 bits
+          while (true) {  // the table is at most half full: an empty place is met
+            const int old = atomicCAS(&key[h], -1, g);
+            if (old == -1 || old == g) break;
+            h = (h + 1) % kAdjTable;
+          }
+          place[o + i] = (int16_t)h;
+        }
+      } else {
+        for (int i = 0; i < local_entity_ndof<P>(la); ++i) place[o + i] = -1;
+      }
     }
+    __syncthreads();
+    for (int i = t; i < kAdjTable; i += kAdjThreads)
+      if (key[i] >= 0) sum[i] = f[key[i]];
+    __syncthreads();
+    const int nq = (int)(npts - q0 < Q ? npts - q0 : Q);
+    if (t < 64)  // one wave: LDS operations in order, an element's DOFs are distinct
+      for (int k = 0; k < nq; ++k) {
+        if (t < n && place[k * n + t] >= 0) {
+          const double2 v = val[k * n + t];
+          double2* s = sum + place[k * n + t];
+          *s = make_double2(s->x + v.x, s->y + v.y);
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+    __syncthreads();
+    for (int i = t; i < kAdjTable; i += kAdjThreads)
+      if (key[i] >= 0) f[key[i]] = sum[i];
+    __syncthreads();
   }
 }
 
@@ -1026,11 +1143,12 @@ int pg_locate_points(int64_t E, const double* coords, int64_t npts, const double
                      int32_t* out, void* stream) {
   if (E <= 0 || npts <= 0 || !coords || !pts || !out) PG_FAIL(PG_ERR_ARG, "bad arguments");
   hipStream_t s = as_stream(stream);
-  hipLaunchKernelGGL(k_fill_i32, dim3(nblocks(npts, 256)), dim3(256), 0, s, npts, out,
-                     (int32_t)0x7fffffff);
-  hipLaunchKernelGGL(k_locate, dim3(nblocks(E, 256)), dim3(256), 0, s, E, coords, npts, pts, tol,
-                     out);
-  hipLaunchKernelGGL(k_notfound, dim3(nblocks(npts, 256)), dim3(256), 0, s, npts, out);
+  hipLaunchKernelGGL(k_fill_i32, dim3(nblocks(npts, 256)), dim3(256), 0, s, npts, out, -1);
+  // few elements: slices of at least eight points, up to half a million threads (at
+  // 29 478 elements and 101 points 20 us with one slice, 7 us with twelve)
+  const int64_t slices = std::max<int64_t>(1, std::min((1 << 19) / E, npts / 8));
+  hipLaunchKernelGGL(k_locate, dim3(nblocks(E, 256), (unsigned)slices), dim3(256), 0, s, E, coords,
+                     npts, pts, tol, out);
   PG_CHECK_LAUNCH();
   return PG_OK;
 }
@@ -1046,10 +1164,11 @@ int pg_source_vector(int p, int32_t e, const double* coords, const int32_t* en, 
   const double om = omega * kMu0;
   hipStream_t s = as_stream(stream);
   double2* bb = reinterpret_cast<double2*>(b);
+  const ElemArrays A{coords, en, ee, edn, fe, dofs};
   switch (p) {
-    case 1: hipLaunchKernelGGL(k_source<1>, dim3(1), dim3(64), 0, s, e, coords, en, ee, edn, fe, dofs, pos, moment, om, bb); break;
-    case 2: hipLaunchKernelGGL(k_source<2>, dim3(1), dim3(64), 0, s, e, coords, en, ee, edn, fe, dofs, pos, moment, om, bb); break;
-    case 3: hipLaunchKernelGGL(k_source<3>, dim3(1), dim3(64), 0, s, e, coords, en, ee, edn, fe, dofs, pos, moment, om, bb); break;
+    case 1: hipLaunchKernelGGL(k_source<1>, dim3(1), dim3(64), 0, s, e, A, pos, moment, om, bb); break;
+    case 2: hipLaunchKernelGGL(k_source<2>, dim3(1), dim3(64), 0, s, e, A, pos, moment, om, bb); break;
+    case 3: hipLaunchKernelGGL(k_source<3>, dim3(1), dim3(64), 0, s, e, A, pos, moment, om, bb); break;
   }
   PG_CHECK_LAUNCH();
   return PG_OK;
@@ -1065,13 +1184,15 @@ int pg_receiver_fields(int p, int64_t npts, const double* pts, const int32_t* el
     PG_FAIL(PG_ERR_ARG, "bad arguments");
   const double om = omega * kMu0;
   hipStream_t s = as_stream(stream);
-  const dim3 g(nblocks(npts, 64)), b(64);
+  const int nl = p == 1 ? 6 : (p == 2 ? 10 : 11);  // threads per receiver
+  const dim3 g(nblocks(npts, 256 / nl)), b(256);
+  const ElemArrays A{coords, en, ee, edn, fe, dofs};
   const double2* xx = reinterpret_cast<const double2*>(x);
   double2* f = reinterpret_cast<double2*>(fields);
   switch (p) {
-    case 1: hipLaunchKernelGGL(k_receivers<1>, g, b, 0, s, npts, pts, elem, coords, en, ee, edn, fe, dofs, xx, om, f); break;
-    case 2: hipLaunchKernelGGL(k_receivers<2>, g, b, 0, s, npts, pts, elem, coords, en, ee, edn, fe, dofs, xx, om, f); break;
-    case 3: hipLaunchKernelGGL(k_receivers<3>, g, b, 0, s, npts, pts, elem, coords, en, ee, edn, fe, dofs, xx, om, f); break;
+    case 1: hipLaunchKernelGGL(k_receivers<1>, g, b, 0, s, npts, pts, elem, A, xx, om, f); break;
+    case 2: hipLaunchKernelGGL(k_receivers<2>, g, b, 0, s, npts, pts, elem, A, xx, om, f); break;
+    case 3: hipLaunchKernelGGL(k_receivers<3>, g, b, 0, s, npts, pts, elem, A, xx, om, f); break;
   }
   PG_CHECK_LAUNCH();
   return PG_OK;
@@ -1087,10 +1208,11 @@ int pg_adjoint_rhs(int p, int64_t npts, const double* pts, const int32_t* elem,
   hipStream_t s = as_stream(stream);
   const double2* c = reinterpret_cast<const double2*>(coef);
   double2* ff = reinterpret_cast<double2*>(f);
+  const ElemArrays A{coords, en, ee, edn, fe, dofs};
   switch (p) {
-    case 1: hipLaunchKernelGGL(k_adjoint_rhs<1>, dim3(1), dim3(64), 0, s, npts, pts, elem, coords, en, ee, edn, fe, dofs, c, ff); break;
-    case 2: hipLaunchKernelGGL(k_adjoint_rhs<2>, dim3(1), dim3(64), 0, s, npts, pts, elem, coords, en, ee, edn, fe, dofs, c, ff); break;
-    case 3: hipLaunchKernelGGL(k_adjoint_rhs<3>, dim3(1), dim3(64), 0, s, npts, pts, elem, coords, en, ee, edn, fe, dofs, c, ff); break;
+    case 1: hipLaunchKernelGGL(k_adjoint_rhs<1>, dim3(1), dim3(kAdjThreads), 0, s, npts, pts, elem, A, c, ff); break;
+    case 2: hipLaunchKernelGGL(k_adjoint_rhs<2>, dim3(1), dim3(kAdjThreads), 0, s, npts, pts, elem, A, c, ff); break;
+    case 3: hipLaunchKernelGGL(k_adjoint_rhs<3>, dim3(1), dim3(kAdjThreads), 0, s, npts, pts, elem, A, c, ff); break;
   }
   PG_CHECK_LAUNCH();
   return PG_OK;
