@@ -102,17 +102,17 @@ int pg_plan_destroy(void *plan);
 /* First pair of every entity: the pairs (A, B) of entity A are
  * [entity_pair[A], entity_pair[A+1]) (n_entities + 1 values, host array), and
  * (max_rowlen, nullable) the longest row of an entity with DOFs.
- * PG_ERR_UNSUPPORTED when an entity's rows exceed the bounds of the row-major
- * numeric assembly (192 columns, 96 coupled entities, 24 elements); leave
+ * PG_ERR_UNSUPPORTED when an entity exceeds the bounds of this export (192
+ * columns, 96 coupled entities, 24 elements); leave
  * pg_plan_dev.entity_pair NULL then.  Part of the plan export above
  * (createParallelMatrix preallocation, petgem/parallel.py:150-177). */
 int pg_plan_entity_pairs(const void *plan, int32_t *entity_pair, int32_t *max_rowlen);
 
 /* Device view of an exported plan (all device pointers).  entity_pair
  * (nullable, from pg_plan_entity_pairs, with entity_row_max its max_rowlen)
- * selects the row-major numeric assembly (p = 1-3): one workgroup per entity
- * sums its CSR rows in LDS and writes them contiguously; without it the
- * two-phase (p <= 2) or one-pass (p = 3) kernels run (same values, bitwise). */
+ * saves the numeric assembly a search for its entities' first pairs (small p = 3
+ * systems: selects the form that sums an entity's rows in LDS).  Same values,
+ * bitwise. */
 typedef struct pg_plan_dev {
   int32_t p;
   int64_t n_edges, n_faces, n_elems;
@@ -126,8 +126,8 @@ typedef struct pg_plan_dev {
 
 /* Numeric assembly, atomic-free: CSR values (nnz complex128) of
  * A = sum_e (K_e - i*omega*mu0*M_e), each slot summed over its contributing
- * elements in ascending element order, element matrices recomputed from the
- * tables (never stored).  entity_bc (nullable, one byte per entity) folds the
+ * elements in ascending element order, element matrices recomputed (never
+ * stored).  entity_bc (nullable, one byte per entity) folds the
  * PEC condition in (zero rows/columns, unit diagonal).  Replaces the element
  * loop and assembly of Solver.assembly (petgem/solver.py:191-235). */
 int pg_assemble(const void *tables, const pg_plan_dev *plan, const void *workspace,

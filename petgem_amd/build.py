@@ -13,7 +13,8 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libpetgem_amd.so")
 SOURCES = ["pg_api.cpp", "pg_plan.cpp", "pg_element.hip", "pg_krylov.hip", "pg_batch.hip",
-           "pg_multi.hip", "pg_elemop.hip", "pg_adjoint.hip"]
+           "pg_multi.hip", "pg_elemop.hip", "pg_adjoint.hip",
+           "pg_rows.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["-O3", "-fPIC", "-std=c++17", "--offload-arch=gfx950",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -23,7 +24,7 @@ FLAGS = ["-O3", "-fPIC", "-std=c++17", "--offload-arch=gfx950",
 # per-source flags: the factored element products unroll loops over constant
 # tables, past the default size limit of a fully unrolled loop
 UNROLL = ["-mllvm", "-pragma-unroll-threshold=2000000"]
-EXTRA = {"pg_elemop.hip": UNROLL, "pg_adjoint.hip": UNROLL}
+EXTRA = {"pg_elemop.hip": UNROLL, "pg_adjoint.hip": UNROLL, "pg_rows.hip": UNROLL}
 
 
 def _stale(obj, src):

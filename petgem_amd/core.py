@@ -136,7 +136,7 @@ class DeviceMesh:
 
 
 class Tables:
-    """Device-resident reference-element tables for order p."""
+    """Handle of the element operators of order p."""
 
     def __init__(self, p):
         L = nat.lib()
@@ -178,8 +178,8 @@ class Plan:
             nat.check(L.pg_plan_export(h, nat.ptr(rowptr), nat.ptr(cols), nat.ptr(slot0),
                                        nat.ptr(rowlen), nat.ptr(cbeg), nat.ptr(ab),
                                        nat.ptr(contrib)))
-            # first pair per entity, when every entity fits the row-major
-            # numeric assembly (else the two-phase kernels run)
+            # first pair per entity, when every entity is within the export's
+            # bounds (else the assembly does without)
             epair = np.empty(self.n_entities + 1, dtype=np.int32)
             row_max = ctypes.c_int32(0)
             rc = L.pg_plan_entity_pairs(h, nat.ptr(epair), ctypes.byref(row_max))

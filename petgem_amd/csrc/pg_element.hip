@@ -8,8 +8,8 @@
 //     M_ij = det J * sum_{a<=b} G'_ab T^M_ab[v_i][v_j]
 //     K_ij =         sum_{a<=b} H'_ab T^K_ab[v_i][v_j]
 // where v_i is the orientation "variant" of local DOF i and T are quadrature
-// contractions of the reference basis computed once per order (tables.cpp
-// part below).  This equals the per-quadrature-point loop of
+// contractions of the reference basis (build_table below, on the host; the
+// kernels of pg_rows.hip form the same products without tables).  This equals the per-quadrature-point loop of
 // computeElementalMatrices (petgem/hvfem.py:258-314) up to summation order.
 #include <hip/hip_runtime.h>
 
@@ -22,6 +22,7 @@
 #include "pg_basis.h"
 #include "pg_common.h"
 #include "pg_rowasm.h"
+#include "pg_rows.h"
 
 namespace pg {
 
@@ -78,10 +79,10 @@ static void build_table(int p, std::vector<double>& T) {
 
 struct Tables {
   int p;
-  int V;
-  int device;
-  double* d_T;
+  double* d_T;  // p = 3 only (the other orders' kernels form their products without)
 };
+// p = 3: elements from which on the factored kernels are the faster
+constexpr int64_t kFactoredElements = 4096;
 
 // -------------------------------------------------------------------------
 // geometry + orientation (one thread per element)
@@ -191,8 +192,28 @@ __global__ void k_orientation(int64_t E, const int32_t* __restrict__ en,
   for (int i = 0; i < 4; ++i) fo_out[4 * e + i] = fo[i];
 }
 
+// local entities carrying DOFs, and their DOFs
+template <int P>
+constexpr int asm_nloc() {
+  return P == 1 ? 6 : (P == 2 ? 10 : 11);
+}
+template <int P>
+__device__ inline int local_entity_ndof(int la) {
+  return la < 6 ? P : (la < 10 ? P * (P - 1) : P * (P - 1) * (P - 2) / 2);
+}
+
 // -------------------------------------------------------------------------
-// element matrices (one thread per (element, i, j))
+// Element matrices and assembly from the tables: p = 3 below kFactoredElements
+// elements (above, and at p <= 2: pg_rows.hip).  An entry is 12 multiplications on a
+// gathered table row and independent of the others, so these are bound by the gathers
+// on a full chip, but short on an empty one, where a factored row of p = 3 (some 3000
+// operations one after another, for K_e and then for M_e) is the time of the call:
+// assembly of 384 elements 15.6 us (factored 26.6), 1296 32 (46), 4374 93 (92),
+// 10 368 261 (246), 20 250 476 (426); the matrices of 384 elements 10 us (17), of 4374
+// 77 (58).  Both or neither: the assembled values are the ordered sums of the element
+// matrices bit for bit.
+//
+// Element matrices: one thread per (element, i, j).
 // -------------------------------------------------------------------------
 template <int P>
 __device__ inline void dof_entity(int i, int& la, int& k) {
@@ -226,7 +247,7 @@ __device__ inline void contract(const double* __restrict__ t, const double* __re
 }
 
 template <int P>
-__global__ void k_element_matrices(int64_t E, const double* __restrict__ T,
+__global__ void k_table_matrices(int64_t E, const double* __restrict__ T,
                                    const double* __restrict__ coef,
                                    const int32_t* __restrict__ orient, double* __restrict__ M,
                                    double* __restrict__ K) {
@@ -260,15 +281,12 @@ __device__ inline int entity_ndof_global(int64_t g, int64_t nE, int64_t nF) {
 }
 
 // -------------------------------------------------------------------------
-// One-pass assembly (p = 3 plans beyond the row-major bounds): one thread per
-// (entity pair, block row)
-// that loops over the pair's contributors in ascending element order, contracting
-// each entry from the tables and the element's coefficients.  At p = 3 the
-// two-phase form below would pad every local block to 6 x 6 (a 5.8 GB scratch
-// at C3) and loses to this form.
+// Assembly of plans beyond the bounds of pg_rowasm.h: one thread per (entity pair, block
+// row) that loops over the pair's contributors in ascending element order, contracting
+// each entry from the tables and the element's coefficients.
 // -------------------------------------------------------------------------
 template <int P>
-__global__ void __launch_bounds__(256) k_assemble(
+__global__ void __launch_bounds__(256) k_table_pairs(
     int64_t npairs, int64_t nE, int64_t nF, const double* __restrict__ T,
     const int32_t* __restrict__ pair_slot0, const int32_t* __restrict__ pair_rowlen,
     const int32_t* __restrict__ pair_cbeg, const int32_t* __restrict__ pair_ab,
@@ -332,166 +350,18 @@ __global__ void __launch_bounds__(256) k_assemble(
 }
 
 // -------------------------------------------------------------------------
-// Two-phase assembly (p = 1, 2), atomic-free, every CSR slot the sum of its
-// contributors in the plan's ascending element order (the order of the
-// reference's single-rank ADD_VALUES), bitwise the one-pass kernel's result:
-//  k_asm_blocks  one thread per (local entity la, local entity lb, element):
-//                the lanes of a wave take consecutive elements at the same
-//                local pair, so their coefficient loads are contiguous and
-//                their table rows repeat with the few orientation patterns of
-//                neighbouring elements (cache hits instead of a gather per
-//                lane), and the nloc^2 workgroups of one block of elements run
-//                one after another (its coefficients read once from L2); each
-//                writes its d(la) x d(lb)
-//                block of (K_e, -omega mu0 M_e) entries (or (K_e, M_e)):
-//                blk[t][k][l], t = (la nloc + lb) E + e, MAXD x MAXD per t;
-//  k_asm_sums    one thread per (entity pair, row k of its block): sums its
-//                contributors' rows k of those blocks in the plan's ascending
-//                element order and stores the pair block's row.
-// Traffic: the blocks are written and read once (2.46 GB at C2) besides the
-// CSR values, but every load is either a broadcast (an element's coefficients)
-// or contiguous, where one thread per slot row gathering coefficients and
-// table rows per contributor was bound by divergent gathers.
-// -------------------------------------------------------------------------
-// streaming (non-temporal) stores of the block scratch: written once, read
-// once by the sums, so it should not evict the tables and coefficients from L2
-typedef double asm_d2 __attribute__((ext_vector_type(2)));
-__device__ inline void nt_store(double2* p, double2 v) {
-  __builtin_nontemporal_store(asm_d2{v.x, v.y}, reinterpret_cast<asm_d2*>(p));
-}
-
-template <int P>
-constexpr int asm_nloc() {
-  return P == 1 ? 6 : (P == 2 ? 10 : 11);
-}
-template <int P>
-constexpr int asm_maxd() {
-  return P == 1 ? 1 : P * (P - 1);
-}
-template <int P>
-__device__ inline int local_entity_ndof(int la) {
-  return la < 6 ? P : (la < 10 ? P * (P - 1) : P * (P - 1) * (P - 2) / 2);
-}
-
-template <int P>
-__global__ void __launch_bounds__(256) k_asm_blocks(int64_t E, const double* __restrict__ T,
-                                                    const double* __restrict__ coef,
-                                                    const int32_t* __restrict__ orient,
-                                                    double omega_mu, int km,
-                                                    double2* __restrict__ blk) {
-  constexpr int NL = asm_nloc<P>(), MAXD = asm_maxd<P>();
-  constexpr int V = 12 * P + 24 * P * (P - 1) + P * (P - 1) * (P - 2) / 2;
-  // p = 2: the workgroup's blocks (4 values each) are staged in LDS and written
-  // as one contiguous run, instead of four stores 64 bytes apart per lane
-  constexpr bool kStage = P == 2;
-  __shared__ double2 stage[kStage ? 256 * MAXD * MAXD : 1];
-  // workgroup b: local pair ll = b mod nloc^2 of the element block b / nloc^2,
-  // so that the nloc^2 workgroups of one block of 256 elements run together
-  // and read its coefficients from L2 (the pair as the slow index re-read all
-  // coefficients once per pair)
-  const int ll = (int)(blockIdx.x % (NL * NL)), la = ll / NL, lb = ll % NL;
-  const int64_t e0 = (int64_t)(blockIdx.x / (NL * NL)) * blockDim.x, e = e0 + threadIdx.x;
-  const int64_t t = (int64_t)ll * E + e;
-  if (!kStage && e >= E) return;
-  if (e < E) {
-    const int dA = local_entity_ndof<P>(la), dB = local_entity_ndof<P>(lb);
-    const int pk = orient[e];
-    const double* cf = coef + 12 * e;
-    const int va0 = entity_variant_base(la, orient_of(pk, la), P);
-    const int vb = entity_variant_base(lb, orient_of(pk, lb), P);
-    double2* out = kStage ? stage + threadIdx.x * (MAXD * MAXD) : blk + t * (MAXD * MAXD);
-    for (int k = 0; k < dA; ++k) {
-      const double* trow = T + ((size_t)(va0 + k) * V + vb) * 12;
-#pragma unroll
-      for (int l = 0; l < MAXD; ++l)
-        if (l < dB) {
-          double m, kk;
-          contract(trow + 12 * l, cf, &m, &kk);
-          // separately rounded product, as the reference forms i*w*mu0*M_e before adding
-          const double2 v = make_double2(kk, km ? m : -__dmul_rn(omega_mu, m));
-          if constexpr (kStage) out[k * MAXD + l] = v;
-          else nt_store(out + k * MAXD + l, v);
-        }
-    }
-  }
-  if constexpr (kStage) {
-    __syncthreads();
-    const int64_t t0 = (int64_t)ll * E + e0;
-    const int64_t n = (E - e0 < (int64_t)blockDim.x ? E - e0 : (int64_t)blockDim.x) *
-                      (MAXD * MAXD);
-    for (int i = threadIdx.x; i < n; i += blockDim.x) nt_store(blk + t0 * (MAXD * MAXD) + i, stage[i]);
-  }
-}
-
-template <int P>
-__global__ void __launch_bounds__(256) k_asm_sums(
-    int64_t npairs, int64_t nE, int64_t nF, int64_t E, const int32_t* __restrict__ pair_slot0,
-    const int32_t* __restrict__ pair_rowlen, const int32_t* __restrict__ pair_cbeg,
-    const int32_t* __restrict__ pair_ab, const uint32_t* __restrict__ contrib,
-    const double2* __restrict__ blk, const uint8_t* __restrict__ ent_bc,
-    double2* __restrict__ values, double* __restrict__ Kout, double* __restrict__ Mout) {
-  constexpr int NL = asm_nloc<P>(), MAXD = asm_maxd<P>();
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t pair = t / MAXD;
-  const int k = (int)(t - pair * MAXD);
-  if (pair >= npairs) return;
-  const int64_t A = pair_ab[2 * pair], B = pair_ab[2 * pair + 1];
-  const int dA = entity_ndof_global<P>(A, nE, nF);
-  const int dB = entity_ndof_global<P>(B, nE, nF);
-  if (k >= dA) return;
-  double re[MAXD], im[MAXD];
-#pragma unroll
-  for (int l = 0; l < MAXD; ++l) re[l] = im[l] = 0.0;
-  const int c0 = pair_cbeg[pair], c1 = pair_cbeg[pair + 1];
-  for (int c = c0; c < c1; ++c) {
-    const uint32_t u = contrib[c];
-    const int64_t e = u >> 8;
-    const int la = (u >> 4) & 15, lb = u & 15;
-    const double2* row = blk + ((int64_t)(la * NL + lb) * E + e) * (MAXD * MAXD) + k * MAXD;
-#pragma unroll
-    for (int l = 0; l < MAXD; ++l)
-      if (l < dB) {
-        const double2 v = row[l];
-        re[l] += v.x;
-        im[l] += v.y;
-      }
-  }
-  if (ent_bc != nullptr && (ent_bc[A] | ent_bc[B])) {
-#pragma unroll
-    for (int l = 0; l < MAXD; ++l) {
-      re[l] = (A == B && k == l && ent_bc[A]) ? 1.0 : 0.0;
-      im[l] = 0.0;
-    }
-  }
-  const int64_t s0 = (int64_t)pair_slot0[pair] + (int64_t)k * pair_rowlen[pair];
-  if (Kout) {
-#pragma unroll
-    for (int l = 0; l < MAXD; ++l)
-      if (l < dB) {
-        Kout[s0 + l] = re[l];
-        Mout[s0 + l] = im[l];
-      }
-  } else {
-#pragma unroll
-    for (int l = 0; l < MAXD; ++l)
-      if (l < dB) values[s0 + l] = make_double2(re[l], im[l]);
-  }
-}
-
-// -------------------------------------------------------------------------
-// Row-major assembly (p = 1-3; plans within the bounds of pg_rowasm.h): one
-// single-wave workgroup per entity A with DOFs keeps A's d(A) CSR rows in LDS
+// Assembly of plans within the bounds of pg_rowasm.h: one single-wave workgroup per entity A with DOFs keeps A's d(A) CSR rows in LDS
 // and walks the elements containing A in ascending order (the contributors of
 // the diagonal pair (A, A)).  For each element its lanes form the entries of
 // the element's block row la(A) -- row k < d(A), every local DOF j -- from the
 // tables and the element's coefficients (one element per step: wave-uniform
 // loads) and add each into the LDS row at the column of entity(e, lb).  Every
 // slot is thus the sum of its contributors in ascending element order, bitwise
-// the two-phase result, with no block scratch; A's rows then leave as one
-// contiguous run of d(A) * rowlen values.
+// the result of k_table_pairs; A's rows then leave as one contiguous run of
+// d(A) * rowlen values.
 // -------------------------------------------------------------------------
-template <int P, int LEN>
-__global__ void __launch_bounds__(64) k_asm_rows(
+template <int P>
+__global__ void __launch_bounds__(64) k_table_rows(
     int64_t nE, int64_t nF, const int32_t* __restrict__ epair, const double* __restrict__ T,
     const int32_t* __restrict__ rowptr, const int32_t* __restrict__ pair_slot0,
     const int32_t* __restrict__ pair_cbeg, const int32_t* __restrict__ pair_ab,
@@ -499,7 +369,7 @@ __global__ void __launch_bounds__(64) k_asm_rows(
     const int32_t* __restrict__ orient, double omega_mu, int km,
     const uint8_t* __restrict__ ent_bc, double2* __restrict__ values, double* __restrict__ Kout,
     double* __restrict__ Mout) {
-  constexpr int NL = asm_nloc<P>(), MAXD = asm_maxd<P>();
+  constexpr int NL = asm_nloc<P>(), MAXD = P == 1 ? 1 : P * (P - 1), LEN = kRowAsmMaxLen;
   constexpr int DE = P, DF = P * (P - 1), DV = P * (P - 1) * (P - 2) / 2;
   constexpr int NLD = 6 * DE + 4 * DF + DV;
   constexpr int V = 12 * P + 24 * P * (P - 1) + P * (P - 1) * (P - 2) / 2;
@@ -963,23 +833,22 @@ int pg_tables_host(int p, double* out, int64_t out_len) {
 int pg_tables_create(int p, void** tables) {
   if (!tables) PG_FAIL(PG_ERR_ARG, "tables is NULL");
   if (p < 1 || p > kMaxP) PG_FAIL(PG_ERR_UNSUPPORTED, "order p=%d not supported (1..3)", p);
-  std::vector<double> T;
-  build_table(p, T);
+  int device;
+  PG_HIP(hipGetDevice(&device));
+  double* d_T = nullptr;
+  if (p == 3) {
+    std::vector<double> T;
+    build_table(p, T);
+    PG_HIP(hipMalloc(&d_T, T.size() * sizeof(double)));
+    const hipError_t err = hipMemcpy(d_T, T.data(), T.size() * sizeof(double), hipMemcpyHostToDevice);
+    if (err != hipSuccess) {
+      (void)hipFree(d_T);
+      PG_FAIL(PG_ERR_HIP, "hipMemcpy(tables): %s", hipGetErrorString(err));
+    }
+  }
   Tables* t = new Tables();
   t->p = p;
-  t->V = n_variants(p);
-  hipError_t err = hipGetDevice(&t->device);
-  if (err == hipSuccess) err = hipMalloc(&t->d_T, T.size() * sizeof(double));
-  if (err != hipSuccess) {
-    delete t;
-    PG_FAIL(PG_ERR_HIP, "hipMalloc(tables): %s", hipGetErrorString(err));
-  }
-  err = hipMemcpy(t->d_T, T.data(), T.size() * sizeof(double), hipMemcpyHostToDevice);
-  if (err != hipSuccess) {
-    (void)hipFree(t->d_T);
-    delete t;
-    PG_FAIL(PG_ERR_HIP, "hipMemcpy(tables): %s", hipGetErrorString(err));
-  }
+  t->d_T = d_T;
   *tables = t;
   return PG_OK;
 }
@@ -1030,16 +899,12 @@ int pg_element_matrices(const void* tables, int64_t E, const void* ws, double* M
                         void* stream) {
   if (!tables || !ws || !M || !K || E <= 0) PG_FAIL(PG_ERR_ARG, "bad arguments");
   const Tables* t = static_cast<const Tables*>(tables);
-  const int n = ndof_element(t->p);
-  const int64_t total = E * n * n;
   void* w = const_cast<void*>(ws);
-  const dim3 g(nblocks(total, 256)), b(256);
-  hipStream_t s = as_stream(stream);
-  switch (t->p) {
-    case 1: hipLaunchKernelGGL(k_element_matrices<1>, g, b, 0, s, E, t->d_T, ws_coef(w), ws_orient(w, E), M, K); break;
-    case 2: hipLaunchKernelGGL(k_element_matrices<2>, g, b, 0, s, E, t->d_T, ws_coef(w), ws_orient(w, E), M, K); break;
-    case 3: hipLaunchKernelGGL(k_element_matrices<3>, g, b, 0, s, E, t->d_T, ws_coef(w), ws_orient(w, E), M, K); break;
-  }
+  if (t->p == 3 && E < kFactoredElements)
+    hipLaunchKernelGGL(k_table_matrices<3>, dim3(nblocks(E * 45 * 45, 256)), dim3(256), 0,
+                       as_stream(stream), E, t->d_T, ws_coef(w), ws_orient(w, E), M, K);
+  else
+    launch_element_matrices(t->p, E, ws_coef(w), ws_orient(w, E), M, K, as_stream(stream));
   PG_CHECK_LAUNCH();
   return PG_OK;
 }
@@ -1050,70 +915,25 @@ static int assemble_impl(const void* tables, const pg_plan_dev* pl, const void* 
   const Tables* t = static_cast<const Tables*>(tables);
   if (pl->p != t->p) PG_FAIL(PG_ERR_ARG, "plan order %d != tables order %d", pl->p, t->p);
   if (pl->n_elems >= (1LL << 24)) PG_FAIL(PG_ERR_UNSUPPORTED, "more than 2^24 elements");
-  const int maxd = t->p == 1 ? 1 : t->p * (t->p - 1);
-  const int nloc = t->p == 1 ? 6 : (t->p == 2 ? 10 : 11);
-  const int64_t threads = pl->npairs * maxd;
-  const int64_t nblk = pl->n_elems * nloc * nloc;
   void* w = const_cast<void*>(ws);
-  const double om = omega * kMu0;
-  const dim3 g(nblocks(threads, 256)), gb(nblocks(pl->n_elems, 256) * nloc * nloc), b(256);
   hipStream_t s = as_stream(stream);
+  const double* coef = ws_coef(w);
+  const int32_t* orient = ws_orient(w, pl->n_elems);
+  const double om = omega * kMu0;
   double2* v = reinterpret_cast<double2*>(values);
-  if (pl->entity_pair) {
-    const int64_t nent = t->p == 1 ? pl->n_edges
-                                   : pl->n_edges + pl->n_faces + (t->p == 3 ? pl->n_elems : 0);
-    const int km = Kout ? 1 : 0;
-    // the short-row variant when the plan's longest row fits it (more workgroups resident)
-    const bool short_rows = pl->entity_row_max > 0 && pl->entity_row_max <= kRowAsmShortLen;
-#define PG_ROWS(P, LEN)                                                                        \
-  hipLaunchKernelGGL((k_asm_rows<P, LEN>), dim3((unsigned)nent), dim3(64), 0, s, pl->n_edges,   \
-                     pl->n_faces, pl->entity_pair, t->d_T, pl->rowptr, pl->pair_slot0,          \
-                     pl->pair_cbeg, pl->pair_ab, pl->contrib, ws_coef(w),                       \
-                     ws_orient(w, pl->n_elems), om, km, ent_bc, v, Kout, Mout)
-    if (t->p == 1 && short_rows) {
-      PG_ROWS(1, kRowAsmShortLen);
-    } else if (t->p == 1) {
-      PG_ROWS(1, kRowAsmMaxLen);
-    } else if (t->p == 2 && short_rows) {
-      PG_ROWS(2, kRowAsmShortLen);
-    } else if (t->p == 2) {
-      PG_ROWS(2, kRowAsmMaxLen);
-    } else if (short_rows) {
-      PG_ROWS(3, kRowAsmShortLen);
-    } else {
-      PG_ROWS(3, kRowAsmMaxLen);
-    }
-#undef PG_ROWS
-    PG_CHECK_LAUNCH();
-    return PG_OK;
-  }
-  if (t->p == 3) {
-    hipLaunchKernelGGL(k_assemble<3>, g, b, 0, s, pl->npairs, pl->n_edges, pl->n_faces, t->d_T,
-                       pl->pair_slot0, pl->pair_rowlen, pl->pair_cbeg, pl->pair_ab, pl->contrib,
-                       ws_coef(w), ws_orient(w, pl->n_elems), om, ent_bc, v, Kout, Mout);
-    PG_CHECK_LAUNCH();
-    return PG_OK;
-  }
-  // the element blocks: stream-ordered scratch (the pool keeps it between calls)
-  double2* blk = nullptr;
-  PG_HIP(hipMallocAsync(reinterpret_cast<void**>(&blk),
-                        (size_t)nblk * maxd * maxd * sizeof(double2), s));
-  const int km = Kout ? 1 : 0;
-#define PG_ASM(P)                                                                             \
-  hipLaunchKernelGGL(k_asm_blocks<P>, gb, b, 0, s, pl->n_elems, t->d_T, ws_coef(w),             \
-                     ws_orient(w, pl->n_elems), om, km, blk);                                  \
-  hipLaunchKernelGGL(k_asm_sums<P>, g, b, 0, s, pl->npairs, pl->n_edges, pl->n_faces,           \
-                     pl->n_elems,                                                              \
-                     pl->pair_slot0, pl->pair_rowlen, pl->pair_cbeg, pl->pair_ab, pl->contrib, \
-                     blk, ent_bc, v, Kout, Mout)
-  if (t->p == 1) {
-    PG_ASM(1);
-  } else {
-    PG_ASM(2);
-  }
-#undef PG_ASM
+  if (t->p < 3 || pl->n_elems >= kFactoredElements)
+    launch_assembly(*pl, coef, orient, om, ent_bc, v, Kout, Mout, s);
+  else if (pl->entity_pair)
+    hipLaunchKernelGGL(k_table_rows<3>, dim3((unsigned)(pl->n_edges + pl->n_faces + pl->n_elems)),
+                       dim3(64), 0, s, pl->n_edges, pl->n_faces, pl->entity_pair, t->d_T, pl->rowptr,
+                       pl->pair_slot0, pl->pair_cbeg, pl->pair_ab, pl->contrib, coef, orient, om,
+                       Kout ? 1 : 0, ent_bc, v, Kout, Mout);
+  else
+    hipLaunchKernelGGL(k_table_pairs<3>, dim3(nblocks(pl->npairs * 6, 256)), dim3(256), 0, s,
+                       pl->npairs, pl->n_edges, pl->n_faces, t->d_T, pl->pair_slot0, pl->pair_rowlen,
+                       pl->pair_cbeg, pl->pair_ab, pl->contrib, coef, orient, om, ent_bc, v, Kout,
+                       Mout);
   PG_CHECK_LAUNCH();
-  PG_HIP(hipFreeAsync(blk, s));
   return PG_OK;
 }
 
