@@ -117,3 +117,33 @@ def test_adjoint_gradient_on_arbitrary_orientations(p, n, keep, nrhs, rows):
                  nrhs, ctypes.c_int64(T.ndof), nat.ptr(x), nat.ptr(lam), nat.ptr(omega),
                  nat.ptr(g), nat.stream_handle()))
     assert float((g - ref).abs().max()) <= 1e-12 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("sizes", [(8, 3, 9), (16, 17, 4), (40,), (5,) * 1700, (5,) * 6000])
+def test_p3_sums_of_many_elements(sizes):
+    """y = A x at p = 3 over fans of tetrahedra around an edge each: one, two and more
+    steps of eight elements, and both sides of the 131 072 entities up to which a thread
+    sums one DOF (61 200 and 216 000 here).  Same bounds as above."""
+    pts, tets, b = [], [], 0
+    for f, m in enumerate(sizes):
+        a = 2 * np.pi * np.arange(m) / m
+        x = 4.0 * f
+        pts += [np.array([(x, 0.0, -1.0), (x, 0.1, 1.0)]),
+                np.stack([x + np.cos(a), np.sin(a), 0.1 * np.cos(3 * a)], axis=1)]
+        i = np.arange(m)
+        tets.append(np.sort(np.stack([0 * i + b, 0 * i + b + 1, b + 2 + i, b + 2 + (i + 1) % m],
+                                     axis=1), axis=1))
+        b += m + 2
+    T = Topology(np.concatenate(pts), np.concatenate(tets), 3)
+    mesh = core.DeviceMesh.from_topology(T, DEV)
+    asm = core.Assembler(mesh)
+    asm.geometry(np.random.default_rng(1).uniform(0.1, 2.0, (T.n_elems, 2)))
+    om = core.omega_of(1.0)
+    vals = asm.assemble(om)
+    eop = core.ElementOperator(asm, om, None, mesh.entity_order())
+    x = torch.randn((T.ndof, 2), dtype=torch.float64, device=DEV,
+                    generator=torch.Generator(DEV).manual_seed(3))
+    ref = core.spmv(asm.plan, vals, x)
+    for dt, bar in ((torch.float64, 1e-12), (torch.float32, 1e-5)):
+        y = eop.apply(x.to(dt)).double()
+        assert float((y - ref).abs().max()) <= bar * float(ref.abs().max())
