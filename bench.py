@@ -10,8 +10,8 @@ One step = numeric assembly (element geometry + fused atomic-free CSR
 assembly) + point-dipole source + PEC boundary condition + preconditioner
 set-up + Krylov solve to a true relative residual <= 1e-8, with every input
 already resident in HBM.  The Krylov iterations apply A either with a CSR
-SpMV of the assembled matrix or element by element (the element matrices
-recomputed from the tables at every product), whichever the solver's
+SpMV of the assembled matrix or element by element (every element's product
+formed again from its geometry), whichever the solver's
 autotuner measures faster; the true residual always uses the assembled CSR.
 The headline value is the FP64 step time (complex128 throughout, the
 workload as stated); the mixed-precision step (complex64 Krylov iterations
@@ -305,7 +305,7 @@ def c3_leg(args, log):
     """Mixed precision at p = 3: 24^3 Kuhn hexes x 6 = 82,944 tets (p = 3), the
     layered model with the resistive block, HED at (0, 0, -950) m, 1 Hz and
     0.25 Hz.  At each frequency the FP64 solve (COCG + entity-block Jacobi,
-    products on the FP64 matrix cores or the CSR, as the autotuner picks) and
+    products element by element or from the CSR, as the autotuner picks) and
     the mixed solve (complex64 iterations under FP64 refinement) of the same
     system, one warm-up and one timed solve each; receiver fields of the two
     compared."""

@@ -9,8 +9,9 @@
 //     K_ij =         sum_{a<=b} H'_ab T^K_ab[v_i][v_j]
 // where v_i is the orientation "variant" of local DOF i and T are quadrature
 // contractions of the reference basis (build_table below, on the host; the
-// kernels of pg_rows.hip form the same products without tables).  This equals the per-quadrature-point loop of
-// computeElementalMatrices (petgem/hvfem.py:258-314) up to summation order.
+// kernels of pg_rows.hip form the same products without tables).  This equals
+// the per-quadrature-point loop of computeElementalMatrices
+// (petgem/hvfem.py:258-314) up to summation order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

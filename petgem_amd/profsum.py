@@ -25,7 +25,7 @@ from collections import defaultdict
 def short_name(name):
     """`void pg::k_spmv_er<16, 4, 2, 1, HIP_vector_type<float, 2u>, ...>(args)` ->
     `k_spmv_er<16,4,2,1,float2,float2>`."""
-    s = re.sub(r"^void ", "", name.strip())
+    s = re.sub(r"^void ", "", name.strip()).replace("(anonymous namespace)::", "")
     depth, cut = 0, len(s)
     for i, ch in enumerate(s):  # drop the argument list (first '(' outside <>)
         if ch == "<":
