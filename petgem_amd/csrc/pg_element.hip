@@ -210,7 +210,7 @@ __device__ inline int local_entity_ndof(int la) {
 // on a full chip, but short on an empty one, where a factored row of p = 3 (some 3000
 // operations one after another, for K_e and then for M_e) is the time of the call:
 // assembly of 384 elements 15.6 us (factored 26.6), 1296 32 (46), 4374 93 (92),
-// 10 368 261 (246), 20 250 476 (426); the matrices of 384 elements 10 us (17), of 4374
+// 10 368 261 (250), 20 250 476 (426); the matrices of 384 elements 10 us (17), of 4374
 // 77 (58).  Both or neither: the assembled values are the ordered sums of the element
 // matrices bit for bit.
 //

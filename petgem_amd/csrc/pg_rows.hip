@@ -127,19 +127,19 @@ __global__ void __launch_bounds__(kWave, (P == 3 ? 1 : 3)) k_element_matrices(
 // in pieces, its slots read back in between.
 // One wave per workgroup: no barriers, and nine workgroups fit into a CU's LDS at
 // p = 2.  What bounds it is latency at two waves per SIMD: the matrix cores have no
-// work here (a row is 400 FP64 operations on 12 coefficients), and bytes (1 GB at
-// 162 000 elements, p = 2: 200 us), VALU (160 us) and LDS (110 us) add up to 430 us
+// work here (a row is some 800 FP64 operations on 12 coefficients), and bytes (1 GB at
+// 162 000 elements, p = 2: 200 us), VALU (160 us) and LDS (110 us) add up to 417 us
 // because too few waves overlap them.  What took most of the time at first was the
 // wait of a batch's first loads for the stores of the batch before (loads and stores
 // return in order): contributors, pairs, orientations and coefficients are now asked
-// for a batch ahead and are there before the stores (560 -> 440 us), which bypass the
-// cache hierarchy's reuse (467 -> 436).  At p <= 2 the sums of K_e stay in
+// for a batch ahead and are there before the stores (546 -> 468 us, then 436 -> 428),
+// which bypass the caches' reuse (467 -> 436).  At p <= 2 the sums of K_e stay in
 // registers until those of M_e are there, so that a slot is written once: written in two
 // halves, 1.25 GB went to HBM in place of 0.7.  p = 3 keeps two passes: its columns
 // do not fit into registers.
-// The whole call, against a thread per (pair, row) with the 12 coefficients of every
-// entry gathered from tables: 162 000 elements p = 2 724 -> 428 us; 10 368 elements
-// p = 3 261 -> 246, 63 888 elements 1533 -> 1164; 162 000 elements p = 1 253 -> 100.
+// The whole call, against a wave per entity that gathered 12 table values for every
+// entry: 162 000 elements p = 2 724 -> 417 us; 10 368 elements
+// p = 3 261 -> 250, 63 888 elements 1533 -> 1206; 162 000 elements p = 1 253 -> 102.
 // ---------------------------------------------------------------------------
 constexpr int kAsmPairs = 256;  // pairs staged at a time: the batches of usual meshes have fewer
 constexpr int kDiagonal = 1 << 24, kEliminated = 2 << 24, kTwo = 4 << 24, kMore = 8 << 24;
@@ -631,8 +631,8 @@ void launch_asm(AsmArgs& a, hipStream_t st) {
   };
   // several batches a wave while they leave every CU several rounds of waves; on an
   // empty chip, where a wave's own time is the call's, less than a batch, and K_e and
-  // M_e by different waves (384 elements, p = 2: 11.6 -> 9.2 us; 3072, two waves per
-  // SIMD as they are: 14.8, split 17.9)
+  // M_e by different waves (p = 2: 384 elements 11.6 -> 9.2 us, 1296 elements 10.8, with
+  // the smallest shares and not split 17.9; 3072 elements, not split, 15.0)
   a.share = 16;
   while (a.share > 4 && blocks(a.share) < 10240) a.share /= 2;
   while (a.share > 1 && blocks(a.share) < 512) a.share /= 2;
