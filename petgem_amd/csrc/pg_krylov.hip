@@ -19,10 +19,10 @@
 //    reproducible).  The kernel boundary makes the partials visible, so no
 //    workgroup issues a device-scope fence (those force L2 write-backs
 //    across the XCDs and cost ~0.2 ms per kernel at this size);
-//  * every kernel returns once the device-side `done` flag is set (read first,
-//    looked at when its first loads are under way: the flag comes from memory,
-//    about 1 us on a kernel that takes 4), so the host enqueues batches of
-//    iterations and reads the flags only between batches;
+//  * every kernel returns once an earlier one has set the device-side `done` flag
+//    (pg_stop.h; read first, looked at when its first loads are under way: the flag
+//    comes from memory, about 1 us on a kernel that takes 4), so the host enqueues
+//    batches of iterations and reads the flags only between batches;
 //  * each XCD owns a contiguous eighth of the rows; in the SpMV its
 //    workgroups sweep that eighth together (row-interleaved) so that the
 //    gathers of x stay in the XCD's L2, in the vector kernels each workgroup
@@ -47,6 +47,7 @@
 #include "pg_blockinv.h"
 #include "pg_common.h"
 #include "pg_eop.h"
+#include "pg_stop.h"
 
 namespace pg {
 
@@ -69,7 +70,9 @@ struct Scal {
   Rec rec[2];
   double res2, bnorm2, tol2, ref2;
   double res64;
-  int32_t iter, maxit, done, status;
+  int32_t iter, maxit;
+  int32_t done;  // 0, or who stopped the recursion (pg_stop.h)
+  int32_t status;
   int32_t stall_limit, stalled;
 };
 
@@ -481,12 +484,12 @@ __device__ inline bool step_alpha(double2 rho, double2 mu, double2* alpha) {
   *alpha = zdiv(rho, mu);
   return (mu.x != 0.0 || mu.y != 0.0) && isfinite(alpha->x) && isfinite(alpha->y);
 }
-__device__ inline void store_alpha(Scal* s, double2 mu, double2 alpha, bool ok) {
+__device__ inline void store_alpha(Scal* s, double2 mu, double2 alpha, bool ok, int32_t self) {
   s->mu = mu;
   s->alpha = ok ? alpha : make_double2(0.0, 0.0);
   if (!ok) {
     s->status = PG_ERR_BREAKDOWN;
-    s->done = 1;
+    s->done = self;
   }
 }
 
@@ -517,23 +520,25 @@ __device__ inline Step step_update(const Scal* s, const Rec& old, const double (
   }
   return t;
 }
-__device__ inline void store_step(Scal* s, Rec* to, const Step& t, double res2) {
+__device__ inline void store_step(Scal* s, Rec* to, const Step& t, double res2, int32_t self) {
   s->beta = t.beta;
   s->res2 = res2;
   s->iter = t.rec.iter;
   *to = t.rec;
   if (t.broken) s->status = PG_ERR_BREAKDOWN;
   if (t.stalled) s->stalled = 1;
-  if (t.stop) s->done = 1;
+  if (t.stop) s->done = self;
 }
 
-// alpha from the product's partials; false = return (a breakdown)
-__device__ inline bool get_alpha(Scal* s, const double* part, int np, int slot, double2* al) {
+// alpha from the product's partials, in launch `self` (pg_stop.h); false = return (a
+// breakdown)
+__device__ inline bool get_alpha(Scal* s, const double* part, int np, int slot, int32_t self,
+                                 double2* al) {
   double tot[2];
   sum_partials<2>(part, np, tot);
   const double2 mu = make_double2(tot[0], tot[1]);
   const bool ok = step_alpha(s->rec[slot].rho, mu, al);
-  if (blockIdx.x == 0 && threadIdx.x == 0) store_alpha(s, mu, *al, ok);
+  if (blockIdx.x == 0 && threadIdx.x == 0) store_alpha(s, mu, *al, ok, self);
   return ok;
 }
 
@@ -557,7 +562,7 @@ __global__ void __launch_bounds__(kBS) k_update(Scal* s, int64_t n, XT* __restri
                                                 const XT* __restrict__ q,
                                                 const XT* __restrict__ dinv, XT* __restrict__ z,
                                                 const double* pin, int np, int slot,
-                                                double* part) {
+                                                int32_t self, double* part) {
   const int32_t done = s->done;
   int64_t lo, hi;
   chunk(n, kBS, &lo, &hi);
@@ -572,9 +577,9 @@ __global__ void __launch_bounds__(kBS) k_update(Scal* s, int64_t n, XT* __restri
     }
   };
   load();
-  if (done) return;
+  if (stopped_before(done, self)) return;
   double2 al;
-  if (!get_alpha(s, pin, np, slot, &al)) return;
+  if (!get_alpha(s, pin, np, slot, self, &al)) return;
   const XT na = from_d<XT>(make_double2(-al.x, -al.y));
   double red[3] = {0.0, 0.0, 0.0};
   while (i < hi) {
@@ -597,10 +602,10 @@ template <typename XT>
 __global__ void __launch_bounds__(kBS) k_update_blk(
     Scal* s, int64_t nb, const int32_t* __restrict__ bptr, const int32_t* __restrict__ boff,
     XT* __restrict__ r, const XT* __restrict__ q, const XT* __restrict__ binv,
-    XT* __restrict__ z, const double* pin, int np, int slot, double* part) {
-  if (s->done) return;
+    XT* __restrict__ z, const double* pin, int np, int slot, int32_t self, double* part) {
+  if (stopped_before(s->done, self)) return;
   double2 al;
-  if (!get_alpha(s, pin, np, slot, &al)) return;
+  if (!get_alpha(s, pin, np, slot, self, &al)) return;
   const XT na = from_d<XT>(make_double2(-al.x, -al.y));
   int64_t lo, hi;
   chunk(nb, kBS, &lo, &hi);
@@ -641,7 +646,8 @@ __global__ void __launch_bounds__(kBS) k_update_blk2(Scal* s, int64_t nb, XT* __
                                                      const XT* __restrict__ q,
                                                      const XT* __restrict__ binv,
                                                      XT* __restrict__ z, const double* pin,
-                                                     int np, int slot, double* part) {
+                                                     int np, int slot, int32_t self,
+                                                     double* part) {
   using V = typename PairOf<XT>::type;
   const int32_t done = s->done;
   int64_t lo, hi;
@@ -662,9 +668,9 @@ __global__ void __launch_bounds__(kBS) k_update_blk2(Scal* s, int64_t nb, XT* __
     }
   };
   load();
-  if (done) return;
+  if (stopped_before(done, self)) return;
   double2 al;
-  if (!get_alpha(s, pin, np, slot, &al)) return;
+  if (!get_alpha(s, pin, np, slot, self, &al)) return;
   const XT na = from_d<XT>(make_double2(-al.x, -al.y));
   double red[3] = {0.0, 0.0, 0.0};
   while (k < hi) {
@@ -696,7 +702,7 @@ __global__ void __launch_bounds__(kBS) k_fin_update(Scal* __restrict__ s, const 
   sum_partials<3>(part, np, tot);
   if (threadIdx.x != 0) return;
   const Rec old = s->rec[from];
-  store_step(s, &s->rec[to], step_update(s, old, tot), tot[2]);
+  store_step(s, &s->rec[to], step_update(s, old, tot), tot[2], kStopOther);
 }
 
 // x += alpha p (the previous iteration's step: alpha is still that iteration's,
@@ -705,7 +711,8 @@ __global__ void __launch_bounds__(kBS) k_fin_update(Scal* __restrict__ s, const 
 template <typename XT, bool FUSE>
 __global__ void __launch_bounds__(kBS) k_pupdate(Scal* s, int64_t n, const XT* __restrict__ z,
                                                  XT* __restrict__ p, XT* __restrict__ x,
-                                                 const double* pin, int np, int from, int to) {
+                                                 const double* pin, int np, int from, int to,
+                                                 int32_t self) {
   const int32_t done = s->done;
   int64_t lo, hi;
   chunk(n, kBS, &lo, &hi);
@@ -719,13 +726,13 @@ __global__ void __launch_bounds__(kBS) k_pupdate(Scal* s, int64_t n, const XT* _
     }
   };
   load();
-  if (done) return;
+  if (stopped_before(done, self)) return;
   double2 beta;
   if (FUSE) {
     double tot[3];
     sum_partials<3>(pin, np, tot);
     const Step t = step_update(s, s->rec[from], tot);
-    if (blockIdx.x == 0 && threadIdx.x == 0) store_step(s, &s->rec[to], t, tot[2]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) store_step(s, &s->rec[to], t, tot[2], self);
     if (t.stop) return;  // every workgroup decides the same
     beta = t.beta;
   } else {
@@ -1349,23 +1356,23 @@ static void launch_iteration(Solver* S, hipStream_t st, const SpmvCfg& c, const 
   const dim3 b(kBS);
   if (k > 0)
     hipLaunchKernelGGL((k_pupdate<XT, true>), dim3(S->gv), b, 0, st, S->s, S->n, z, p, x,
-                       S->part2, gu, slot ^ 1, slot);
+                       S->part2, gu, slot ^ 1, slot, stop_direction(k));
   else
     hipLaunchKernelGGL((k_pupdate<XT, false>), dim3(S->gv), b, 0, st, S->s, S->n, z, p, x,
-                       nullptr, 0, 0, 0);
+                       nullptr, 0, 0, 0, stop_direction(k));
   // a failed record only loses this timing sample (the elapsed-time query fails)
   if (sample) (void)hipEventRecord(S->ev[0], st);
   spmv<1, VT, XT>(S, c, st, vals, p, q, nullptr, sample && c.kind == 3 ? S->ev[2] : nullptr);
   if (sample) (void)hipEventRecord(S->ev[1], st);
   if (blk && S->blk2)  // r, q, z: the solver's own 256-byte aligned buffers
     hipLaunchKernelGGL(k_update_blk2<XT>, dim3(gu), b, 0, st, S->s, S->nblocks, r, q, binv, z,
-                       S->part, c.grid, slot, S->part2);
+                       S->part, c.grid, slot, stop_update(k), S->part2);
   else if (blk)
     hipLaunchKernelGGL(k_update_blk<XT>, dim3(gu), b, 0, st, S->s, S->nblocks, S->bptr, S->boff,
-                       r, q, binv, z, S->part, c.grid, slot, S->part2);
+                       r, q, binv, z, S->part, c.grid, slot, stop_update(k), S->part2);
   else
     hipLaunchKernelGGL(k_update<XT>, dim3(gu), b, 0, st, S->s, S->n, r, q, dinv, z, S->part,
-                       c.grid, slot, S->part2);
+                       c.grid, slot, stop_update(k), S->part2);
   if (k == count - 1)
     hipLaunchKernelGGL(k_fin_update, dim3(1), b, 0, st, S->s, S->part2, gu, slot, 0);
 }
