@@ -343,7 +343,7 @@ int pg_eop_create_multi(int p, int nmesh, const int64_t *n_elems, const void *co
 /* Re-read the element coefficients after pg_element_geometry (new conductivity)
  * or for a new frequency. */
 int pg_eop_refresh(void *op, const void *ws, double omega, void *stream);
-/* y = A x in complex128 / complex64 (interleaved, length 2 ndof). */
+/* y = A x in complex128 / complex64 (interleaved, length 2 ndof); y may be x. */
 int pg_eop_apply_z(const void *op, const double *x, double *y, void *stream);
 int pg_eop_apply_c(const void *op, const float *x, float *y, void *stream);
 int pg_eop_destroy(void *op);

@@ -624,6 +624,13 @@ __global__ void k_eop_coef(int64_t nslot, const int32_t* __restrict__ perm,
   }
 }
 
+template <typename R>
+__global__ void __launch_bounds__(kBS) k_eop_copy(int64_t n, const R* __restrict__ x,
+                                                  R* __restrict__ y) {
+  const int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x;
+  if (i < n) y[i] = x[i];
+}
+
 }  // namespace eop
 
 struct ElemOp {
@@ -652,6 +659,8 @@ struct ElemOp {
   int32_t *bslot = nullptr, *bcode = nullptr, *bdofs = nullptr;
   uint32_t* bpos = nullptr;
   int2* em = nullptr;
+  // its x where the caller's y overlaps it (2 ndof reals)
+  double* xcopy = nullptr;
   // multi-mesh operator (pg_eop_create_multi): segment of every wave, omega mu0
   // of every segment, first schedule position of every segment (nseg + 1)
   int nseg = 0;
@@ -1136,6 +1145,7 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     PG_A(op->bdofs, B.dofs.size());
     PG_A(op->bpos, B.pos.size());
     PG_A(op->em, B.em.size());
+    PG_A(op->xcopy, 2 * ndof);
   } else {
     PG_A(op->ye64, nslot * N);
     PG_A(op->ye32, nslot * N);
@@ -1184,6 +1194,29 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     PG_FAIL(PG_ERR_HIP, "element operator setup failed");
   }
   *out = op;
+  return PG_OK;
+}
+
+// y = A x.  y may be x or overlap it: the one-kernel product stores y while other
+// workgroups still gather x, so it then reads a copy (the two kernels finish the
+// gathers before the first store).
+template <typename R>
+static int apply(const void* handle, const R* x, R* y, void* stream) {
+  if (!handle || !x || !y) PG_FAIL(PG_ERR_ARG, "bad arguments");
+  using C = typename eop::Cx<R>::T;
+  const ElemOp* op = static_cast<const ElemOp*>(handle);
+  hipStream_t st = as_stream(stream);
+  const int64_t n = 2 * op->ndof;
+  const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y);
+  if (op->xcopy && xa < ya + n * sizeof(R) && ya < xa + n * sizeof(R)) {
+    R* copy = reinterpret_cast<R*>(op->xcopy);
+    hipLaunchKernelGGL(eop::k_eop_copy<R>, dim3((unsigned)((n + eop::kBS - 1) / eop::kBS)),
+                       dim3(eop::kBS), 0, st, n, x, copy);
+    x = copy;
+  }
+  eop_launch(op, 0, nullptr, reinterpret_cast<const C*>(x), reinterpret_cast<C*>(y), nullptr,
+             nullptr, st);
+  PG_CHECK_LAUNCH();
   return PG_OK;
 }
 
@@ -1311,19 +1344,11 @@ int pg_eop_refresh(void* op, const void* ws, double omega, void* stream) {
 }
 
 int pg_eop_apply_z(const void* op, const double* x, double* y, void* stream) {
-  if (!op || !x || !y) PG_FAIL(PG_ERR_ARG, "bad arguments");
-  eop_launch(static_cast<const ElemOp*>(op), 0, nullptr, reinterpret_cast<const double2*>(x),
-             reinterpret_cast<double2*>(y), nullptr, nullptr, as_stream(stream));
-  PG_CHECK_LAUNCH();
-  return PG_OK;
+  return apply<double>(op, x, y, stream);
 }
 
 int pg_eop_apply_c(const void* op, const float* x, float* y, void* stream) {
-  if (!op || !x || !y) PG_FAIL(PG_ERR_ARG, "bad arguments");
-  eop_launch(static_cast<const ElemOp*>(op), 0, nullptr, reinterpret_cast<const float2*>(x),
-             reinterpret_cast<float2*>(y), nullptr, nullptr, as_stream(stream));
-  PG_CHECK_LAUNCH();
-  return PG_OK;
+  return apply<float>(op, x, y, stream);
 }
 
 int pg_eop_destroy(void* op) {
