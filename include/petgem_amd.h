@@ -37,7 +37,7 @@ const char *pg_last_error(void);
 
 /* ------------------------------------------------------------------------
  * Reference-element tables for uniform order p (1..3), resident on the
- * current device: per-orientation basis contractions over the order-2p
+ * current device where its kernels read them (p > 1): per-orientation basis contractions over the order-2p
  * quadrature.  Replaces the per-element quadrature loop of
  * computeElementalMatrices (petgem/hvfem.py:250-310) and the basis
  * evaluation of shape3DETet (petgem/hvfem.py:319-464).
@@ -110,8 +110,8 @@ int pg_plan_entity_pairs(const void *plan, int32_t *entity_pair, int32_t *max_ro
 
 /* Device view of an exported plan (all device pointers).  entity_pair
  * (nullable, from pg_plan_entity_pairs, with entity_row_max its max_rowlen)
- * saves the numeric assembly a search for its entities' first pairs (small p = 3
- * systems: selects the form that sums an entity's rows in LDS).  Same values,
+ * saves the numeric assembly a search for its entities' first pairs (small p = 2
+ * and 3 systems: selects the form that sums an entity's rows in LDS).  Same values,
  * bitwise. */
 typedef struct pg_plan_dev {
   int32_t p;

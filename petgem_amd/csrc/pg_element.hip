@@ -80,10 +80,10 @@ static void build_table(int p, std::vector<double>& T) {
 
 struct Tables {
   int p;
-  double* d_T;  // p = 3 only (the other orders' kernels form their products without)
+  double* d_T;  // p > 1 (at p = 1 every kernel forms its products without)
 };
-// p = 3: elements from which on the factored kernels are the faster
-constexpr int64_t kFactoredElements = 4096;
+// elements from which on the factored kernels (pg_rows.hip) are the faster
+constexpr int64_t factored_elements(int p) { return p == 1 ? 0 : (p == 2 ? 2048 : 4096); }
 
 // -------------------------------------------------------------------------
 // geometry + orientation (one thread per element)
@@ -204,15 +204,22 @@ __device__ inline int local_entity_ndof(int la) {
 }
 
 // -------------------------------------------------------------------------
-// Element matrices and assembly from the tables: p = 3 below kFactoredElements
-// elements (above, and at p <= 2: pg_rows.hip).  An entry is 12 multiplications on a
+// Element matrices and assembly from the tables: systems of fewer than
+// factored_elements() (above: pg_rows.hip).  An entry is 12 multiplications on a
 // gathered table row and independent of the others, so these are bound by the gathers
-// on a full chip, but short on an empty one, where a factored row of p = 3 (some 3000
-// operations one after another, for K_e and then for M_e) is the time of the call:
-// assembly of 384 elements 15.6 us (factored 26.6), 1296 32 (46), 4374 93 (92),
-// 10 368 261 (250), 20 250 476 (426); the matrices of 384 elements 10 us (17), of 4374
-// 77 (58).  Both or neither: the assembled values are the ordered sums of the element
-// matrices bit for bit.
+// on a full chip, but short on an empty one, where a factored row is the time of the
+// call: at p = 3 some 3000 operations one after another, for K_e and then for M_e, at
+// p = 2 the loads that lead to a wave's first row and the sums through LDS.
+//   p = 3, assembly of 384 elements 15.6 us (factored 26.6), 1296 32 (46), 4374 93 (92),
+//   10 368 261 (250), 20 250 476 (426); the matrices of 384 elements 10 us (17), of
+//   4374 77 (58).
+//   p = 2, assembly of 384 elements 7.7 us (factored 9.2), 750 7.9 (9.7), 1296 9.2
+//   (10.8), 2058 12.2 (12.6), 3072 16.1 (14.9); the matrices of 3072 14.1 (10.4), of
+//   fewer the same (10.4, what the calls themselves take).
+// (p = 1: geometry and assembly of 162 to 3072 elements 51.7 to 54.7 us from tables, 51.1
+// to 53.5 factored, which is therefore the only form.)
+// Both or neither: the assembled values are the ordered sums of the element matrices
+// bit for bit.
 //
 // Element matrices: one thread per (element, i, j).
 // -------------------------------------------------------------------------
@@ -249,9 +256,9 @@ __device__ inline void contract(const double* __restrict__ t, const double* __re
 
 template <int P>
 __global__ void k_table_matrices(int64_t E, const double* __restrict__ T,
-                                   const double* __restrict__ coef,
-                                   const int32_t* __restrict__ orient, double* __restrict__ M,
-                                   double* __restrict__ K) {
+                                 const double* __restrict__ coef,
+                                 const int32_t* __restrict__ orient, double* __restrict__ M,
+                                 double* __restrict__ K) {
   constexpr int n = P * (P + 2) * (P + 3) / 2;
   constexpr int V = 12 * P + 24 * P * (P - 1) + P * (P - 1) * (P - 2) / 2;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -351,8 +358,8 @@ __global__ void __launch_bounds__(256) k_table_pairs(
 }
 
 // -------------------------------------------------------------------------
-// Assembly of plans within the bounds of pg_rowasm.h: one single-wave workgroup per entity A with DOFs keeps A's d(A) CSR rows in LDS
-// and walks the elements containing A in ascending order (the contributors of
+// Assembly of plans within the bounds of pg_rowasm.h: one single-wave workgroup per
+// entity A with DOFs keeps A's d(A) CSR rows in LDS and walks the elements containing A in ascending order (the contributors of
 // the diagonal pair (A, A)).  For each element its lanes form the entries of
 // the element's block row la(A) -- row k < d(A), every local DOF j -- from the
 // tables and the element's coefficients (one element per step: wave-uniform
@@ -837,7 +844,7 @@ int pg_tables_create(int p, void** tables) {
   int device;
   PG_HIP(hipGetDevice(&device));
   double* d_T = nullptr;
-  if (p == 3) {
+  if (p > 1) {
     std::vector<double> T;
     build_table(p, T);
     PG_HIP(hipMalloc(&d_T, T.size() * sizeof(double)));
@@ -896,18 +903,33 @@ int pg_element_orientation(int64_t E, const int32_t* en, const int32_t* ee, cons
   return PG_OK;
 }
 
-int pg_element_matrices(const void* tables, int64_t E, const void* ws, double* M, double* K,
-                        void* stream) {
-  if (!tables || !ws || !M || !K || E <= 0) PG_FAIL(PG_ERR_ARG, "bad arguments");
-  const Tables* t = static_cast<const Tables*>(tables);
-  void* w = const_cast<void*>(ws);
-  if (t->p == 3 && E < kFactoredElements)
-    hipLaunchKernelGGL(k_table_matrices<3>, dim3(nblocks(E * 45 * 45, 256)), dim3(256), 0,
-                       as_stream(stream), E, t->d_T, ws_coef(w), ws_orient(w, E), M, K);
+}  // extern "C"
+
+namespace pg {
+
+template <int P>
+static void table_matrices(const double* T, int64_t E, const double* coef, const int32_t* orient,
+                           double* M, double* K, hipStream_t s) {
+  constexpr int n = P * (P + 2) * (P + 3) / 2;
+  hipLaunchKernelGGL(k_table_matrices<P>, dim3(nblocks(E * n * n, 256)), dim3(256), 0, s, E, T,
+                     coef, orient, M, K);
+}
+
+template <int P>
+static void table_assembly(const double* T, const pg_plan_dev* pl, const double* coef,
+                           const int32_t* orient, double om, const uint8_t* ent_bc, double2* v,
+                           double* Kout, double* Mout, hipStream_t s) {
+  const int64_t nent = pl->n_edges + pl->n_faces + (P > 2 ? pl->n_elems : 0);
+  if (pl->entity_pair)
+    hipLaunchKernelGGL(k_table_rows<P>, dim3((unsigned)nent), dim3(64), 0, s, pl->n_edges,
+                       pl->n_faces, pl->entity_pair, T, pl->rowptr, pl->pair_slot0, pl->pair_cbeg,
+                       pl->pair_ab, pl->contrib, coef, orient, om, Kout ? 1 : 0, ent_bc, v, Kout,
+                       Mout);
   else
-    launch_element_matrices(t->p, E, ws_coef(w), ws_orient(w, E), M, K, as_stream(stream));
-  PG_CHECK_LAUNCH();
-  return PG_OK;
+    hipLaunchKernelGGL(k_table_pairs<P>, dim3(nblocks(pl->npairs * P * (P - 1), 256)), dim3(256), 0, s,
+                       pl->npairs, pl->n_edges, pl->n_faces, T, pl->pair_slot0,
+                       pl->pair_rowlen, pl->pair_cbeg, pl->pair_ab, pl->contrib, coef, orient, om,
+                       ent_bc, v, Kout, Mout);
 }
 
 static int assemble_impl(const void* tables, const pg_plan_dev* pl, const void* ws, double omega,
@@ -922,18 +944,31 @@ static int assemble_impl(const void* tables, const pg_plan_dev* pl, const void* 
   const int32_t* orient = ws_orient(w, pl->n_elems);
   const double om = omega * kMu0;
   double2* v = reinterpret_cast<double2*>(values);
-  if (t->p < 3 || pl->n_elems >= kFactoredElements)
+  if (pl->n_elems >= factored_elements(t->p))
     launch_assembly(*pl, coef, orient, om, ent_bc, v, Kout, Mout, s);
-  else if (pl->entity_pair)
-    hipLaunchKernelGGL(k_table_rows<3>, dim3((unsigned)(pl->n_edges + pl->n_faces + pl->n_elems)),
-                       dim3(64), 0, s, pl->n_edges, pl->n_faces, pl->entity_pair, t->d_T, pl->rowptr,
-                       pl->pair_slot0, pl->pair_cbeg, pl->pair_ab, pl->contrib, coef, orient, om,
-                       Kout ? 1 : 0, ent_bc, v, Kout, Mout);
+  else if (t->p == 2)
+    table_assembly<2>(t->d_T, pl, coef, orient, om, ent_bc, v, Kout, Mout, s);
   else
-    hipLaunchKernelGGL(k_table_pairs<3>, dim3(nblocks(pl->npairs * 6, 256)), dim3(256), 0, s,
-                       pl->npairs, pl->n_edges, pl->n_faces, t->d_T, pl->pair_slot0, pl->pair_rowlen,
-                       pl->pair_cbeg, pl->pair_ab, pl->contrib, coef, orient, om, ent_bc, v, Kout,
-                       Mout);
+    table_assembly<3>(t->d_T, pl, coef, orient, om, ent_bc, v, Kout, Mout, s);
+  PG_CHECK_LAUNCH();
+  return PG_OK;
+}
+
+}  // namespace pg
+
+extern "C" {
+
+int pg_element_matrices(const void* tables, int64_t E, const void* ws, double* M, double* K,
+                        void* stream) {
+  if (!tables || !ws || !M || !K || E <= 0) PG_FAIL(PG_ERR_ARG, "bad arguments");
+  const Tables* t = static_cast<const Tables*>(tables);
+  void* w = const_cast<void*>(ws);
+  const double* coef = ws_coef(w);
+  const int32_t* orient = ws_orient(w, E);
+  hipStream_t s = as_stream(stream);
+  if (E >= factored_elements(t->p)) launch_element_matrices(t->p, E, coef, orient, M, K, s);
+  else if (t->p == 2) table_matrices<2>(t->d_T, E, coef, orient, M, K, s);
+  else table_matrices<3>(t->d_T, E, coef, orient, M, K, s);
   PG_CHECK_LAUNCH();
   return PG_OK;
 }

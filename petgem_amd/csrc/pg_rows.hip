@@ -631,8 +631,8 @@ void launch_asm(AsmArgs& a, hipStream_t st) {
   };
   // several batches a wave while they leave every CU several rounds of waves; on an
   // empty chip, where a wave's own time is the call's, less than a batch, and K_e and
-  // M_e by different waves (p = 2: 384 elements 11.6 -> 9.2 us, 1296 elements 10.8, with
-  // the smallest shares and not split 17.9; 3072 elements, not split, 15.0)
+  // M_e by different waves (p = 1: 384 elements 9.9 -> 7.9 us, 2058 10.1 -> 7.7; p = 2:
+  // 2058 elements 13.7 -> 12.5, 3072, the same either way, 14.9)
   a.share = 16;
   while (a.share > 4 && blocks(a.share) < 10240) a.share /= 2;
   while (a.share > 1 && blocks(a.share) < 512) a.share /= 2;
