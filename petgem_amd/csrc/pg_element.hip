@@ -1001,8 +1001,10 @@ int pg_locate_points(int64_t E, const double* coords, int64_t npts, const double
   hipStream_t s = as_stream(stream);
   hipLaunchKernelGGL(k_fill_i32, dim3(nblocks(npts, 256)), dim3(256), 0, s, npts, out, -1);
   // few elements: slices of at least eight points, up to half a million threads (at
-  // 29 478 elements and 101 points 20 us with one slice, 7 us with twelve)
-  const int64_t slices = std::max<int64_t>(1, std::min((1 << 19) / E, npts / 8));
+  // 29 478 elements and 101 points 20 us with one slice, 7 us with twelve) and what a
+  // grid's second dimension holds
+  const int64_t slices =
+      std::max<int64_t>(1, std::min({(int64_t)(1 << 19) / E, npts / 8, (int64_t)65535}));
   hipLaunchKernelGGL(k_locate, dim3(nblocks(E, 256), (unsigned)slices), dim3(256), 0, s, E, coords,
                      npts, pts, tol, out);
   PG_CHECK_LAUNCH();
