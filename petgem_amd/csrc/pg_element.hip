@@ -748,7 +748,7 @@ __global__ void __launch_bounds__(256) k_receivers(int64_t npts, const double* _
 // place of a DOF depends on it), the table is filled from f, the receivers' products
 // are added to it one receiver after another, and it is stored.  (A single thread
 // taking one receiver after another needed 510 us for 101 receivers at p = 2; this
-// takes @@ us.)
+// takes 24.)
 // -------------------------------------------------------------------------
 constexpr int kAdjThreads = 512, kAdjValues = 1024, kAdjTable = 2048;
 
@@ -800,13 +800,15 @@ __global__ void __launch_bounds__(kAdjThreads) k_adjoint_rhs(int64_t npts,
       if (key[i] >= 0) sum[i] = f[key[i]];
     __syncthreads();
     const int nq = (int)(npts - q0 < Q ? npts - q0 : Q);
-    if (t < 64)  // one wave: LDS operations in order, an element's DOFs are distinct
+    if (t < 64)  // one wave, a fence between receivers; an element's DOFs are distinct
       for (int k = 0; k < nq; ++k) {
         if (t < n && place[k * n + t] >= 0) {
           const double2 v = val[k * n + t];
           double2* s = sum + place[k * n + t];
           *s = make_double2(s->x + v.x, s->y + v.y);
         }
+        // the next receiver's lanes read what other lanes stored
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
       }
     __syncthreads();
