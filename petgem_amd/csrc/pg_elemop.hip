@@ -624,6 +624,22 @@ __global__ void k_eop_coef(int64_t nslot, const int32_t* __restrict__ perm,
   }
 }
 
+// k_eop_blk's orientations and entities from its slots
+__global__ void __launch_bounds__(kBS) k_eop_blk_elements(int64_t n, int nle,
+                                                          const int32_t* __restrict__ bslot,
+                                                          const int32_t* __restrict__ ocode,
+                                                          const int32_t* __restrict__ edofs,
+                                                          int32_t* __restrict__ bcode,
+                                                          int32_t* __restrict__ bdofs) {
+  const int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x;
+  if (i >= n) return;
+  const int64_t s = bslot[i], g = i / kGroup, l = i % kGroup;
+  bcode[i] = s >= 0 ? ocode[s] : 0;
+  for (int la = 0; la < nle; ++la)
+    bdofs[(g * nle + la) * kGroup + l] =
+        s >= 0 ? edofs[(s / kWave * nle + la) * kWave + s % kWave] : -1;
+}
+
 template <typename R>
 __global__ void __launch_bounds__(kBS) k_eop_copy(int64_t n, const R* __restrict__ x,
                                                   R* __restrict__ y) {
@@ -900,33 +916,32 @@ static int check_block_ptr(int p, const int32_t* bp, int64_t nblocks, int64_t nd
   return PG_OK;
 }
 
-// Blocks of k_eop_blk from the schedule (gm, and per incidence its slot and local
-// entity), each slot's orientation and entities: entities are taken in schedule
-// order while the elements around them fit `passes` groups and their local results
-// the LDS budget.  False when one entity alone does not fit.
+// Blocks of k_eop_blk from the schedule (gm, and per incidence its slot * NLE + local
+// entity): entities are taken in schedule order while the elements around them fit
+// `passes` groups and their local results the LDS budget.  False when one entity alone
+// does not fit.
 struct Blocks {
   std::vector<int4> meta;
-  std::vector<int32_t> slot, code, dofs;
-  std::vector<uint32_t> pos;
+  std::vector<int32_t> slot;
+  std::vector<uint16_t> pos;  // (two to a word of bpos)
   std::vector<int2> em;
   int lds_values = 1;
 };
-static bool make_blocks(int nle, int passes, const std::vector<int4>& gm,
-                        const std::vector<int32_t>& islot, const std::vector<uint8_t>& ila,
-                        const std::vector<int32_t>& hoc, const std::vector<int32_t>& hed,
-                        Blocks* B) {
+template <int NLE>
+static bool make_blocks(int passes, int64_t nslot, const std::vector<int4>& gm,
+                        const std::vector<int32_t>& inc, Blocks* B) {
   constexpr int G = eop::kGroup;
   constexpr int kMaxEnt = 1024;     // entities per block (PEC entities have no elements)
   constexpr int kMaxValues = 3072;  // complex128 values of LDS: 48 KB, three workgroups
+  constexpr int NQ = (NLE + 1) / 2;
   const int64_t nent = (int64_t)gm.size();
-  const int nq = (nle + 1) / 2;
-  std::vector<int32_t> stamp(hoc.size(), -1);  // block that last took the slot
-  std::vector<int32_t> place(hoc.size());      // and its element number there
-  const size_t ng0 = hoc.size() / G * 5 / 2 + 1;  // each element about twice
+  struct Mark {
+    int32_t block, place;  // block that last took the slot, its element number there
+  };
+  std::vector<Mark> mark(nslot, Mark{-1, 0});
+  const size_t ng0 = nslot / G * 5 / 2 + 1;  // each element about twice
   B->slot.reserve(ng0 * G);
-  B->code.reserve(ng0 * G);
-  B->dofs.reserve(ng0 * G * nle);
-  B->pos.reserve(ng0 * G * nq);
+  B->pos.reserve(ng0 * G * 2 * NQ);
   B->em.resize(nent);
   for (int64_t i = 0; i < nent;) {
     const int32_t b = (int32_t)B->meta.size();
@@ -935,30 +950,27 @@ static bool make_blocks(int nle, int passes, const std::vector<int4>& gm,
     for (; i < nent && i - i0 < kMaxEnt; ++i) {
       const int4 m = gm[i];
       const int n = m.w - m.z;
-      int fresh = 0;
-      for (int k = m.z; k < m.w; ++k) fresh += stamp[islot[k]] != b;
+      int fresh = n;  // at most; counted where that matters
+      if (ne + n > passes * G) {
+        fresh = 0;
+        for (int k = m.z; k < m.w; ++k) fresh += mark[inc[k] / NLE].block != b;
+      }
       if (n > 0xFFF || ne + fresh > passes * G || nv + n * m.y > kMaxValues) break;
       B->em[i] = make_int2(m.x, (int)((uint32_t)nv | (uint32_t)n << 16 | (uint32_t)m.y << 28));
       for (int k = m.z; k < m.w; ++k) {
-        const int64_t s = islot[k];
-        if (stamp[s] != b) {
-          stamp[s] = b;
-          place[s] = ne++;
-          const int64_t g = g0 + place[s] / G, e = place[s] % G;
+        const int s = inc[k] / NLE, la = inc[k] % NLE;
+        Mark& mk = mark[s];
+        if (mk.block != b) {
+          mk = Mark{b, ne++};
+          const int64_t g = g0 + mk.place / G, e = mk.place % G;
           if (e == 0) {
             B->slot.resize((g + 1) * G, -1);
-            B->code.resize((g + 1) * G, 0);
-            B->dofs.resize((g + 1) * G * nle, -1);
-            B->pos.resize((g + 1) * G * nq, 0xFFFFFFFFu);
+            B->pos.resize((g + 1) * G * 2 * NQ, 0xFFFF);
           }
-          B->slot[g * G + e] = (int32_t)s;
-          B->code[g * G + e] = hoc[s];
-          for (int la = 0; la < nle; ++la)
-            B->dofs[(g * nle + la) * G + e] = hed[(s / kWave * nle + la) * kWave + s % kWave];
+          B->slot[g * G + e] = s;
         }
-        const int la = ila[k];
-        uint32_t& at = B->pos[((g0 + place[s] / G) * nq + la / 2) * G + place[s] % G];
-        at = (la & 1) ? (at & 0xFFFFu) | (uint32_t)nv << 16 : (at & 0xFFFF0000u) | (uint32_t)nv;
+        B->pos[(((g0 + mk.place / G) * NQ + la / 2) * G + mk.place % G) * 2 + la % 2] =
+            (uint16_t)nv;
         nv += m.y;
       }
     }
@@ -967,6 +979,17 @@ static bool make_blocks(int nle, int passes, const std::vector<int4>& gm,
     B->lds_values = std::max(B->lds_values, nv);
   }
   return true;
+}
+
+// slot * (local entities) + local entity -> its first local result, (group * N + first
+// local DOF) * 64 + element of the group
+template <int P>
+static void local_results(std::vector<int32_t>& list) {
+  constexpr int NLE = eop::n_local_entities<P>(), N = fac::n_dofs<P>();
+  for (int32_t& v : list) {
+    const int s = v / NLE;
+    v = (s / kWave * N + entity_local_offset(v % NLE, P)) * kWave + s % kWave;
+  }
 }
 
 static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32_t* bp,
@@ -983,7 +1006,7 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
     for (int d = bp[g]; d < bp[g + 1]; ++d) ent_of[d] = (int32_t)g;
   // each local entity's global entity; its DOFs must be that entity's range in order
   std::vector<int32_t> eg((size_t)E * nle);
-  std::vector<int64_t> cnt(nblocks, 0);
+  std::vector<int32_t> cnt(nblocks, 0);
   for (int64_t e = 0; e < E; ++e)
     for (int la = 0; la < nle; ++la) {
       const int off = entity_local_offset(la, p), nd = entity_ndof(la, p);
@@ -1016,13 +1039,18 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   }
   // element order: by segment (multi-mesh operator), then by the earliest schedule
   // position of the element's entities (spatial order when the schedule is)
+  // (from here on an element's entities are known by their schedule positions, so that
+  // what follows, element after element in that order, finds an entity's data near the
+  // last one's)
   std::vector<int32_t> key(E);
   std::vector<int32_t> es(E, 0);
   for (int64_t e = 0; e < E; ++e) {
-    int32_t m = pos[eg[e * nle]], mx = m;
+    int32_t* ep = &eg[e * nle];
+    int32_t m = ep[0] = pos[ep[0]], mx = m;
     for (int la = 1; la < nle; ++la) {
-      m = std::min(m, pos[eg[e * nle + la]]);
-      mx = std::max(mx, pos[eg[e * nle + la]]);
+      ep[la] = pos[ep[la]];
+      m = std::min(m, ep[la]);
+      mx = std::max(mx, ep[la]);
     }
     key[e] = m;
     if (seg) {
@@ -1053,50 +1081,34 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   }
   const int64_t nw = (int64_t)wsg.size(), nslot = nw * kWave;
   if (nslot * N >= (1LL << 31)) PG_FAIL(PG_ERR_UNSUPPORTED, "too many elements");
-  std::vector<int32_t> hoc(nslot, 0);  // orientation per slot
-  for (int64_t s = 0; s < nslot; ++s)
-    if (perm[s] >= 0) hoc[s] = hor[perm[s]];
-  // per slot and local entity: the entity's first DOF (-1: PEC or empty)
-  std::vector<int32_t> hed((size_t)nslot * nle, -1);
-  for (int64_t s = 0; s < nslot; ++s) {
-    const int64_t e = perm[s];
-    if (e < 0) continue;
-    const int64_t w = s / kWave, l = s % kWave;
-    for (int la = 0; la < nle; ++la) {
-      const int g = eg[e * nle + la];
-      hed[(w * nle + la) * kWave + l] = hbc[g] ? -1 : bp[g];
-    }
-  }
-  // per-entity lists of local-result slots, in schedule order; within an
-  // entity in ascending slot order (a fixed summation order)
-  std::vector<int64_t> start(nblocks + 1, 0);
-  for (int64_t i = 0; i < nblocks; ++i) {
-    const int64_t g = order ? order[i] : i;
-    start[i + 1] = start[i] + (hbc[g] ? 0 : cnt[g]);
-  }
-  if (start[nblocks] >= (1LL << 31)) PG_FAIL(PG_ERR_UNSUPPORTED, "too many incidences");
-  std::vector<int32_t> gslot(start[nblocks]), islot(start[nblocks]);  // local result, slot
-  std::vector<uint8_t> ila(start[nblocks]);                           // local entity
-  std::vector<int64_t> cur(nblocks);
-  for (int64_t g = 0; g < nblocks; ++g) cur[g] = start[pos[g]];
-  for (int64_t s = 0; s < nslot; ++s) {
-    const int64_t e = perm[s];
-    if (e < 0) continue;
-    const int64_t w = s / kWave, l = s % kWave;
-    for (int la = 0; la < nle; ++la) {
-      const int g = eg[e * nle + la];
-      if (hbc[g]) continue;
-      const int64_t c = cur[g]++;
-      gslot[c] = (int32_t)((w * N + entity_local_offset(la, p)) * kWave + l);
-      islot[c] = (int32_t)s;
-      ila[c] = (uint8_t)la;
-    }
-  }
+  // scheduled entities with their lists of local results (in schedule order; the list's
+  // end counts up as it is filled, -1: PEC)
   std::vector<int4> gm(nblocks);
+  int64_t total = 0;
   for (int64_t i = 0; i < nblocks; ++i) {
     const int64_t g = order ? order[i] : i;
-    gm[i] = make_int4(bp[g], bp[g + 1] - bp[g], (int)start[i], (int)start[i + 1]);
+    gm[i] = make_int4(bp[g], bp[g + 1] - bp[g], (int)total, hbc[g] ? -1 : (int)total);
+    total += hbc[g] ? 0 : cnt[g];
+    if (total >= (1LL << 31)) PG_FAIL(PG_ERR_UNSUPPORTED, "too many incidences");
   }
+  // per slot its orientation, per slot and local entity the entity's first DOF (-1: PEC
+  // or empty), and the lists: slot * nle + local entity, within an entity in ascending
+  // slot order (a fixed summation order)
+  std::vector<int32_t> hoc(nslot, 0), hed((size_t)nslot * nle, -1), inc(total);
+  for (int64_t s = 0; s < nslot; ++s) {
+    const int64_t e = perm[s];
+    if (e < 0) continue;
+    const int64_t w = s / kWave, l = s % kWave;
+    hoc[s] = hor[e];
+    for (int la = 0; la < nle; ++la) {
+      int4& m = gm[eg[e * nle + la]];
+      if (m.w < 0) continue;
+      hed[(w * nle + la) * kWave + l] = m.x;
+      inc[m.w++] = (int32_t)(s * nle + la);
+    }
+  }
+  for (int4& m : gm)
+    if (m.w < 0) m.w = m.z;
   // The one-kernel product at p <= 2.  Two groups per block from 131 072 elements:
   // fewer elements are computed twice (1.8 against 2.1 times each, p = 2), but a
   // block takes two passes, which pays once the blocks fill the chip several
@@ -1107,7 +1119,14 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   // (product at 82 944 elements 58 against 80 us, at 10 000 the same).
   Blocks B;
   const int passes = E >= (1 << 17) ? 2 : 1;
-  if (seg || p > 2 || !make_blocks(nle, passes, gm, islot, ila, hoc, hed, &B)) B = Blocks();
+  if (seg || p > 2 ||
+      !(p == 1 ? make_blocks<6>(passes, nslot, gm, inc, &B)
+               : make_blocks<10>(passes, nslot, gm, inc, &B)))
+    B = Blocks();
+  std::vector<int32_t>& gslot = inc;
+  if (p == 1) local_results<1>(gslot);
+  else if (p == 2) local_results<2>(gslot);
+  else local_results<3>(gslot);
   int rc = PG_OK;
   ElemOp* op = new ElemOp();
   op->p = p;
@@ -1141,9 +1160,9 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
   if (op->nblk > 0) {
     PG_A(op->bmeta, B.meta.size());
     PG_A(op->bslot, B.slot.size());
-    PG_A(op->bcode, B.code.size());
-    PG_A(op->bdofs, B.dofs.size());
-    PG_A(op->bpos, B.pos.size());
+    PG_A(op->bcode, B.slot.size());
+    PG_A(op->bdofs, B.slot.size() * nle);
+    PG_A(op->bpos, B.pos.size() / 2);
     PG_A(op->em, B.em.size());
     PG_A(op->xcopy, 2 * ndof);
   } else {
@@ -1174,9 +1193,7 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
             {op->gslot, gslot.data(), gslot.size() * sizeof(int32_t)},
             {op->bmeta, B.meta.data(), B.meta.size() * sizeof(int4)},
             {op->bslot, B.slot.data(), op->nblk ? B.slot.size() * sizeof(int32_t) : 0},
-            {op->bcode, B.code.data(), op->nblk ? B.code.size() * sizeof(int32_t) : 0},
-            {op->bdofs, B.dofs.data(), op->nblk ? B.dofs.size() * sizeof(int32_t) : 0},
-            {op->bpos, B.pos.data(), op->nblk ? B.pos.size() * sizeof(uint32_t) : 0},
+            {op->bpos, B.pos.data(), op->nblk ? B.pos.size() * sizeof(uint16_t) : 0},
             {op->em, B.em.data(), op->nblk ? B.em.size() * sizeof(int2) : 0},
             {op->wseg, wsg.data(), op->wseg ? wsg.size() * sizeof(int32_t) : 0},
             {op->womu, womu.data(), womu.size() * sizeof(double)}};
@@ -1185,6 +1202,12 @@ static int eop_build(int p, int64_t E, const void* ws, int64_t ndof, const int32
       delete op;
       PG_FAIL(PG_ERR_HIP, "element operator upload failed");
     }
+  if (op->nblk > 0) {
+    const int64_t n = (int64_t)B.slot.size();
+    hipLaunchKernelGGL(eop::k_eop_blk_elements, dim3((unsigned)((n + eop::kBS - 1) / eop::kBS)),
+                       dim3(eop::kBS), 0, st, n, nle, op->bslot, op->ocode, op->edofs, op->bcode,
+                       op->bdofs);
+  }
   if ((rc = eop_refresh(op, ws, omega, st)) != PG_OK) {
     delete op;
     return rc;
