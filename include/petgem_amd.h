@@ -109,7 +109,7 @@ int pg_plan_destroy(void *plan);
 int pg_plan_entity_pairs(const void *plan, int32_t *entity_pair, int32_t *max_rowlen);
 
 /* Device view of an exported plan (all device pointers).  entity_pair
- * (nullable, from pg_plan_entity_pairs, with entity_row_max its max_rowlen)
+ * (nullable, from pg_plan_entity_pairs)
  * saves the numeric assembly a search for its entities' first pairs (small p = 2
  * and 3 systems: selects the form that sums an entity's rows in LDS).  Same values,
  * bitwise. */
@@ -121,7 +121,7 @@ typedef struct pg_plan_dev {
   const int32_t *pair_slot0, *pair_rowlen, *pair_cbeg, *pair_ab;
   const uint32_t *contrib;
   const int32_t *entity_pair;
-  int32_t entity_row_max;
+  int32_t entity_row_max; /* not read (max_rowlen of pg_plan_entity_pairs) */
 } pg_plan_dev;
 
 /* Numeric assembly, atomic-free: CSR values (nnz complex128) of
@@ -283,7 +283,8 @@ typedef struct pg_solve_info {
   int32_t spmv_samples;     /* launches sampled for spmv_ms */
   int32_t pad2;
   double spmv_first_ms;     /* element-by-element operator: mean duration of its first
-                               kernel (the element products) within spmv_ms; else 0 */
+                               kernel within spmv_ms (the element products; where one
+                               kernel is the whole product, all of it); else 0 */
 } pg_solve_info;
 
 /* Create a solver for an n x n complex symmetric CSR matrix on the device
@@ -386,9 +387,8 @@ int pg_batch_set_mixed(void *batch, double inner_rtol, int stall_iters, void *st
 int pg_batch_set_block_jacobi(void *batch, void *stream);
 /* Optional: apply A_r with the element-by-element operator `eop` of the same
  * system (pg_eop_create on the geometry workspace `workspace`, p = 1 or 2,
- * PEC entities as in K and M) instead of the CSR products: per element and
- * batch of columns the entries of K_e and M_e are formed once and applied to
- * every column with its own frequency.  nrhs must be 64, 128, 192 or 256.
+ * PEC entities as in K and M) instead of the CSR products: K_e x_e and
+ * M_e x_e of every element and column, with the column's own frequency.  nrhs must be 64, 128, 192 or 256.
  * The true residuals still use K and M.  The operator must outlive the batch;
  * after new element geometry, pg_eop_refresh must accompany pg_batch_refresh.
  * Replaces, like the batch itself, one KSP per right-hand side

@@ -10,15 +10,16 @@ namespace pg {
 
 struct ElemOp;
 
-// Workgroups of the per-entity summation kernel: the number of reduction
+// Workgroups of the kernel that sums per entity: the number of reduction
 // partials (per quantity) that MODE 1 and MODE 2 leave in `part`.
 int eop_grid(const ElemOp* op);
 int64_t eop_ndof(const ElemOp* op);
 
 // MODE 0: y = A x.  MODE 1: y = A x and partials of x^T y (two per workgroup,
 // part[k * grid + b]).  MODE 2: y = b - A x and partials of |y|^2.  With `done`
-// non-null both kernels return at once while *done is set.  A non-null `mid`
-// is recorded on `st` between the two kernels (timing of the element products).
+// non-null the product's kernels return at once while *done is set.  A non-null `mid`
+// is recorded on `st` after the first of them (timing of the element products; the
+// whole product where it is one kernel, p <= 2).
 void eop_launch(const ElemOp* op, int mode, const int32_t* done, const double2* x, double2* y,
                 const double2* b, double* part, hipStream_t st, hipEvent_t mid = nullptr);
 void eop_launch(const ElemOp* op, int mode, const int32_t* done, const float2* x, float2* y,

@@ -1221,8 +1221,8 @@ struct Solver {
   double* dnorm = nullptr;
   int32_t* skip = nullptr;  // GMRES: second Gram-Schmidt pass not needed
   int restart = 30;
-  // SpMV sampling inside the solve: before, between the element operator's two
-  // kernels, after
+  // SpMV sampling inside the solve: before, after (1) and after the element
+  // operator's first kernel (2)
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   std::vector<void*> owned;
 
@@ -1428,7 +1428,7 @@ static int cocg_solve(Solver* S, const double2* b, double2* x, pg_solve_info* in
   while (true) {
     // the first iteration of every batch runs in full (the flags were clear
     // when the batch was enqueued): time its SpMV with events on this stream
-    const bool two_kernels = (low ? S->c32 : S->c64).kind == 3;
+    const bool element = (low ? S->c32 : S->c64).kind == 3;
     for (int k = 0; k < check; ++k) {
       if (low)
         launch_iteration<float2, float2>(S, st, S->c32, S->vals32, S->x32, S->r32, S->p32, S->q32,
@@ -1445,7 +1445,7 @@ static int cocg_solve(Solver* S, const double2* b, double2* x, pg_solve_info* in
         spmv_ms += ms;
         ++spmv_n;
       }
-      if (two_kernels && hipEventElapsedTime(&ms, S->ev[0], S->ev[2]) == hipSuccess) {
+      if (element && hipEventElapsedTime(&ms, S->ev[0], S->ev[2]) == hipSuccess) {
         first_ms += ms;
         ++first_n;
       }

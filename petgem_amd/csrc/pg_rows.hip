@@ -496,17 +496,17 @@ __device__ inline void assemble_class(const AsmArgs& a, int64_t block, AsmShared
 #pragma unroll
                   for (int l = 0; l < CL; ++l) {
                     const int64_t z = pr.x + l + (int64_t)k * pr.z;
-                  const double2 y = pr.y & kEliminated ? make_double2(0.0, 0.0)
-                                                       : make_double2(ks[j][k][l], v[k][l]);
-                  if (a.stride == 2) {
-                    typedef double dv2 __attribute__((ext_vector_type(2)));
-                    dv2 yy = {y.x, y.y};
-                    __builtin_nontemporal_store(yy, reinterpret_cast<dv2*>(a.K) + z);
-                  } else {
-                    a.K[z] = y.x;
-                    a.M[z] = y.y;
+                    const double2 y = pr.y & kEliminated ? make_double2(0.0, 0.0)
+                                                         : make_double2(ks[j][k][l], v[k][l]);
+                    if (a.stride == 2) {
+                      typedef double dv2 __attribute__((ext_vector_type(2)));
+                      dv2 yy = {y.x, y.y};
+                      __builtin_nontemporal_store(yy, reinterpret_cast<dv2*>(a.K) + z);
+                    } else {
+                      a.K[z] = y.x;
+                      a.M[z] = y.y;
+                    }
                   }
-                }
               }
             }
           }
