@@ -104,12 +104,14 @@ __device__ inline int face_code(int g0, int g1, const int32_t* fe) {
     if (g1 == fe[k]) k2 = k + 1;
   }
   const int sel = k1 * 10 + k2;
-  if (sel == 31) return 1;
-  if (sel == 23) return 2;
-  if (sel == 32) return 3;
-  if (sel == 13) return 4;
-  if (sel == 21) return 5;
-  return 0;
+  // (selects, not branches)
+  int code = 0;
+  code = sel == 31 ? 1 : code;
+  code = sel == 23 ? 2 : code;
+  code = sel == 32 ? 3 : code;
+  code = sel == 13 ? 4 : code;
+  code = sel == 21 ? 5 : code;
+  return code;
 }
 
 __device__ inline int element_orientation(const int32_t* en, const int32_t* ee, const int32_t* edn,
